@@ -1130,15 +1130,10 @@ static double* pfield(dpm_system* s, int f) {
     return nullptr;
 }
 
-int bumpy_upload(dpm_system* s, int f, const void* data, int64_t count,
-                 const std::vector<int>& sidx) {
+int bumpy_upload(dpm_system* s, int f, const void* data, int64_t count) {
     if (double* p = pfield(s, f)) {
         if (count != s->N) { set_error("dpm_upload: count mismatch"); return -1; }
-        const double* src = (const double*)data;
-        std::vector<double> h(s->N);
-        for (int64_t k = 0; k < s->N; ++k) h[k] = src[sidx[k]];
-        if (scopy(s, p, h.data(), sizeof(double) * s->N, hipMemcpyHostToDevice)) return -1;
-        return 0;
+        return field_set(s, 'D', 0, p, (const double*)data);
     }
     if (f == DPM_F_VERTEX_X || f == DPM_F_VERTEX_Y || f == DPM_F_VERTEX_MASS) {
         if (count != s->Nv) { set_error("dpm_upload: count mismatch"); return -1; }
@@ -1161,25 +1156,16 @@ int bumpy_upload(dpm_system* s, int f, const void* data, int64_t count,
     return -1;
 }
 
-int bumpy_download(dpm_system* s, int f, void* data, int64_t count,
-                   const std::vector<int>& sidx) {
+int bumpy_download(dpm_system* s, int f, void* data, int64_t count) {
     if (double* p = pfield(s, f)) {
         if (count != s->N) { set_error("dpm_download: count mismatch"); return -1; }
-        std::vector<double> h(s->N);
-        if (scopy(s, h.data(), p, sizeof(double) * s->N, hipMemcpyDeviceToHost)) return -1;
-        double* dst = (double*)data;
-        for (int64_t k = 0; k < s->N; ++k) dst[sidx[k]] = h[k];
-        return 0;
+        return field_get(s, 'D', 0, p, data);
     }
     if (f == DPM_F_NUM_VERTICES || f == DPM_F_VERTEX_CONTACTS) {
         if (count != s->N) { set_error("dpm_download: count mismatch"); return -1; }
         int* src = f == DPM_F_NUM_VERTICES ? s->d.nverts : s->d.vcontacts;
         if (!src) { set_error("dpm_download: field not computed"); return -1; }
-        std::vector<int> h(s->N);
-        if (scopy(s, h.data(), src, sizeof(int) * s->N, hipMemcpyDeviceToHost)) return -1;
-        int64_t* dst = (int64_t*)data;
-        for (int64_t k = 0; k < s->N; ++k) dst[sidx[k]] = h[k];
-        return 0;
+        return field_get(s, 'I', 0, src, data);
     }
     if (f == DPM_F_VERTEX_X || f == DPM_F_VERTEX_Y || f == DPM_F_VERTEX_MASS) {
         if (count != s->Nv) { set_error("dpm_download: count mismatch"); return -1; }

@@ -470,6 +470,7 @@ __device__ __forceinline__ double sum_value(const Dev& d, int what, int64_t i) {
         }
         case S_TQW: return d.torque[i] * d.omega[i];
         case S_COUNT: return (double)d.contacts[i];
+        case S_VCOUNT: return (double)d.vcontacts[i];
     }
     return 0.0;
 }
@@ -597,6 +598,54 @@ __global__ void k_add_velocity(Dev d, double ax, double ay, double scale) {
         v.y -= ay;
     }
     d.vel[i] = v;
+}
+
+// One per-particle field between the internal order and the static order, through a plain
+// double (or, for counts, int64) array on the device, so that a transfer moves 8 bytes per
+// particle in its final order.  Bound by the page faults of the caller's fresh array: 1.8 ms
+// for 8 MB against 12 ms when the record, the index array and a host-side scatter went over
+// (N = 1,000,003).
+__global__ __launch_bounds__(BLOCK) void k_field_get(Dev d, char kind, int comp,
+                                                     const void* plain, double* out) {
+    const int64_t k = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (k >= d.N) return;
+    const int id = d.sidx[k];
+    if (kind == 'I') {
+        ((long long*)out)[id] = ((const int*)plain)[k];
+    } else if (kind == 'S') {  // the permutation itself, in internal order
+        ((long long*)out)[k] = id;
+    } else if (kind == 'P') {
+        out[id] = ((const double*)(d.P0 + k))[comp];
+    } else if (kind == 'V' || kind == 'F') {
+        const double2 w = kind == 'V' ? d.vel[k] : d.frc[k];
+        out[id] = comp ? w.y : w.x;
+    } else {
+        out[id] = ((const double*)plain)[k];
+    }
+}
+
+__global__ __launch_bounds__(BLOCK) void k_field_set(Dev d, char kind, int comp, double* plain,
+                                                     const double* in) {
+    const int64_t k = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (k >= d.N) return;
+    const double w = in[d.sidx[k]];
+    if (kind == 'P') {
+        double4 q = d.P0[k];
+        if (comp == 0) q.x = w;
+        else if (comp == 1) q.y = w;
+        else if (comp == 2) q.z = w;
+        else q.w = w;
+        d.P0[k] = q;
+        d.P1[k] = q;
+    } else if (kind == 'V' || kind == 'F') {
+        double2* a = kind == 'V' ? d.vel : d.frc;
+        double2 v = a[k];
+        if (comp) v.y = w;
+        else v.x = w;
+        a[k] = v;
+    } else {
+        plain[k] = w;
+    }
 }
 
 // kernelAdamStep, src/particles/base/kernels.cu:550-611
@@ -1364,6 +1413,46 @@ int scopy(dpm_system* s, void* dst, const void* src, size_t bytes, hipMemcpyKind
     return 0;
 }
 
+// Between the caller's (pageable) array and the device staging array sp.P.  Small transfers
+// pass through a pinned buffer of the system: 16 us against 26 at 8 KB, 60 against 157 at
+// 256 KB; from 1 MB both take the same (the caller's page faults), so the buffer stays small.
+constexpr size_t STAGE_BYTES = 512 << 10;
+static int stage_copy(dpm_system* s, void* host, size_t bytes, bool to_device) {
+    void* dev = s->sp.P;
+    if (bytes > STAGE_BYTES)
+        return to_device ? scopy(s, dev, host, bytes, hipMemcpyHostToDevice)
+                         : scopy(s, host, dev, bytes, hipMemcpyDeviceToHost);
+    if (!s->hstage) {
+        const size_t want = std::min(STAGE_BYTES, sizeof(double) * (size_t)s->N);
+        DPM_HIP(hipHostMalloc(&s->hstage, want, hipHostMallocDefault));
+    }
+    if (to_device) std::memcpy(s->hstage, host, bytes);
+    DPM_HIP(hipMemcpyAsync(to_device ? dev : s->hstage, to_device ? s->hstage : dev, bytes,
+                           to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost,
+                           s->stream));
+    DPM_HIP(hipStreamSynchronize(s->stream));
+    if (!to_device) std::memcpy(host, s->hstage, bytes);
+    return 0;
+}
+
+// One per-particle array in static order: 'P' component of P0 (mirrored in P1), 'V'/'F'
+// component of vel/frc, 'D' a plain double array, 'I' an int array (int64 to the caller),
+// 'S' the static ids.  sp.P holds the array on its way (the rebuild's scratch: free between
+// calls, which are ordered on the stream).
+int field_get(dpm_system* s, char kind, int comp, const void* plain, void* host) {
+    hipLaunchKernelGGL(k_field_get, pgrid(s->N), dim3(BLOCK), 0, s->stream, s->d, kind, comp,
+                       plain, (double*)s->sp.P);
+    if (check_launch()) return -1;
+    return stage_copy(s, host, sizeof(double) * s->N, false);
+}
+
+int field_set(dpm_system* s, char kind, int comp, double* plain, const double* host) {
+    if (stage_copy(s, (void*)host, sizeof(double) * s->N, true)) return -1;
+    hipLaunchKernelGGL(k_field_set, pgrid(s->N), dim3(BLOCK), 0, s->stream, s->d, kind, comp,
+                       plain, (const double*)s->sp.P);
+    return check_launch();
+}
+
 // The fast minimum image is exact when L/2 exceeds every contact and list cutoff.
 static bool fast_ok(const dpm_system* s) {
     double lim = 2.0 * s->rmax;
@@ -1426,14 +1515,20 @@ int launch_chunk_sum(dpm_system* s, int what, double* out_dev) {
     return check_launch();
 }
 
-int sum_to_host(dpm_system* s, int what, double* out) {
-    double* dv = &s->d.ctl->scal[0];
-    if (launch_chunk_sum(s, what, dv)) return -1;
-    return scopy(s, out, dv, sizeof(double), hipMemcpyDeviceToHost);
+// The final kernel of a reduction stores its result in pinned host memory, so a reduction
+// ends with the wait for the stream and no copy (8-byte readbacks into pageable memory cost
+// 24 us each).  Several quantities share one wait.
+int sums_to_host(dpm_system* s, const int* what, int n, double* out) {
+    for (int k = 0; k < n; ++k)
+        if (launch_chunk_sum(s, what[k], s->hscal_dev + k)) return -1;
+    DPM_HIP(hipStreamSynchronize(s->stream));
+    for (int k = 0; k < n; ++k) out[k] = ((volatile double*)s->hscal)[k];
+    return 0;
 }
 
+int sum_to_host(dpm_system* s, int what, double* out) { return sums_to_host(s, &what, 1, out); }
+
 int max_to_host(dpm_system* s, int what, double* out) {
-    double* dv = &s->d.ctl->scal[1];
     const double* src = nullptr;
     int64_t n = s->nblk;
     if (what == M_ND) src = s->d.pmax_nd;
@@ -1443,9 +1538,11 @@ int max_to_host(dpm_system* s, int what, double* out) {
         hipLaunchKernelGGL(k_block_max, pgrid(s->N), dim3(BLOCK), 0, s->stream, s->d, what, tmp);
         src = tmp;
     }
-    hipLaunchKernelGGL(k_final_max, dim3(1), dim3(BLOCK), 0, s->stream, src, n, dv);
+    hipLaunchKernelGGL(k_final_max, dim3(1), dim3(BLOCK), 0, s->stream, src, n, s->hscal_dev);
     if (check_launch()) return -1;
-    return scopy(s, out, dv, sizeof(double), hipMemcpyDeviceToHost);
+    DPM_HIP(hipStreamSynchronize(s->stream));
+    *out = *(volatile double*)s->hscal;
+    return 0;
 }
 
 // =========================================================================
@@ -2183,9 +2280,13 @@ dpm_system* dpm_create(int kind, int64_t n, int64_t nv) {
         ok = ok && scopy(s, d.ctl, &c, sizeof(Ctl), hipMemcpyHostToDevice) == 0;
     }
     // fine-grained (coherent) pinned memory: kernels write the status into it directly
-    ok = ok && hipHostMalloc((void**)&s->hctl, 4 * sizeof(Ctl),
+    ok = ok && hipHostMalloc((void**)&s->hctl, 4 * sizeof(Ctl) + HSCAL * sizeof(double),
                              hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess;
     ok = ok && hipHostGetDevicePointer((void**)&s->d.hpub, s->hctl, 0) == hipSuccess;
+    if (ok) {  // behind the four mirrors: the reductions' results
+        s->hscal = (double*)(s->hctl + 4);
+        s->hscal_dev = (double*)(s->d.hpub + 4);
+    }
     for (int k = 0; ok && k < 4; ++k)
         ok = hipEventCreateWithFlags(&s->poll_ev[k], hipEventDisableTiming) == hipSuccess;
     if (ok && kind == DPM_BUMPY) ok = bumpy_alloc(s) == 0;
@@ -2216,6 +2317,7 @@ void dpm_destroy(dpm_system* s) {
     for (auto e : s->poll_ev)
         if (e) (void)hipEventDestroy(e);
     if (s->hctl) (void)hipHostFree(s->hctl);
+    if (s->hstage) (void)hipHostFree(s->hstage);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
 }
@@ -2259,10 +2361,8 @@ int dpm_upload(dpm_system* s, int f, const void* data, int64_t count) {
 }
 
 static int upload_field(dpm_system* s, int f, const void* data, int64_t count) {
-    std::vector<int> sidx;
-    if (fetch_sidx(s, sidx)) return -1;
     if (s->kind == DPM_BUMPY && ((f >= DPM_F_ANGLE && f <= DPM_F_MOI) || f >= DPM_F_VERTEX_X))
-        return bumpy_upload(s, f, data, count, sidx);
+        return bumpy_upload(s, f, data, count);
     if (count != s->N) {
         set_error("dpm_upload: count mismatch");
         return -1;
@@ -2275,60 +2375,34 @@ static int upload_field(dpm_system* s, int f, const void* data, int64_t count) {
         set_error("dpm_upload: field not uploadable");
         return -1;
     }
-    if (kind == 'D') {
-        std::vector<double> h(s->N);
-        for (int64_t k = 0; k < s->N; ++k) h[k] = src[sidx[k]];
-        return scopy(s, plain, h.data(), sizeof(double) * s->N, hipMemcpyHostToDevice);
-    }
-    if (kind == 'P') {
-        std::vector<double4> h(s->N);
-        if (scopy(s, h.data(), s->d.P0, sizeof(double4) * s->N, hipMemcpyDeviceToHost)) return -1;
-        for (int64_t k = 0; k < s->N; ++k) (&h[k].x)[comp] = src[sidx[k]];
-        if (f == DPM_F_RAD) {
-            double m = 0.0, mn = HUGE_VAL;
-            for (int64_t k = 0; k < s->N; ++k) {
-                m = std::max(m, h[k].z);
-                mn = std::min(mn, h[k].z);
-            }
-            s->rmax = m;
-            s->rmin = mn;
-            s->gen++;
+    if (f == DPM_F_RAD) {
+        double m = 0.0, mn = HUGE_VAL;
+        for (int64_t k = 0; k < s->N; ++k) {
+            m = std::max(m, src[k]);
+            mn = std::min(mn, src[k]);
         }
-        if (scopy(s, s->d.P0, h.data(), sizeof(double4) * s->N, hipMemcpyHostToDevice)) return -1;
-        return scopy(s, s->d.P1, h.data(), sizeof(double4) * s->N, hipMemcpyHostToDevice);
+        s->rmax = m;
+        s->rmin = mn;
+        s->gen++;
     }
-    double2* p2 = kind == 'V' ? s->d.vel : s->d.frc;
-    std::vector<double2> h(s->N);
-    if (scopy(s, h.data(), p2, sizeof(double2) * s->N, hipMemcpyDeviceToHost)) return -1;
-    for (int64_t k = 0; k < s->N; ++k) (comp ? h[k].y : h[k].x) = src[sidx[k]];
-    return scopy(s, p2, h.data(), sizeof(double2) * s->N, hipMemcpyHostToDevice);
+    return field_set(s, kind, comp, plain, src);
 }
 
 int dpm_download(dpm_system* s, int f, void* data, int64_t count) {
-    std::vector<int> sidx;
-    if (fetch_sidx(s, sidx)) return -1;
     if (s->kind == DPM_BUMPY && ((f >= DPM_F_ANGLE && f <= DPM_F_MOI) || f >= DPM_F_VERTEX_X))
-        return bumpy_download(s, f, data, count, sidx);
+        return bumpy_download(s, f, data, count);
     if (count != s->N) {
         set_error("dpm_download: count mismatch");
         return -1;
     }
-    if (f == DPM_F_STATIC_INDEX) {
-        int64_t* dst = (int64_t*)data;
-        for (int64_t k = 0; k < s->N; ++k) dst[k] = sidx[k];
-        return 0;
-    }
+    if (f == DPM_F_STATIC_INDEX) return field_get(s, 'S', 0, nullptr, data);
     if (f == DPM_F_NUM_NEIGHBORS || f == DPM_F_CONTACTS) {
         int* src = f == DPM_F_NUM_NEIGHBORS ? s->d.nnum : s->d.contacts;
         if (!src) {
             set_error("dpm_download: field not computed");
             return -1;
         }
-        std::vector<int> h(s->N);
-        if (scopy(s, h.data(), src, sizeof(int) * s->N, hipMemcpyDeviceToHost)) return -1;
-        int64_t* dst = (int64_t*)data;
-        for (int64_t k = 0; k < s->N; ++k) dst[sidx[k]] = h[k];
-        return 0;
+        return field_get(s, 'I', 0, src, data);
     }
     char kind;
     int comp;
@@ -2337,24 +2411,7 @@ int dpm_download(dpm_system* s, int f, void* data, int64_t count) {
         set_error("dpm_download: unknown or unallocated field");
         return -1;
     }
-    double* dst = (double*)data;
-    if (kind == 'D') {
-        std::vector<double> h(s->N);
-        if (scopy(s, h.data(), plain, sizeof(double) * s->N, hipMemcpyDeviceToHost)) return -1;
-        for (int64_t k = 0; k < s->N; ++k) dst[sidx[k]] = h[k];
-        return 0;
-    }
-    if (kind == 'P') {
-        std::vector<double4> h(s->N);
-        if (scopy(s, h.data(), s->d.P0, sizeof(double4) * s->N, hipMemcpyDeviceToHost)) return -1;
-        for (int64_t k = 0; k < s->N; ++k) dst[sidx[k]] = (&h[k].x)[comp];
-        return 0;
-    }
-    double2* p2 = kind == 'V' ? s->d.vel : s->d.frc;
-    std::vector<double2> h(s->N);
-    if (scopy(s, h.data(), p2, sizeof(double2) * s->N, hipMemcpyDeviceToHost)) return -1;
-    for (int64_t k = 0; k < s->N; ++k) dst[sidx[k]] = comp ? h[k].y : h[k].x;
-    return 0;
+    return field_get(s, kind, comp, plain, data);
 }
 
 int dpm_neighbor_config(dpm_system* s, int method, double cutoff, double thr_sq, int64_t ncd,
@@ -2527,14 +2584,11 @@ int dpm_reduce(dpm_system* s, int what, double* out) {
             return 0;
         }
         case DPM_RED_POWER: {
-            double a, b;
-            if (sum_to_host(s, S_FXVX, &a) || sum_to_host(s, S_FYVY, &b)) return -1;
-            double p = a + b;
-            if (s->kind == DPM_BUMPY) {
-                double c;
-                if (sum_to_host(s, S_TQW, &c)) return -1;
-                p = p + c;
-            }
+            const int w[3] = {S_FXVX, S_FYVY, S_TQW};
+            double v[3];
+            if (sums_to_host(s, w, s->kind == DPM_BUMPY ? 3 : 2, v)) return -1;
+            double p = v[0] + v[1];
+            if (s->kind == DPM_BUMPY) p = p + v[2];
             *out = p;
             return 0;
         }
@@ -2550,16 +2604,18 @@ int dpm_reduce(dpm_system* s, int what, double* out) {
             return 0;
         }
         case DPM_RED_FORCE_BALANCE: {
-            double a, b;
-            if (sum_to_host(s, S_FX, &a) || sum_to_host(s, S_FY, &b)) return -1;
-            *out = std::sqrt(a * a + b * b);
+            const int w[2] = {S_FX, S_FY};
+            double v[2];
+            if (sums_to_host(s, w, 2, v)) return -1;
+            *out = std::sqrt(v[0] * v[0] + v[1] * v[1]);
             return 0;
         }
         case DPM_RED_PRESSURE: {
             if (dpm_compute_stress(s)) return -1;
-            double a, b;
-            if (sum_to_host(s, S_SXX, &a) || sum_to_host(s, S_SYY, &b)) return -1;
-            *out = (a + b) / 2;
+            const int w[2] = {S_SXX, S_SYY};
+            double v[2];
+            if (sums_to_host(s, w, 2, v)) return -1;
+            *out = (v[0] + v[1]) / 2;
             return 0;
         }
         case DPM_RED_STRESS_XX:
@@ -2576,13 +2632,8 @@ int dpm_reduce(dpm_system* s, int what, double* out) {
         case DPM_RED_CONTACTS:
         case DPM_RED_VERTEX_CONTACTS: {
             if (dpm_count_contacts(s)) return -1;
-            std::vector<int> h(s->N);
-            int* src = what == DPM_RED_CONTACTS ? s->d.contacts : s->d.vcontacts;
-            if (scopy(s, h.data(), src, sizeof(int) * s->N, hipMemcpyDeviceToHost)) return -1;
-            int64_t t = 0;
-            for (int v : h) t += v;
-            *out = (double)t;
-            return 0;
+            // whole numbers below 2^53: exact in any order
+            return sum_to_host(s, what == DPM_RED_CONTACTS ? S_COUNT : S_VCOUNT, out);
         }
         case DPM_RED_PACKING_FRACTION: {
             double a;
@@ -2804,9 +2855,10 @@ int dpm_snapshot_restore(dpm_system* s) {
 
 // Particle::removeMeanVelocities (particle.cu:865-869)
 int dpm_remove_mean_velocity(dpm_system* s) {
-    double a, b;
-    if (sum_to_host(s, S_VX, &a) || sum_to_host(s, S_VY, &b)) return -1;
-    double mx = a / s->N, my = b / s->N;
+    const int w[2] = {S_VX, S_VY};
+    double v[2];
+    if (sums_to_host(s, w, 2, v)) return -1;
+    double mx = v[0] / s->N, my = v[1] / s->N;
     hipLaunchKernelGGL(k_add_velocity, pgrid(s->N), dim3(BLOCK), 0, s->stream, s->d, mx, my, 0.0);
     return check_launch();
 }

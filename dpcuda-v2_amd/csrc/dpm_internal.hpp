@@ -54,7 +54,6 @@ struct Ctl {
     int bad_pos;              // a non-finite position was binned
     int closed;               // the closing force of an NVE run has been applied
     int pub_seq;              // launch units published to the host mirror since the reset
-    double scal[16];          // small reduction results
 };
 
 // Device control block of the device-resident FIRE loop.
@@ -66,6 +65,8 @@ struct FireCtl {
     int stopped, done, converged, uphill;
     int pad[4];
 };
+
+constexpr int HSCAL = 4;  // reductions whose results one wait collects
 
 // Device pointers of one system (passed by value to kernels).
 struct Dev {
@@ -179,6 +180,8 @@ struct dpm_system {
     std::map<int64_t, dpm::Graph> nve_graphs, fire_graphs;
     dpm::Ctl* hctl = nullptr;   // pinned host mirror of the control block (4 slots),
                                 // written by the kernel that ends each launch unit
+    double *hscal = nullptr, *hscal_dev = nullptr;  // pinned: reduction results (HSCAL)
+    void* hstage = nullptr;     // pinned staging of small transfers (first use)
     double ktime_ms[3] = {0, 0, 0};
     int64_t klaunch[3] = {0, 0, 0};
     std::vector<hipEvent_t> ev_pool;

@@ -34,7 +34,7 @@ inline dim3 pgrid(int64_t n) {
 // which per-particle quantity a chunk-sum kernel reduces
 enum SumWhat {
     S_PE = 0, S_KE, S_FXVX, S_FYVY, S_FX, S_FY, S_SXX, S_SYY, S_SXY, S_SYX, S_VX, S_VY, S_R2,
-    S_TQW, S_COUNT
+    S_TQW, S_COUNT, S_VCOUNT
 };
 enum MaxWhat { M_ND = 0, M_CD, M_F2, M_T2 };
 
@@ -173,6 +173,9 @@ PairParams params_of(const dpm_system* s);
 NbrParams nbr_params(const dpm_system* s);
 int launch_chunk_sum(dpm_system* s, int what, double* out_dev);
 int sum_to_host(dpm_system* s, int what, double* out);
+int sums_to_host(dpm_system* s, const int* what, int n, double* out);
+int field_get(dpm_system* s, char kind, int comp, const void* plain, void* host);
+int field_set(dpm_system* s, char kind, int comp, double* plain, const double* host);
 int max_to_host(dpm_system* s, int what, double* out);
 int ensure_ell(dpm_system* s, int64_t cap);
 int device_rebuild(dpm_system* s, int mode, int* kind_out);
@@ -211,9 +214,7 @@ int bumpy_nve_run(dpm_system* s, double dt, int64_t n);
 void bumpy_enqueue_fire_forces(dpm_system* s, int kick, int gate, int check_pos = -1);
 void bumpy_enqueue_fire_step(dpm_system* s, int pos);
 int bumpy_snapshot(dpm_system* s, bool save);
-int bumpy_download(dpm_system* s, int field, void* data, int64_t count,
-                   const std::vector<int>& sidx);
-int bumpy_upload(dpm_system* s, int field, const void* data, int64_t count,
-                 const std::vector<int>& sidx);
+int bumpy_download(dpm_system* s, int field, void* data, int64_t count);
+int bumpy_upload(dpm_system* s, int field, const void* data, int64_t count);
 
 }  // namespace dpm
