@@ -166,36 +166,64 @@ __device__ __forceinline__ double pair_hot(double4 qi, double4 q, bool valid, co
     return contact ? num * p.inv2nc : 0.0;
 }
 
+// The value of lane t + S in lane t, for the lanes a halving tree still needs (t < S, and
+// what feeds them): whole rows of 16 lanes move by the row swaps (S = 32, 16), within a row
+// by data-parallel-primitive moves (S <= 8).  __shfl_down goes through the LDS crossbar (two
+// ds_bpermute and a wait per step and double); these stay in the vector pipe.  (Lanes that
+// the tree no longer needs hold other values than with __shfl_down.)
+template <int S>
+__device__ __forceinline__ int lane_down(int x) {
+    if constexpr (S == 32) {
+        return (int)__builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)x, false, false)[1];
+    } else if constexpr (S == 16) {
+        return (int)__builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)x, false, false)[1];
+    } else {
+        static_assert(S == 8 || S == 4 || S == 2 || S == 1, "a power of two below 64");
+        return __builtin_amdgcn_update_dpp(0, x, 0x100 + S, 0xf, 0xf, true);  // row_shl:S
+    }
+}
+
+template <int S>
+__device__ __forceinline__ double lane_down(double v) {
+    return __hiloint2double(lane_down<S>(__double2hiint(v)), lane_down<S>(__double2loint(v)));
+}
+
 // Pairwise-halving tree over the 64 lanes (lane t += lane t+s, s = 32..1);
 // lane 0 receives the canonical chunk sum.
 __device__ __forceinline__ double wave_tree_sum(double v) {
-#pragma unroll
-    for (int s = WAVE / 2; s > 0; s >>= 1) v = v + __shfl_down(v, s, WAVE);
-    return v;
+    v = v + lane_down<32>(v);
+    v = v + lane_down<16>(v);
+    v = v + lane_down<8>(v);
+    v = v + lane_down<4>(v);
+    v = v + lane_down<2>(v);
+    return v + lane_down<1>(v);
 }
 
+// maximum over the wave, in lane 0
 __device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-    for (int s = WAVE / 2; s > 0; s >>= 1) v = fmax(v, __shfl_down(v, s, WAVE));
-    return v;
+    v = fmax(v, lane_down<32>(v));
+    v = fmax(v, lane_down<16>(v));
+    v = fmax(v, lane_down<8>(v));
+    v = fmax(v, lane_down<4>(v));
+    v = fmax(v, lane_down<2>(v));
+    return fmax(v, lane_down<1>(v));
 }
 
 __device__ __forceinline__ int wave_max_i(int v) {
-#pragma unroll
-    for (int s = WAVE / 2; s > 0; s >>= 1) v = max(v, __shfl_down(v, s, WAVE));
-    return v;
+    v = max(v, lane_down<32>(v));
+    v = max(v, lane_down<16>(v));
+    v = max(v, lane_down<8>(v));
+    v = max(v, lane_down<4>(v));
+    v = max(v, lane_down<2>(v));
+    return max(v, lane_down<1>(v));
 }
 
-// Block-wide maxima of two values at once (the two shuffle chains interleave);
+// Block-wide maxima of two values at once;
 // results valid in thread 0.
 __device__ __forceinline__ void block_max2(double& a, double& b) {
     __shared__ double sm2[2][BLOCK / WAVE];
-#pragma unroll
-    for (int s = WAVE / 2; s > 0; s >>= 1) {
-        double ta = __shfl_down(a, s, WAVE), tb = __shfl_down(b, s, WAVE);
-        a = fmax(a, ta);
-        b = fmax(b, tb);
-    }
+    a = wave_max(a);
+    b = wave_max(b);
     int w = threadIdx.x / WAVE, l = threadIdx.x % WAVE;
     if (l == 0) {
         sm2[0][w] = a;
