@@ -688,14 +688,11 @@ __global__ __launch_bounds__(BLOCK) void k_b_force(BDev b) {
 }
 
 // kernelUpdateVertexNeighborList (rigid_bumpy/kernels.cu:870-922) for the rigid systems
-// whose particle rows were rebuilt in this step: for vertex v of particle p, over p's
-// particle row in order, the particles q whose centre lies within vp of v, then q's
-// vertices in order within vc of v (k_bumpy_vertex_build's row order).  A half-wave per
-// particle slot, its lanes over the particle's vertices: the row entries and q's vertex
-// positions are the same address for the 32 lanes (one load serves them all).  Two
-// consecutive slots share a wave, and a 64-slot chunk belongs to one system, so every
-// early return is uniform over the wave.  q's vertices are scanned only when v lies
-// within ring_reach of q's centre (vertex_ring_near): the rows are unchanged.
+// whose particle rows were rebuilt in this step: a half-wave per particle slot, its lanes
+// over the particle's vertices (vertex_row, as k_bumpy_vertex_rows; the rings of the arena
+// come from ring_vertex and move rigidly, so they are evenly spaced).  Two consecutive
+// slots share a wave, and a 64-slot chunk belongs to one system, so every early return is
+// uniform over the wave.
 constexpr int RB_HALF = 32;
 __global__ __launch_bounds__(BLOCK) void k_rb_vbuild(BDev b) {
     const long long t = (long long)blockIdx.x * BLOCK + threadIdx.x;
@@ -710,74 +707,24 @@ __global__ __launch_bounds__(BLOCK) void k_rb_vbuild(BDev b) {
     const double vc = sqrt(S.vc2);
     const bool shift = fmin(pp.halfLx, pp.halfLy) > vertex_shift_limit(S.rmax, S.rv, vc);
     const int hs = (int)(threadIdx.x % WAVE) / RB_HALF * RB_HALF;  // the half's first lane
-    const unsigned lt = (1u << lane) - 1u;  // the half's lanes below this one
+    const bool live = i - S.off < S.n;  // uniform over the half-wave
+    const int st = live ? b.vst[i] : 0, nv = live ? b.nvt[i] : 0;
+    const int nn = live ? min(b.nnum[i], b.cap) : 0;
+    const double4 cp = b.P[live ? i : S.off];
     int mx = 0;
-    if (i - S.off < S.n) {  // uniform over the half-wave
-        const int st = b.vst[i], nv = b.nvt[i];
-        const int nn = min(b.nnum[i], b.cap);
-        // the particle row, one entry per lane (nn <= cap = RB_HALF): the neighbour's
-        // record and vertex range, loaded at once and passed round by cross-lane reads
-        // instead of two dependent loads per entry
-        int rf = 0, rn = 0;
-        double rx = 0.0, ry = 0.0, rr = 0.0;
-        if (lane < nn) {
-            const int q = b.nbr[(long long)lane * b.nslot + i];
-            const double4 c = b.P[q];
-            rx = c.x;
-            ry = c.y;
-            rr = c.z;
-            rf = b.vst[q];
-            rn = b.nvt[q];
-        }
-        for (int a0 = 0; a0 < nv; a0 += RB_HALF) {
-            // lane: vertex a0 + lane of this particle; the rows of the half's vertices grow
-            // together, q by q, each q's vertices tested by all 32 lanes at once for one
-            // gated vertex after another
-            const bool has = a0 + lane < nv;
-            const double2 xv = has ? b.vpos[st + a0 + lane] : make_double2(0.0, 0.0);
-            int cnt = 0;
-            for (int k = 0; k < nn; ++k) {
-                const double4 cq = make_double4(__shfl(rx, k, RB_HALF), __shfl(ry, k, RB_HALF),
-                                                __shfl(rr, k, RB_HALF), 0.0);
-                const int f0 = __shfl(rf, k, RB_HALF), nq = __shfl(rn, k, RB_HALF);
-                const double kx = image_index(xv.x - cq.x, pp.Lx, pp.invLx, pp.halfLx, pp.fast);
-                const double ky = image_index(xv.y - cq.y, pp.Ly, pp.invLy, pp.halfLy, pp.fast);
-                const double dx = pbc_known(xv.x, cq.x, pp.Lx, kx, pp.fast);  // = pbc(xv, cq)
-                const double dy = pbc_known(xv.y, cq.y, pp.Ly, ky, pp.fast);
-                const double d2 = dx * dx + dy * dy;
-                const bool gate = has && d2 < S.vp2 && vertex_ring_near(d2, cq.z, S.rv, vc);
-                unsigned gm = (unsigned)(__builtin_amdgcn_ballot_w64(gate) >> hs);
-                if (gm == 0) continue;
-                for (int u0 = 0; u0 < nq; u0 += RB_HALF) {
-                    const bool uin = u0 + lane < nq;
-                    const int u = f0 + u0 + lane;
-                    const double2 xu = uin ? b.vpos[u] : make_double2(0.0, 0.0);
-                    for (unsigned m = gm; m != 0; m &= m - 1) {  // gated vertices, in order
-                        const int g = __builtin_ctz(m);
-                        const double gx = __shfl(xv.x, g, RB_HALF), gy = __shfl(xv.y, g, RB_HALF);
-                        double ex, ey;
-                        if (shift) {
-                            ex = pbc_known(gx, xu.x, pp.Lx, __shfl(kx, g, RB_HALF), pp.fast);
-                            ey = pbc_known(gy, xu.y, pp.Ly, __shfl(ky, g, RB_HALF), pp.fast);
-                        } else {
-                            ex = pbc(gx, xu.x, pp.Lx, pp.invLx, pp.halfLx, pp.fast);
-                            ey = pbc(gy, xu.y, pp.Ly, pp.invLy, pp.halfLy, pp.fast);
-                        }
-                        const bool hit = uin && ex * ex + ey * ey < S.vc2;
-                        const unsigned hm = (unsigned)(__builtin_amdgcn_ballot_w64(hit) >> hs);
-                        if (hm == 0) continue;
-                        // ascending u: lane order; vertex g's row continues at its count
-                        const int pos = __shfl(cnt, g, RB_HALF) + __builtin_popcount(hm & lt);
-                        if (hit && pos < b.vcap)
-                            b.vnbr[(long long)pos * b.nvslot + st + a0 + g] = u;
-                        if (lane == g) cnt += __builtin_popcount(hm);
-                    }
-                }
-            }
-            if (has) {
-                b.vnum[st + a0 + lane] = cnt;
-                mx = max(mx, cnt);
-            }
+    for (int a0 = 0; __builtin_amdgcn_ballot_w64(a0 < nv) != 0; a0 += RB_HALF) {
+        const bool has = a0 + lane < nv;
+        const long long v = st + a0 + lane;
+        const double2 xv = has ? b.vpos[v] : make_double2(0.0, 0.0);
+        const int cnt = vertex_row(
+            pp, b.P, b.vst, b.nvt, b.vpos, S.rv, vc, S.vc2, S.vp2, shift, lane, hs, has, xv, cp,
+            nn, [&](int k) { return b.nbr[(long long)k * b.nslot + i]; },
+            [&](int pos, int u) {
+                if (pos < b.vcap) b.vnbr[(long long)pos * b.nvslot + v] = u;
+            });
+        if (has) {
+            b.vnum[v] = cnt;
+            mx = max(mx, cnt);
         }
     }
     mx = wave_max_i(mx);

@@ -285,11 +285,8 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_build(Dev d, NbrParams n
     }
 }
 
-// The same rows for vertices on their rings (dpm_system::vring): a half-wave per particle,
-// lanes over its vertices; q's vertices are tested against one gated vertex at a time by
-// all 32 lanes (q's row entry and centre are the same address for the half), and the hits
-// append to that vertex's row in ascending order (ballot ranks).  Grid-stride over the
-// particles.
+// The same rows for evenly spaced rings (dpm_system::vuniform): a half-wave per particle,
+// lanes over its vertices (vertex_row).  Grid-stride over the particles.
 constexpr int VB_HALF = 32;
 __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb, double rv,
                                                              double rmax, int gated) {
@@ -298,56 +295,28 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb
     const bool shift = fmin(nb.halfLx, nb.halfLy) > vertex_shift_limit(rmax, rv, vc);
     const int lane = (int)(threadIdx.x % VB_HALF);
     const int hs = (int)(threadIdx.x % WAVE) / VB_HALF * VB_HALF;
-    const unsigned lt = (1u << lane) - 1u;
     const int64_t halves = (int64_t)gridDim.x * (BLOCK / VB_HALF);
     int mx = 0;
-    for (int64_t p = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) / VB_HALF; p < d.N;
-         p += halves) {
-        const int st = d.vstart[p], nv = d.nverts[p];
-        const int nn = min(d.nnum[p], d.cap);
-        for (int a0 = 0; a0 < nv; a0 += VB_HALF) {
+    // (whole waves stay in the loop together: the odd half of the last wave has no particle)
+    for (int64_t p0 = ((int64_t)blockIdx.x * BLOCK + threadIdx.x - lane - hs) / VB_HALF;
+         p0 < d.N; p0 += halves) {
+        const int64_t p = p0 + hs / VB_HALF;
+        const bool live = p < d.N;
+        const int st = live ? d.vstart[p] : 0, nv = live ? d.nverts[p] : 0;
+        const int nn = live ? min(d.nnum[p], d.cap) : 0;
+        const double4 cp = d.P0[live ? p : 0];
+        for (int a0 = 0; __builtin_amdgcn_ballot_w64(a0 < nv) != 0; a0 += VB_HALF) {
             const bool has = a0 + lane < nv;
-            const double2 xv = has ? d.vpos[st + a0 + lane] : make_double2(0.0, 0.0);
-            int cnt = 0;
-            for (int k = 0; k < nn; ++k) {
-                const int q = d.nbr[(int64_t)k * d.N + p];
-                const double4 cq = d.P0[q];
-                const double kx = image_index(xv.x - cq.x, nb.Lx, nb.invLx, nb.halfLx, nb.fast);
-                const double ky = image_index(xv.y - cq.y, nb.Ly, nb.invLy, nb.halfLy, nb.fast);
-                const double dx = pbc_known(xv.x, cq.x, nb.Lx, kx, nb.fast);  // = pbc(xv, cq)
-                const double dy = pbc_known(xv.y, cq.y, nb.Ly, ky, nb.fast);
-                const double d2 = dx * dx + dy * dy;
-                const bool gate = has && d2 < nb.vp2 && vertex_ring_near(d2, cq.z, rv, vc);
-                const unsigned gm = (unsigned)(__builtin_amdgcn_ballot_w64(gate) >> hs);
-                if (gm == 0) continue;
-                const int f0 = d.vstart[q], nq = d.nverts[q];
-                for (int u0 = 0; u0 < nq; u0 += VB_HALF) {
-                    const bool uin = u0 + lane < nq;
-                    const int u = f0 + u0 + lane;
-                    const double2 xu = uin ? d.vpos[u] : make_double2(0.0, 0.0);
-                    for (unsigned m = gm; m != 0; m &= m - 1) {
-                        const int g = __builtin_ctz(m);
-                        const double gx = __shfl(xv.x, g, VB_HALF), gy = __shfl(xv.y, g, VB_HALF);
-                        double ex, ey;
-                        if (shift) {
-                            ex = pbc_known(gx, xu.x, nb.Lx, __shfl(kx, g, VB_HALF), nb.fast);
-                            ey = pbc_known(gy, xu.y, nb.Ly, __shfl(ky, g, VB_HALF), nb.fast);
-                        } else {
-                            ex = pbc(gx, xu.x, nb.Lx, nb.invLx, nb.halfLx, nb.fast);
-                            ey = pbc(gy, xu.y, nb.Ly, nb.invLy, nb.halfLy, nb.fast);
-                        }
-                        const bool hit = uin && ex * ex + ey * ey < nb.vc2;
-                        const unsigned hm = (unsigned)(__builtin_amdgcn_ballot_w64(hit) >> hs);
-                        if (hm == 0) continue;
-                        const int pos = __shfl(cnt, g, VB_HALF) + __builtin_popcount(hm & lt);
-                        if (hit && pos < d.vcap)
-                            d.vnbr[(int64_t)pos * d.Nv + st + a0 + g] = u;
-                        if (lane == g) cnt += __builtin_popcount(hm);
-                    }
-                }
-            }
+            const int64_t v = st + a0 + lane;
+            const double2 xv = has ? d.vpos[v] : make_double2(0.0, 0.0);
+            const int cnt = vertex_row(
+                nb, d.P0, d.vstart, d.nverts, d.vpos, rv, vc, nb.vc2, nb.vp2, shift, lane, hs,
+                has, xv, cp, nn, [&](int k) { return d.nbr[(int64_t)k * d.N + p]; },
+                [&](int pos, int u) {
+                    if (pos < d.vcap) d.vnbr[(int64_t)pos * d.Nv + v] = u;
+                });
             if (has) {
-                d.vnum[st + a0 + lane] = cnt;
+                d.vnum[v] = cnt;
                 mx = max(mx, cnt);
             }
         }
@@ -937,7 +906,7 @@ int bumpy_ensure_vcap(dpm_system* s, int64_t cap) {
 // particle list build; overflow is detected by the chain's end kernel.
 void bumpy_enqueue_vertex_build(dpm_system* s, int gated) {
     // grid-stride: a gated launch that skips stays cheap
-    if (s->vring) {
+    if (s->vuniform) {
         dim3 g(std::min<unsigned>(pgrid(s->N * VB_HALF).x, 2048u));
         hipLaunchKernelGGL(k_bumpy_vertex_rows, g, dim3(BLOCK), 0, s->stream, s->d,
                            nbr_params(s), s->rv, s->rmax, gated);
@@ -1006,8 +975,10 @@ int bumpy_stress(dpm_system* s) {
 }
 
 // Whether every vertex lies at r - r_v from its particle's centre to a relative 1e-9
-// (vertex_ring_near's assumption): true after dpm_bumpy_setup, checked again on the host
-// after an upload of positions, radii or vertex positions.
+// (vertex_ring_near's assumption), and whether the vertices of each particle are also evenly
+// spaced around it, counterclockwise and in the centre's own image, to 1e-6 (ring_window's):
+// both true after dpm_bumpy_setup, checked again on the host after an upload of positions,
+// radii or vertex positions.
 int bumpy_check_ring(dpm_system* s) {
     std::vector<double4> P(s->N);
     std::vector<int> st(s->N), nv(s->N);
@@ -1018,9 +989,24 @@ int bumpy_check_ring(dpm_system* s) {
         scopy(s, vp.data(), s->d.vpos, sizeof(double2) * s->Nv, hipMemcpyDeviceToHost))
         return -1;
     auto img = [](double d, double L) { return d - L * std::round(d / L); };
-    bool ok = true;
+    bool ok = true, even = true;
+    int turn_nv = 0;
+    double turn_s = 0.0, turn_c = 1.0;
     for (int64_t p = 0; p < s->N && ok; ++p) {
         const double inner = P[p].z - s->rv;
+        if (nv[p] != turn_nv) {
+            turn_nv = nv[p];
+            turn_s = std::sin(2 * M_PI / turn_nv);
+            turn_c = std::cos(2 * M_PI / turn_nv);
+        }
+        double ex = vp[st[p]].x - P[p].x, ey = vp[st[p]].y - P[p].y;  // where vertex k belongs
+        for (int k = 0; k < nv[p] && even; ++k) {
+            const double2 u = vp[st[p] + k];
+            even = std::fabs(u.x - P[p].x - ex) + std::fabs(u.y - P[p].y - ey) <= 1e-6 * inner;
+            const double t = ex * turn_c - ey * turn_s;
+            ey = ex * turn_s + ey * turn_c;
+            ex = t;
+        }
         for (int k = 0; k < nv[p] && ok; ++k) {
             const double2 u = vp[st[p] + k];
             const double dx = img(u.x - P[p].x, s->box[0]), dy = img(u.y - P[p].y, s->box[1]);
@@ -1028,7 +1014,8 @@ int bumpy_check_ring(dpm_system* s) {
         }
     }
     s->vring = ok;
-    s->gen++;  // captured graphs bake the flag
+    s->vuniform = ok && even;
+    s->gen++;  // captured graphs bake the flags
     return 0;
 }
 
@@ -1267,7 +1254,6 @@ int dpm_bumpy_setup(dpm_system* s, const int64_t* nvp, double rv, int rotation) 
     hipLaunchKernelGGL(k_bumpy_init_vertices, pgrid(s->N), dim3(BLOCK), 0, s->stream, s->d, rv);
     if (check_launch()) return -1;
     DPM_HIP(hipStreamSynchronize(s->stream));
-    s->vring = rv > 0;  // rings of radius r - r_v (radii above r_v: checked below)
     if (refresh_rmax(s)) return -1;
     return bumpy_check_ring(s);
 }

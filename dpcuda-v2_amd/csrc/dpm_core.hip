@@ -2828,6 +2828,8 @@ int dpm_snapshot_save(dpm_system* s) {
     if (s->kind == DPM_BUMPY && bumpy_snapshot(s, true)) return -1;
     s->snap_box[0] = s->box[0];
     s->snap_box[1] = s->box[1];
+    s->snap_vring = s->vring;
+    s->snap_vuniform = s->vuniform;
     s->snap_valid = true;
     return 0;
 }
@@ -2848,6 +2850,8 @@ int dpm_snapshot_restore(dpm_system* s) {
     DPM_HIP(cp(s->d.frc, s->snap.frc, sizeof(double2) * n));
     DPM_HIP(cp(s->d.sidx, s->snap.sidx, sizeof(int) * n));
     if (s->kind == DPM_BUMPY && bumpy_snapshot(s, false)) return -1;
+    s->vring = s->snap_vring;  // (dpm_set_box bumps gen: graphs bake the flags)
+    s->vuniform = s->snap_vuniform;
     if (dpm_set_box(s, s->snap_box[0], s->snap_box[1])) return -1;
     if (s->nbr_ready && device_rebuild(s, 2, nullptr)) return -1;
     return 0;
