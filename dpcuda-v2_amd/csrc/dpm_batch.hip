@@ -53,8 +53,11 @@
 //               the closing kick and the chunk partials
 //   k_rb_eval   per particle (a half-wave over its vertices), before k_b_eval: the
 //               stress and contacts of a rigid system that finished a minimisation
+// Disk systems of up to RES_MAX_N particles take none of these launches: k_b_resident
+// (dpm_batch_resident.hpp) runs all their phases in one workgroup, many steps a launch.
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <string>
 #include <vector>
@@ -97,10 +100,11 @@ struct BSys {
     int mode;      // BMode of the next batched step
     int rebuild;   // Verlet rebuild before the next force evaluation
     int snap_op;   // pending for b_prep_slot: 1 save, 2 restore
-    int pad0;
+    int res;       // advanced by k_b_resident; the per-phase kernels leave it alone
     double scale_f;  // pending position scale (0: none)
     // jamming controller (dpm_jam)
-    int jphase, dec_it, status, pad1;
+    int jphase, dec_it, status;
+    int far;       // resident systems: the displacement flag (BP_DMAX's "some wave is far")
     double L_low, L_high, L_last, snapLx, snapLy, pr;
     long long cstep, fire_total, contacts;
     double pe_final, phi_final;
@@ -334,6 +338,7 @@ __global__ __launch_bounds__(BLOCK) void k_b_prep_move(BDev b) {
     const int s = b.sys_of[i];
     if (s < 0) return;  // free arena slots (64-aligned: whole waves)
     const BSys& S = b.sys[s];
+    if (S.res) return;
     const bool rigid = S.kind == BK_RIGID;
     b_prep_slot(b, S, i, rigid);
     if (rigid) rb_move_slot(b, S, i);
@@ -363,7 +368,7 @@ __global__ __launch_bounds__(BLOCK) void k_rb_vmove(BDev b) {
 // the step (the move's, or at a prologue those of the last minimisation's end): some
 // 3 d^2 > thr^2.
 __device__ __forceinline__ bool b_rebuild_now(const BDev& b, const BSys& S) {
-    if (S.mode == BM_DONE || S.mode == BM_EVAL || S.mode == BM_EMPTY) return false;
+    if (S.res || S.mode == BM_DONE || S.mode == BM_EVAL || S.mode == BM_EMPTY) return false;
     if (S.rebuild || S.mode == BM_RESTORE) return true;
     const double* D = bpart(b, BP_DMAX) + S.off / WAVE;  // per wave: some 3 d^2 > thr
     bool far = false;
@@ -619,7 +624,7 @@ __global__ __launch_bounds__(BLOCK) void k_b_force(BDev b) {
     const int s = b.sys_of[i];
     if (s < 0) return;  // free arena slots (64-aligned: whole waves)
     const BSys& S = b.sys[s];
-    if (S.mode != BM_PROLOGUE && S.mode != BM_FIRE) return;
+    if (S.res || (S.mode != BM_PROLOGUE && S.mode != BM_FIRE)) return;
     if (S.kind == BK_RIGID) return;  // k_rb_force
     const int kick = S.mode == BM_FIRE;
     const PairParams p = bparams(b, S);
@@ -927,50 +932,35 @@ __device__ __forceinline__ void enter_eval(const BDev& b, BSys& S, int s) {
     if (S.kind == BK_RIGID) b.evlist[atomicAdd(&b.flags[9], 1)] = s;
 }
 
-// one wave per system: minimizeFire's stop test (minimization.cu:96-105, with the
-// optional |F|max criterion) and Fire::step's decision for the next iteration
-// (fire.cu:14-33) -- k_fire_ctl's arithmetic on the system's chunk partials
-__global__ __launch_bounds__(WAVE) void k_b_ctl(BDev b) {
-    BSys& S = b.sys[blockIdx.x];
-    const int mode = S.mode;
-    if (threadIdx.x == 0) {
-        if (blockIdx.x == 0) b.flags[3] += 1;  // one thread of the step counts it
-        // the controller's requests of the last step are applied (k_b_prep_move)
-        S.snap_op = 0;
-        S.scale_f = 0.0;
+// The controller's requests of the last step are applied; a restore step's lists are current
+// for the restored state, so scaleBox follows and the minimisation begins.  (One thread.)
+__device__ __forceinline__ void b_step_begin(BSys& S) {
+    S.snap_op = 0;
+    S.scale_f = 0.0;
+    if (S.mode == BM_RESTORE) {
+        scale_box_of(S, S.pend_f);
+        S.pend_f = 0.0;
+        S.rebuild = 0;
+        S.mode = BM_PROLOGUE;
     }
-    if (mode == BM_RESTORE) {  // the lists are current for the restored state: scaleBox
-        if (threadIdx.x == 0) {
-            scale_box_of(S, S.pend_f);
-            S.pend_f = 0.0;
-            S.rebuild = 0;
-            S.mode = BM_PROLOGUE;
-        }
-        return;
-    }
-    if (mode != BM_PROLOGUE && mode != BM_FIRE) return;
-    const bool rigid = S.kind == BK_RIGID;
-    const long long c0 = S.off / WAVE;
-    // (the fourth sum is the rigid spin power; a disk system sums its PE array again)
-    double px, py, pe, ptw;
-    wave_final_sum4(bpart(b, BP_PX) + c0, bpart(b, BP_PY) + c0, bpart(b, BP_PE) + c0,
-                    bpart(b, rigid ? BP_TW : BP_PE) + c0, S.nc, px, py, pe, ptw);
-    double fm = 0.0;
-    for (int k = threadIdx.x; k < S.nc; k += WAVE) fm = fmax(fm, bpart(b, BP_F2)[c0 + k]);
-    fm = wave_max(fm);
-    if (threadIdx.x != 0) return;
+}
+
+// minimizeFire's stop test (minimization.cu:96-105, with the optional |F|max criterion) and
+// Fire::step's decision for the next iteration (fire.cu:14-33): k_fire_ctl's arithmetic.  pe:
+// the potential energy, power: F.v (+ tau.w), fm: max F^2.  Returns whether the minimisation
+// has ended.  (One thread.)
+__device__ __forceinline__ bool b_fire_decide(BSys& S, double pe, double power, double fm) {
     S.rebuild = 0;  // the list this step used is current
     const double dof = (double)S.n;
     double avg = pe / dof;
     S.fmax_sq = fm;
     S.avg_pe = avg;
-    if (mode == BM_PROLOGUE) {
+    if (S.mode == BM_PROLOGUE) {
         S.last_avg_pe = avg;
         S.mode = BM_FIRE;
         if (S.J.max_steps <= 0) {
             S.done = 1;
-            enter_eval(b, S, blockIdx.x);
-            return;
+            return true;
         }
     } else {
         double diff = fabs(avg / S.last_avg_pe - 1);
@@ -980,18 +970,13 @@ __global__ __launch_bounds__(WAVE) void k_b_ctl(BDev b) {
         if (diff < S.J.pe_diff_t || avg < S.J.pe_t || fok) {
             S.converged = 1;
             S.done = 1;
-            enter_eval(b, S, blockIdx.x);
-            return;
+            return true;
         }
         if (S.step >= S.J.max_steps) {
             S.done = 1;
-            enter_eval(b, S, blockIdx.x);
-            return;
+            return true;
         }
     }
-    // RigidBumpy::getPowerFire adds sum(tau*w) (rigid_bumpy.cu:1181-1191)
-    double power = px + py;
-    if (rigid) power = power + ptw;
     S.power = power;
     if (power > 0) {
         S.n_good++;
@@ -1008,13 +993,37 @@ __global__ __launch_bounds__(WAVE) void k_b_ctl(BDev b) {
             S.stopped = 1;
             S.step += 1;
             S.done = 1;
-            enter_eval(b, S, blockIdx.x);
-            return;
+            return true;
         }
         S.dt = fmax(S.dt * 0.5, S.dt_min);
         S.alpha = S.J.alpha0;
         S.uphill = 1;
     }
+    return false;
+}
+
+// one wave per system: b_fire_decide on the system's chunk partials
+__global__ __launch_bounds__(WAVE) void k_b_ctl(BDev b) {
+    BSys& S = b.sys[blockIdx.x];
+    if (blockIdx.x == 0 && threadIdx.x == 0) b.flags[3] += 1;  // one thread of the step counts it
+    if (S.res) return;
+    const int mode = S.mode;
+    if (threadIdx.x == 0) b_step_begin(S);
+    if (mode != BM_PROLOGUE && mode != BM_FIRE) return;
+    const bool rigid = S.kind == BK_RIGID;
+    const long long c0 = S.off / WAVE;
+    // (the fourth sum is the rigid spin power; a disk system sums its PE array again)
+    double px, py, pe, ptw;
+    wave_final_sum4(bpart(b, BP_PX) + c0, bpart(b, BP_PY) + c0, bpart(b, BP_PE) + c0,
+                    bpart(b, rigid ? BP_TW : BP_PE) + c0, S.nc, px, py, pe, ptw);
+    double fm = 0.0;
+    for (int k = threadIdx.x; k < S.nc; k += WAVE) fm = fmax(fm, bpart(b, BP_F2)[c0 + k]);
+    fm = wave_max(fm);
+    if (threadIdx.x != 0) return;
+    // RigidBumpy::getPowerFire adds sum(tau*w) (rigid_bumpy.cu:1181-1191)
+    double power = px + py;
+    if (rigid) power = power + ptw;
+    if (b_fire_decide(S, pe, power, fm)) enter_eval(b, S, blockIdx.x);
 }
 
 // after a minimisation: setVelocitiesToZero (minimizeFire's end), then
@@ -1370,6 +1379,20 @@ __device__ __forceinline__ bool b_jam_decide(const BDev& b, BSys& S, double sxx,
     return finished;
 }
 
+// b_jam_decide and, for a system that finishes, its results; returns whether the controller
+// leaves operations that its slots still have to see.
+__device__ __forceinline__ bool b_jam_step(const BDev& b, BSys& S, double sxx, double syy,
+                                           double z, double pe, double r2,
+                                           long long batched_step) {
+    if (!b_jam_decide(b, S, sxx, syy, z)) return false;
+    S.done_step = batched_step;
+    S.pe_final = pe;
+    const double PI = 3.141592653589793238462643383279502884197;
+    S.phi_final = r2 * PI / (S.Lx * S.Ly);
+    S.mode = BM_DONE;
+    return S.snap_op != 0 || S.scale_f != 0.0;
+}
+
 // one wave per system: the jamming controller of dpm_jam after a minimisation.  A
 // system that finishes gets the controller's last snapshot / scaling operations at once
 // (its slots see no further step).
@@ -1384,17 +1407,7 @@ __global__ __launch_bounds__(WAVE) void k_b_jam(BDev b) {
     for (int k = threadIdx.x; k < S.nc; k += WAVE) z += bpart(b, BP_Z)[c0 + k];
     z = wave_tree_sum(z);  // integer counts: exact in any order
     __shared__ int apply;
-    if (threadIdx.x == 0) {
-        const bool finished = b_jam_decide(b, S, sxx, syy, z);
-        apply = finished && (S.snap_op != 0 || S.scale_f != 0.0);
-        if (finished) {
-            S.done_step = b.flags[3];
-            S.pe_final = pe;
-            const double PI = 3.141592653589793238462643383279502884197;
-            S.phi_final = r2 * PI / (S.Lx * S.Ly);
-            S.mode = BM_DONE;
-        }
-    }
+    if (threadIdx.x == 0) apply = b_jam_step(b, S, sxx, syy, z, pe, r2, b.flags[3]);
     __syncthreads();
     if (apply) {
         const bool rigid = S.kind == BK_RIGID;
@@ -1415,6 +1428,8 @@ __global__ __launch_bounds__(WAVE) void k_b_jam(BDev b) {
         b.done_list[k % b.nsys] = (int)blockIdx.x;
     }
 }
+
+#include "dpm_batch_resident.hpp"
 
 }  // namespace dpm
 
@@ -1454,6 +1469,13 @@ struct dpm_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int64_t graph_steps = 0;
+    // resident systems (k_b_resident): their ids by size class, on the device; the launches of
+    // the classes run side by side on streams of their own, forked from and joined to `stream`
+    int* rids = nullptr;
+    int rcount[dpm::RES_CLASSES] = {};
+    bool phased = true;  // some system is advanced by the per-phase kernels
+    hipStream_t rstream[dpm::RES_CLASSES] = {};
+    hipEvent_t rfork = nullptr, rjoin[dpm::RES_CLASSES] = {};
     // DPM_OPT_TIMING: HIP events around every k_b_force launch (eager launches)
     bool timing = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pending;
@@ -1621,6 +1643,11 @@ static BJam jam_constants(const dpm_jam_params* P) {
     return J;
 }
 
+// Steps of one launch of resident systems with no other system in the batch: some tens of
+// milliseconds, so that a finished batch is noticed soon and a launch's end, where the large
+// systems run alone, weighs little.
+constexpr int64_t RES_STEPS = 4096;
+
 static hipEvent_t batch_event(dpm_batch* b) {
     if (b->ev_free.empty()) {
         hipEvent_t e = nullptr;
@@ -1707,6 +1734,76 @@ static void enqueue_batch_step(dpm_batch* b) {
                            dim3(BLOCK), 0, st, d);
     hipLaunchKernelGGL(k_b_eval, slots, dim3(BLOCK), 0, st, d);
     hipLaunchKernelGGL(k_b_jam, dim3((unsigned)b->nsys), dim3(WAVE), 0, st, d);
+}
+
+// Whether a system of n particles is advanced by k_b_resident: disks that fit a workgroup,
+// with a pair law of the short sequences (fastdiv), and no timing of the force pass asked for.
+// The line lies where the LDS ends: up to there one workgroup's step beats seven launches
+// (384 systems of 64 to 2,048 particles: 210 ms against 708 ms).
+static bool resident_size(const dpm_batch* b, int64_t n, bool rigid, bool fastdiv) {
+    return !rigid && fastdiv && !b->timing && n <= RES_MAX_N;
+}
+
+// The resident systems' table from (system, particles) pairs: class by class.  The stream is
+// idle with respect to the table's readers.
+static int resident_table(dpm_batch* b, const std::vector<std::pair<int, int64_t>>& systems) {
+    if (!b->rids && balloc_n(b, &b->rids, b->nsys)) return -1;
+    std::vector<int> ids;
+    for (int c = 0; c < RES_CLASSES; ++c) {
+        const size_t before = ids.size();
+        for (auto& e : systems)
+            if (e.second <= RES_LIMIT[c] && (c == 0 || e.second > RES_LIMIT[c - 1]))
+                ids.push_back(e.first);
+        b->rcount[c] = (int)(ids.size() - before);
+    }
+    if (!ids.empty()) BCOPY(b->rids, ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice);
+    return 0;
+}
+
+// `steps` steps of every resident system (base: the batched steps before them), one launch
+// per class, largest systems first.  They run beside whatever follows on b->stream until
+// resident_join.
+static int resident_launch(dpm_batch* b, int64_t base, int64_t steps) {
+    bool forked = false;
+    for (int c = RES_CLASSES - 1; c >= 0; --c) {
+        if (!b->rcount[c]) continue;
+        if (!b->rstream[c]) {
+            DPM_HIP(hipStreamCreateWithFlags(&b->rstream[c], hipStreamNonBlocking));
+            DPM_HIP(hipEventCreateWithFlags(&b->rjoin[c], hipEventDisableTiming));
+            if (!b->rfork) DPM_HIP(hipEventCreateWithFlags(&b->rfork, hipEventDisableTiming));
+        }
+        if (!forked) DPM_HIP(hipEventRecord(b->rfork, b->stream));
+        forked = true;
+        int first = 0;
+        for (int k = 0; k < c; ++k) first += b->rcount[k];
+        hipStream_t st = b->rstream[c];
+        DPM_HIP(hipStreamWaitEvent(st, b->rfork, 0));
+        const dim3 grid((unsigned)b->rcount[c]);
+        const int* ids = b->rids + first;
+        const long long b0 = base;
+        const int k = (int)steps;
+        switch (c) {
+            case 0: hipLaunchKernelGGL((k_b_resident<256, 1, 32>), grid, dim3(256), 0, st, b->d,
+                                       ids, b0, k); break;
+            case 1: hipLaunchKernelGGL((k_b_resident<512, 1, 32>), grid, dim3(512), 0, st, b->d,
+                                       ids, b0, k); break;
+            case 2: hipLaunchKernelGGL((k_b_resident<1024, 1, 24>), grid, dim3(1024), 0, st,
+                                       b->d, ids, b0, k); break;
+            case 3: hipLaunchKernelGGL((k_b_resident<1024, 2, 16>), grid, dim3(1024), 0, st,
+                                       b->d, ids, b0, k); break;
+            default: hipLaunchKernelGGL((k_b_resident<1024, 4, 0>), grid, dim3(1024), 0, st,
+                                        b->d, ids, b0, k);
+        }
+        if (check_launch()) return -1;
+        DPM_HIP(hipEventRecord(b->rjoin[c], st));
+    }
+    return 0;
+}
+
+static int resident_join(dpm_batch* b) {
+    for (int c = 0; c < RES_CLASSES; ++c)
+        if (b->rcount[c]) DPM_HIP(hipStreamWaitEvent(b->stream, b->rjoin[c], 0));
+    return 0;
 }
 
 static void drop_graph(dpm_batch* b) {
@@ -1869,6 +1966,8 @@ dpm_batch* dpm_batch_create_mixed(int64_t n_systems, const int64_t* n_particles,
 
 void dpm_batch_destroy(dpm_batch* b) {
     if (!b) return;
+    for (auto st : b->rstream)
+        if (st) (void)hipStreamSynchronize(st);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -1880,6 +1979,11 @@ void dpm_batch_destroy(dpm_batch* b) {
     for (auto e : b->poll)
         if (e) (void)hipEventDestroy(e);
     for (auto e : b->ev_all) (void)hipEventDestroy(e);
+    if (b->rfork) (void)hipEventDestroy(b->rfork);
+    for (auto e : b->rjoin)
+        if (e) (void)hipEventDestroy(e);
+    for (auto st : b->rstream)
+        if (st) (void)hipStreamDestroy(st);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -2138,6 +2242,7 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
     batch_common(b, fastdiv);
     const BJam J = jam_constants(P);
     // every system starts minimizeFire (decompression phase) with a fresh list
+    std::vector<std::pair<int, int64_t>> resident;
     for (int64_t s = 0; s < b->nsys; ++s) {
         BSys& S = b->hsys[s];
         BSys f{};
@@ -2159,8 +2264,12 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
         f.jphase = min_only ? BJ_MIN : BJ_DECOMP;
         f.status = 1;
         f.L_low = f.L_high = f.L_last = -1;
+        f.res = resident_size(b, f.n, b->nv[s] > 0, fastdiv) ? 1 : 0;
+        if (f.res) resident.push_back({(int)s, f.n});
         S = f;
     }
+    b->phased = (int64_t)resident.size() < b->nsys;
+    if (resident_table(b, resident)) return -1;
     DPM_HIP(hipMemcpyAsync(d.sys, b->hsys.data(), sizeof(BSys) * b->nsys, hipMemcpyHostToDevice,
                            b->stream));
     b->ran = true;
@@ -2180,14 +2289,21 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
     bool all_done = false;
     while (!all_done) {
         while (inflight < 2 && launched < max_batched_steps) {
-            int64_t k = std::min<int64_t>(b->steps_per_graph, max_batched_steps - launched);
-            if (b->use_graph && !b->timing && k == b->steps_per_graph) {
+            // a launch of resident systems alone ends for each system on its own, so it is
+            // long; beside the per-phase kernels it keeps their pace
+            int64_t k = std::min<int64_t>(b->phased ? b->steps_per_graph : RES_STEPS,
+                                          max_batched_steps - launched);
+            if (resident_launch(b, launched, k)) return -1;
+            if (!b->phased) {
+                // nothing else to launch
+            } else if (b->use_graph && !b->timing && k == b->steps_per_graph) {
                 if (ensure_batch_graph(b, k)) return -1;
                 DPM_HIP(hipGraphLaunch(b->exec, b->stream));
             } else {
                 for (int64_t s = 0; s < k; ++s) enqueue_batch_step(b);
                 if (check_launch()) return -1;
             }
+            if (resident_join(b)) return -1;
             int ws = (slot + inflight) % 2;
             DPM_HIP(hipMemcpyAsync(b->hflags + 4 * ws, d.flags, 4 * sizeof(int),
                                    hipMemcpyDeviceToHost, b->stream));
@@ -2211,8 +2327,12 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
     }
     DPM_HIP(hipStreamSynchronize(b->stream));
     batch_collect_timing(b);
-    if (steps_done) *steps_done = finished_steps;
     BCOPY(b->hsys.data(), d.sys, sizeof(BSys) * b->nsys, hipMemcpyDeviceToHost);
+    if (!b->phased && all_done) {  // the steps until the last system finished
+        finished_steps = 0;
+        for (auto& S : b->hsys) finished_steps = std::max<int64_t>(finished_steps, S.done_step);
+    }
+    if (steps_done) *steps_done = finished_steps;
     for (int64_t s = 0; s < b->nsys; ++s) {
         const BSys& S = b->hsys[s];
         dpm_jam_result& r = out[s];
@@ -2482,7 +2602,7 @@ constexpr int64_t SLOT_BYTES = 32 + 32 + 16 + 16 + 16 + 8 + 4 + 4 + 32 * 4 + 8;
 constexpr int64_t RIGID_SLOT_BYTES = 4 + 4 + 8 * 5 + 16 * 4 + 16 + 4;
 constexpr int64_t VSLOT_BYTES = 4 + 4 + 4 + 32 * 4 + 16 * 2;
 
-static void serve_upload_tiles(dpm_server* sv) {
+static int serve_upload_tiles(dpm_server* sv) {
     dpm_batch* b = sv->b;
     sv->tiles_host.clear();
     for (size_t s = 0; s < sv->sys_req.size(); ++s) {
@@ -2492,8 +2612,16 @@ static void serve_upload_tiles(dpm_server* sv) {
             sv->tiles_host.push_back(make_int2((int)s, (int)(q.off + t)));
     }
     std::vector<int2> ct;
-    for (size_t s = 0; s < sv->sys_req.size(); ++s)
-        if (sv->sys_req[s]) cell_tiles(ct, (int)s, (int)sv->reqs.at(sv->sys_req[s]).n);
+    std::vector<std::pair<int, int64_t>> resident;
+    b->phased = false;
+    for (size_t s = 0; s < sv->sys_req.size(); ++s) {
+        if (!sv->sys_req[s]) continue;
+        const dpm_server_req& q = sv->reqs.at(sv->sys_req[s]);
+        cell_tiles(ct, (int)s, (int)q.n);
+        if (resident_size(b, q.n, q.kind == DPM_BUMPY, true)) resident.push_back({(int)s, q.n});
+        else b->phased = true;
+    }
+    if (resident_table(b, resident)) return -1;
     // the bound of batch_alloc: ct never exceeds d.nctiles entries
     int nt[2] = {(int)sv->tiles_host.size(), (int)std::min<long long>(ct.size(), b->d.nctiles)};
     if (nt[0])
@@ -2504,6 +2632,7 @@ static void serve_upload_tiles(dpm_server* sv) {
                                       hipMemcpyHostToDevice, b->stream));
     (void)bsync(b, hipMemcpyAsync(b->d.flags + 4, nt, 2 * sizeof(int), hipMemcpyHostToDevice,
                                   b->stream));
+    return 0;
 }
 
 // first fit in a map of free ranges (first slot -> length)
@@ -2596,8 +2725,7 @@ static int serve_collect(dpm_server* sv) {
         changed = true;
     }
     sv->seen_done = total;
-    if (changed) serve_upload_tiles(sv);
-    return 0;
+    return changed ? serve_upload_tiles(sv) : 0;
 }
 
 // The request's particles (and a rigid system's angles, vertex layout and vertex ring)
@@ -2652,6 +2780,7 @@ static int serve_place(dpm_server* sv, dpm_server_req& q, int s) {
     f.jphase = q.mode == DPM_REQ_MINIMIZE ? BJ_MIN : BJ_DECOMP;
     f.status = 1;
     f.L_low = f.L_high = f.L_last = -1;
+    f.res = resident_size(b, q.n, rigid, true) ? 1 : 0;
     BCOPY(d.sys + s, &f, sizeof(BSys), hipMemcpyHostToDevice);
     return 0;
 }
@@ -2691,8 +2820,7 @@ static int serve_admit(dpm_server* sv) {
         tiles_changed = true;
         it = sv->queue.erase(it);
     }
-    if (tiles_changed) serve_upload_tiles(sv);
-    return 0;
+    return tiles_changed ? serve_upload_tiles(sv) : 0;
 }
 
 }  // namespace dpm
@@ -2870,7 +2998,9 @@ int dpm_server_progress(dpm_server* sv, int64_t batched_steps, int64_t* finished
         active = sv->active;
     }
     if (active > 0 && batched_steps > 0) {
-        int64_t done = 0;
+        // the resident systems run their steps beside the others'
+        if (resident_launch(b, 0, std::min<int64_t>(batched_steps, INT_MAX))) return -1;
+        int64_t done = b->phased ? 0 : batched_steps;
         while (done < batched_steps) {
             int64_t k = std::min<int64_t>(b->steps_per_graph, batched_steps - done);
             if (b->use_graph && k == b->steps_per_graph) {
@@ -2882,6 +3012,7 @@ int dpm_server_progress(dpm_server* sv, int64_t batched_steps, int64_t* finished
             }
             done += k;
         }
+        if (resident_join(b)) return -1;
         DPM_HIP(hipStreamSynchronize(b->stream));
         std::lock_guard<std::mutex> g(sv->mu);
         if (serve_collect(sv) || serve_admit(sv)) return -1;
