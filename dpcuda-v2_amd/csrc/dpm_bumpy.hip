@@ -491,12 +491,12 @@ __global__ void k_bumpy_init_vertices(Dev d, double rv) {
 // control block, so a halted or finished loop turns the rest of the chunk into no-ops:
 //   k_bfire_move      particles: [uphill: drift(-dt/2), zero v and w] + kick(dt/2) + mix
 //                     + drift(dt), and the rebuild requests of the new positions
-//   k_bfire_vertices  vertices: the rotations of those moves, in the same order
-//   k_bfire_decide    the neighbour check of the step: a list rebuild runs inside the
-//                     chunk, a cell rebuild halts the loop until the chunk's end
+//   k_bfire_vertices  vertices: the rotations of those moves, in the same order; one thread
+//                     makes the neighbour check of the step: a list rebuild runs inside the
+//                     chunk
 //   k_build_cell / k_build_verlet, k_bumpy_vertex_build   (gated on that decision)
-//   k_bfire_forces    an in-chunk rebuild that overflowed the capacity halts the loop;
-//                     else vertex forces, torques, energies (kernelCalcRigidBumpyForces1)
+//   k_bfire_forces    a step that needs a cell rebuild, or whose rebuilt rows overflowed the
+//                     capacity, halts the loop until the chunk's end; else vertex forces, torques, energies (kernelCalcRigidBumpyForces1)
 //                     and their per-particle sums (kernelCalcRigidBumpyParticleForces1),
 //                     one pass
 //   k_bfire_partials  kick(dt/2), then the chunk partials of P = F.v + tau.w, PE and
@@ -506,7 +506,41 @@ __device__ __forceinline__ bool bfire_skip(const Dev& d, int gate) {
     const Ctl* c = d.ctl;
     if (gate == G_NORMAL) return c->halt || d.fire->done;
     if (gate == G_RESUME) return !c->halt || !resumable(d) || c->halt_mode != H_FIRE;
+    if (gate == G_STEP) return c->halt;
     return false;
+}
+
+// The list rebuild of step pos, decided by one thread of the vertex pass (whose other threads
+// do not read the words it writes) for the gated builds behind it: Particle::
+// checkForNeighborUpdate (particle.cu:1137-1161) on the requests the move recorded.  A step
+// that needs cells + list builds nothing here: its force pass halts the loop.
+__device__ __forceinline__ void bstep_decide(Ctl* c, int pos) {
+    const int need = pending_rebuild(c, c->epoch, pos);
+    c->kind = need == 1;
+    if (need == 1) {
+        c->max_nnum = 0;
+        c->max_vnum = 0;
+        c->n_rebuilds += 1;
+    }
+}
+
+// Whether step pos halts at its force pass, the same verdict in every block (the words read
+// are not written while the pass runs, but for halt): it needs cells + list, or the rows it
+// rebuilt did not fit (the host regrows the lists).  The chain at the chunk's end rebuilds
+// and finishes the step.
+__device__ __forceinline__ bool bstep_halts(const Dev& d, int pos) {
+    Ctl* c = d.ctl;
+    const bool cells = pending_rebuild(c, c->epoch, pos) >= 2;
+    const bool over = c->kind >= 1 && (c->max_nnum > d.cap || c->max_vnum > d.vcap);
+    if (!cells && !over) return false;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (over) c->overflow = 1;
+        c->halt_pos = pos;
+        c->halt_mode = H_FIRE;
+        c->halt_kind = cells ? 2 : 1;
+        c->halt = 1;
+    }
+    return true;
 }
 
 // The rigid moves of Fire::step for particle i (src/integrator/fire.cu:20-40 with the
@@ -562,8 +596,13 @@ __global__ __launch_bounds__(BLOCK) void k_bfire_move(Dev d, NbrParams nb, int p
     disp_flags(d, nb, nd, cd, pos & 1, stamp(e, pos));  // maxima: k_disp_partials at the end
 }
 
-__global__ void k_bfire_vertices(Dev d) {
-    if (d.ctl->halt || d.fire->done) return;
+// (lists: the neighbour method rebuilds; one thread decides this step's rebuild)
+__global__ __launch_bounds__(BLOCK) void k_bfire_vertices(Dev d, int pos, int lists) {
+    if (d.ctl->halt || d.fire->done) {
+        if (lists && blockIdx.x == 0 && threadIdx.x == 0) d.ctl->kind = 0;
+        return;
+    }
+    if (lists && blockIdx.x == 0 && threadIdx.x == 0) bstep_decide(d.ctl, pos);
     int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     if (v >= d.Nv) return;
     int p = d.vpart[v];
@@ -575,45 +614,96 @@ __global__ void k_bfire_vertices(Dev d) {
                                  r0.y, r1.x, r1.y, uphill);
 }
 
-// Particle::checkForNeighborUpdate of the step (particle.cu:1137-1161) from the
-// requests k_bfire_move recorded: 1 = list (rebuilt in the chunk), 2 = cells + list
-// (the loop halts; the chain at the chunk's end rebuilds and finishes the step).
-__global__ void k_bfire_decide(Dev d, int pos) {
-    Ctl* c = d.ctl;
-    if (c->halt || d.fire->done) {
-        c->kind = 0;
-        return;
-    }
-    int need = pending_rebuild(c, c->epoch, pos);
-    if (need >= 2) {
-        c->halt = 1;
-        c->halt_pos = pos;
-        c->halt_mode = H_FIRE;
-        c->halt_kind = 2;
-        c->kind = 0;
-        return;
-    }
-    c->kind = need;
-    if (need == 1) {
-        c->max_nnum = 0;
-        c->max_vnum = 0;
-        c->n_rebuilds += 1;
-    }
+// The two-pass force phase's halting test (k_bfire_forces makes it itself).
+__global__ void k_bfire_check(Dev d, int pos, int gate) {
+    if (!bfire_skip(d, gate)) (void)bstep_halts(d, pos);
 }
 
-// An in-chunk list rebuild whose rows did not fit: halt with the step unfinished; the
-// host regrows the lists, rebuilds and finishes the step (fix_overflow).
-__global__ void k_bfire_check(Dev d, int pos) {
+// ---- NVE::step (src/integrator/nve.cu:15-25) of rigid bumpy systems, on the device: per step
+//   k_bnve_move      [closing kick of the step before] + kick(dt/2) + drift(dt), the turn's
+//                    sine and cosine, the rebuild requests
+//   k_bnve_vertices  the vertices' rotation; one thread decides the list rebuild
+//   list and vertex-row builds (gated on that decision), k_bfire_forces
+// with the closing kick of a chunk's last step in k_bnve_kick.  Halts, the rebuild chain and
+// the capacity's regrowth are those of the rigid FIRE loop.  Bound by launch latency up to some thousand particles: 3,001 particles, 200 steps take 5.6 ms (27.5 ms with
+// a dozen stand-alone launches and a blocking readback per step).
+__device__ __forceinline__ void rigid_kick(double2& v, double& w, double2 f, double t, double moi,
+                                           double m, double hdt, int rotation) {
+    // kernelUpdateRigidVelocities, rigid_bumpy/kernels.cu:123-150
+    if (rotation) w += t * hdt / moi;
+    else w = 0.0;
+    v.x += f.x * hdt / m;
+    v.y += f.y * hdt / m;
+}
+
+__global__ __launch_bounds__(BLOCK) void k_bnve_move(Dev d, NbrParams nb, double dt, int pos,
+                                                     int rotation, int close) {
     Ctl* c = d.ctl;
-    if (c->kind < 1) return;
-    if (c->max_nnum > d.cap || c->max_vnum > d.vcap) {
-        c->overflow = 1;
-        c->halt = 1;
-        c->halt_pos = pos;
-        c->halt_mode = H_FIRE;
-        c->halt_kind = 1;
+    if (c->halt) return;
+    const long long e = c->epoch;
+    int tile;
+    const int64_t i = particle_of_thread(tile);
+    double nd = 0.0, cd = 0.0;
+    if (i < d.N) {
+        double4 q = d.P0[i];
+        double2 v = d.vel[i];
+        const double2 f = d.frc[i];
+        const double t = d.torque[i], moi = d.moi[i], hdt = 0.5 * dt;
+        double w = d.omega[i];
+        if (close) rigid_kick(v, w, f, t, moi, q.w, hdt, rotation);
+        rigid_kick(v, w, f, t, moi, q.w, hdt, rotation);
+        // kernelUpdateRigidPositions, rigid_bumpy/kernels.cu:21-78
+        d.lpos[i] = make_double2(q.x, q.y);
+        const double ddx = v.x * dt, ddy = v.y * dt, dda = w * dt;
+        d.dth[i] = dda;
+        double s1, c1;
+        dpm_sincos(dda, &s1, &c1);
+        d.rot1[i] = make_double2(s1, c1);
+        q.x = q.x + ddx;
+        q.y = q.y + ddy;
+        d.P0[i] = q;
+        d.angle[i] = d.angle[i] + dda;
+        d.vel[i] = v;
+        d.omega[i] = w;
+        disp_of(d, i, q.x, q.y, nd, cd);
     }
-    c->kind = 0;
+    disp_flags(d, nb, nd, cd, pos & 1, stamp(e, pos));
+    if (close && blockIdx.x == 0 && threadIdx.x == 0) c->progress = pos;
+}
+
+__global__ __launch_bounds__(BLOCK) void k_bnve_vertices(Dev d, int pos, int lists) {
+    if (d.ctl->halt) {
+        if (lists && blockIdx.x == 0 && threadIdx.x == 0) d.ctl->kind = 0;
+        return;
+    }
+    if (lists && blockIdx.x == 0 && threadIdx.x == 0) bstep_decide(d.ctl, pos);
+    const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (v >= d.Nv) return;
+    // kernelTranslateAndRotateVertices1, rigid_bumpy/kernels.cu:152-201
+    const int p = d.vpart[v];
+    const double4 n = d.P0[p];
+    const double2 o = d.lpos[p], x = d.vpos[v], r = d.rot1[p];
+    const double rx = x.x - o.x, ry = x.y - o.y;
+    const double rxr = rx * r.y - ry * r.x;
+    const double ryr = rx * r.x + ry * r.y;
+    d.vpos[v] = make_double2(n.x + rxr, n.y + ryr);
+}
+
+// The closing kick of a chunk's last step, or (G_RESUME) of a halted step the chain finishes.
+__global__ __launch_bounds__(BLOCK) void k_bnve_kick(Dev d, double dt, int rotation, int progress,
+                                                     int gate) {
+    if (bfire_skip(d, gate)) return;
+    const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (i == 0) {
+        if (gate == G_RESUME) d.ctl->progress += 1;
+        else d.ctl->progress = progress;
+    }
+    if (i >= d.N) return;
+    double2 v = d.vel[i];
+    double w = d.omega[i];
+    rigid_kick(v, w, d.frc[i], d.torque[i], d.moi[i], d.P0[i].w, 0.5 * dt, rotation);
+    d.vel[i] = v;
+    d.omega[i] = w;
 }
 
 __global__ __launch_bounds__(BLOCK) void k_bfire_vforce(Dev d, PairParams p, double rv,
@@ -656,19 +746,7 @@ __global__ __launch_bounds__(bf_threads<LDSV>(), (bf_waves<LDSV, HOT>())) void k
     Dev d, PairParams p, double rv, int gate, int check_pos) {
     constexpr int NT = bf_threads<LDSV>();
     if (bfire_skip(d, gate)) return;
-    if (check_pos >= 0) {  // k_bfire_check's test, made by every block (same words read)
-        Ctl* c = d.ctl;
-        if (c->kind >= 1 && (c->max_nnum > d.cap || c->max_vnum > d.vcap)) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                c->overflow = 1;
-                c->halt = 1;
-                c->halt_pos = check_pos;
-                c->halt_mode = H_FIRE;
-                c->halt_kind = 1;
-            }
-            return;
-        }
-    }
+    if (check_pos >= 0 && bstep_halts(d, check_pos)) return;
     __shared__ double sv[4][LDSV];       // per vertex: fx, fy, torque, energy
     __shared__ double sres[4][BF_TILE];  // per particle: the sums of those
     // XCD-aware tile order: each XCD's L2 holds the vertex positions its tiles gather
@@ -868,6 +946,7 @@ __global__ __launch_bounds__(BLOCK) void k_bfire_reduce(Dev d, int kick, int gat
 }
 
 // ------------------------------------------------------------------ host side
+bool bumpy_enqueue_loop_forces(dpm_system* s, int gate, int check_pos, int kick = 0);
 int bumpy_alloc(dpm_system* s) {
     Dev& d = s->d;
     int64_t n = s->N, v = s->Nv;
@@ -1025,20 +1104,62 @@ int bumpy_contacts(dpm_system* s) {
     return check_launch();
 }
 
-// NVE::step for rigid bodies, one step at a time (src/integrator/nve.cu:15-25)
-int bumpy_nve_run(dpm_system* s, double dt, int64_t n) {
-    for (int64_t k = 0; k < n; ++k) {
-        if (bumpy_kick(s, 0.5 * dt) || bumpy_drift(s, dt) || check_and_rebuild(s, nullptr) ||
-            dpm_zero_forces(s) || bumpy_forces(s, 1) || bumpy_kick(s, 0.5 * dt))
-            return -1;
+static bool bumpy_lists(const dpm_system* s) {
+    return s->method == DPM_NBR_CELL || s->method == DPM_NBR_VERLET;
+}
+
+// The step's list rebuilds, gated on the vertex pass's decision.
+static void bumpy_enqueue_step_lists(dpm_system* s) {
+    if (!bumpy_lists(s)) return;
+    Timed t(s, DPM_K_REBUILD);
+    enqueue_list_build(s, 1);
+    bumpy_enqueue_vertex_build(s, 1);
+}
+
+// c steps of the device-resident NVE loop (positions 0..c-1); the chain follows.
+void bumpy_enqueue_nve_steps(dpm_system* s, double dt, int64_t c) {
+    const Dev& d = s->d;
+    const NbrParams nb = nbr_params(s);
+    const int lists = bumpy_lists(s);
+    for (int64_t k = 0; k < c; ++k) {
+        {
+            Timed t(s, DPM_K_DRIFT);
+            hipLaunchKernelGGL(k_bnve_move, pgrid(s->N), dim3(BLOCK), 0, s->stream, d, nb, dt,
+                               (int)k, (int)s->rotation, (int)(k > 0));
+            hipLaunchKernelGGL(k_bnve_vertices, pgrid(s->Nv), dim3(BLOCK), 0, s->stream, d,
+                               (int)k, lists);
+        }
+        bumpy_enqueue_step_lists(s);
+        Timed t(s, DPM_K_FORCE);
+        bumpy_enqueue_loop_forces(s, G_STEP, lists ? (int)k : -1);
     }
+    hipLaunchKernelGGL(k_bnve_kick, pgrid(s->N), dim3(BLOCK), 0, s->stream, d, dt,
+                       (int)s->rotation, (int)c, (int)G_STEP);
+}
+
+// The rest of a halted NVE step, behind the chain's rebuild.
+void bumpy_enqueue_nve_resume(dpm_system* s, double dt) {
+    bumpy_enqueue_loop_forces(s, G_RESUME, -1);
+    hipLaunchKernelGGL(k_bnve_kick, pgrid(s->N), dim3(BLOCK), 0, s->stream, s->d, dt,
+                       (int)s->rotation, 0, (int)G_RESUME);
+}
+
+// One NVE::step for rigid bodies (src/integrator/nve.cu:15-25) by the stand-alone pieces: the
+// last step of a run, which leaves the per-vertex forces that a later dpm_compute_forces
+// without dpm_zero_forces adds to.
+int bumpy_nve_step(dpm_system* s, double dt) {
+    if (bumpy_kick(s, 0.5 * dt) || bumpy_drift(s, dt) || check_and_rebuild(s, nullptr) ||
+        dpm_zero_forces(s) || bumpy_forces(s, 1) || bumpy_kick(s, 0.5 * dt))
+        return -1;
     DPM_HIP(hipStreamSynchronize(s->stream));
     return 0;
 }
 
 
 // ---- device-resident FIRE (the loop driver is minimize_fire in dpm_core.hip) ----
-void bumpy_enqueue_fire_forces(dpm_system* s, int kick, int gate, int check_pos) {
+// Forces, torques and energies of the particles (the two-pass form also leaves the chunk
+// partials).  check_pos >= 0: the position whose halting test the pass makes.
+bool bumpy_enqueue_loop_forces(dpm_system* s, int gate, int check_pos, int kick) {
     PairParams p = params_of(s);
     if (BF_TILE + s->nv_max - 1 <= BF_LDS) {
         unsigned nb = (unsigned)((s->Nv + BF_TILE - 1) / BF_TILE);
@@ -1048,38 +1169,37 @@ void bumpy_enqueue_fire_forces(dpm_system* s, int kick, int gate, int check_pos)
                        : (hot ? k_bfire_forces<BF_LDS, true> : k_bfire_forces<BF_LDS, false>);
         hipLaunchKernelGGL(k, dim3(nb), dim3(small ? bf_threads<BF_LDS_SMALL>() : bf_threads<BF_LDS>()),
                            0, s->stream, s->d, p, s->rv, gate, check_pos);
-        hipLaunchKernelGGL(k_bfire_partials, dim3((unsigned)s->nblk), dim3(BLOCK), 0, s->stream,
-                           s->d, gate, kick, (int)s->rotation);
-        return;
+        return true;
     }
     if (check_pos >= 0)
-        hipLaunchKernelGGL(k_bfire_check, dim3(1), dim3(1), 0, s->stream, s->d, check_pos);
+        hipLaunchKernelGGL(k_bfire_check, dim3(1), dim3(1), 0, s->stream, s->d, check_pos, gate);
     hipLaunchKernelGGL(k_bfire_vforce, pgrid(s->Nv), dim3(BLOCK), 0, s->stream, s->d, p, s->rv,
                        gate);
     hipLaunchKernelGGL(k_bfire_reduce, dim3((unsigned)s->nblk), dim3(BLOCK), 0, s->stream, s->d,
                        kick, gate, (int)s->rotation);
+    return false;
+}
+
+void bumpy_enqueue_fire_forces(dpm_system* s, int kick, int gate, int check_pos) {
+    if (bumpy_enqueue_loop_forces(s, gate, check_pos, kick))
+        hipLaunchKernelGGL(k_bfire_partials, dim3((unsigned)s->nblk), dim3(BLOCK), 0, s->stream,
+                           s->d, gate, kick, (int)s->rotation);
 }
 
 void bumpy_enqueue_fire_step(dpm_system* s, int pos) {
     const Dev& d = s->d;
     NbrParams nb = nbr_params(s);
     hipStream_t st = s->stream;
+    const int lists = bumpy_lists(s);
     {
         Timed t(s, DPM_K_DRIFT);
         hipLaunchKernelGGL(k_bfire_move, pgrid(s->N), dim3(BLOCK), 0, st, d, nb, pos,
                            (int)s->rotation);
-        hipLaunchKernelGGL(k_bfire_vertices, pgrid(s->Nv), dim3(BLOCK), 0, st, d);
+        hipLaunchKernelGGL(k_bfire_vertices, pgrid(s->Nv), dim3(BLOCK), 0, st, d, pos, lists);
     }
-    if (s->method == DPM_NBR_CELL || s->method == DPM_NBR_VERLET) {
-        Timed t(s, DPM_K_REBUILD);
-        hipLaunchKernelGGL(k_bfire_decide, dim3(1), dim3(1), 0, st, d, pos);
-        enqueue_list_build(s, 1);
-        bumpy_enqueue_vertex_build(s, 1);
-    }
+    bumpy_enqueue_step_lists(s);
     Timed t(s, DPM_K_FORCE);
-    // the overflow test of an in-step rebuild (k_bfire_check) runs in the force kernel
-    bumpy_enqueue_fire_forces(s, 1, G_NORMAL,
-                              s->method == DPM_NBR_CELL || s->method == DPM_NBR_VERLET ? pos : -1);
+    bumpy_enqueue_fire_forces(s, 1, G_NORMAL, lists ? pos : -1);
 }
 
 

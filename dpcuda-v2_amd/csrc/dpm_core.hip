@@ -1663,7 +1663,8 @@ static void enqueue_rebuild(dpm_system* s, int gated) {
     if (s->kind == DPM_BUMPY) bumpy_enqueue_vertex_build(s, gated);
 }
 
-// The halted step's remaining work. resume: 0 none, 1 NVE, 2 FIRE, 3 rigid bumpy FIRE.
+// The halted step's remaining work. resume: 0 none, 1 NVE, 2 FIRE, 3 rigid bumpy FIRE, 4 rigid
+// bumpy NVE.
 static void enqueue_resume(dpm_system* s, int resume, double dt) {
     const Dev& d = s->d;
     NbrParams nb = nbr_params(s);
@@ -1681,6 +1682,8 @@ static void enqueue_resume(dpm_system* s, int resume, double dt) {
     } else if (resume == 3) {  // rigid bumpy FIRE
         bumpy_enqueue_fire_forces(s, 1, G_RESUME);
         hipLaunchKernelGGL(k_fire_ctl, dim3(1), dim3(WAVE), 0, st, d, 0, 0, (int)G_RESUME);
+    } else if (resume == 4) {
+        bumpy_enqueue_nve_resume(s, dt);
     }
 }
 
@@ -1830,6 +1833,11 @@ static void bumpy_fire_chunk(dpm_system* s, double, int64_t c) {
     enqueue_chain(s, 3, 0.0);
 }
 
+static void bumpy_nve_chunk(dpm_system* s, double dt, int64_t c) {
+    bumpy_enqueue_nve_steps(s, dt, c);
+    enqueue_chain(s, 4, dt);
+}
+
 static void recovery_fill(dpm_system* s, double dt, int64_t) { enqueue_chain(s, 1, dt); }
 
 // The closing force + kick of an NVE run (the last step's second half); it records in
@@ -1943,7 +1951,7 @@ static int run_chunks(dpm_system* s, int64_t total, double dt, int resume, Chunk
                 need_recovery = false;
             } else if (planned < total) {
                 int64_t c = std::min<int64_t>(cur, total - planned);
-                if (graphs && (tail || c == cur)) {
+                if (graphs && (tail || resume == 4 || c == cur)) {
                     c = graph_len(c);
                     if (ensure_graph(s, cache, c, dt, chunk_fn)) return -1;
                     DPM_HIP(hipGraphLaunch(cache[c].exec, s->stream));
@@ -2025,7 +2033,11 @@ static int run_chunks(dpm_system* s, int64_t total, double dt, int resume, Chunk
 }
 
 int nve_run(dpm_system* s, double dt, int64_t n) {
-    if (s->kind == DPM_BUMPY) return bumpy_nve_run(s, dt, n);
+    if (s->kind == DPM_BUMPY && (n <= 1 || !s->nbr_ready)) {
+        for (int64_t k = 0; k < n; ++k)
+            if (bumpy_nve_step(s, dt)) return -1;
+        return 0;
+    }
     if (!s->nbr_ready) {
         set_error("nve_run: neighbour list not initialised");
         return -1;
@@ -2034,6 +2046,11 @@ int nve_run(dpm_system* s, double dt, int64_t n) {
     const Dev& d = s->d;
     hipStream_t st = s->stream;
     hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(1), 0, st, d, 0);
+    if (s->kind == DPM_BUMPY) {
+        if (check_launch()) return -1;
+        if (run_chunks(s, n - 1, dt, 4, bumpy_nve_chunk, s->nve_graphs, false, false)) return -1;
+        return bumpy_nve_step(s, dt);
+    }
     {  // opening kick + drift of the first step; its request is checked at position 0
         Timed t(s, DPM_K_DRIFT);
         hipLaunchKernelGGL(k_nve_kick_drift, pgrid(s->N), dim3(BLOCK), 0, st, d, nbr_params(s),

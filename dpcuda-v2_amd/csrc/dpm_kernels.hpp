@@ -40,8 +40,9 @@ enum MaxWhat { M_ND = 0, M_CD, M_F2, M_T2 };
 
 // How a loop kernel decides whether to run: G_NORMAL inside a chunk (skip after a
 // halt, halt on a matching rebuild request), G_RESUME in the rebuild chain (run only
-// to finish a halted step), G_ALWAYS unconditionally.
-enum Gate { G_NORMAL = 0, G_RESUME = 1, G_ALWAYS = 2 };
+// to finish a halted step), G_ALWAYS unconditionally, G_STEP inside a chunk of the rigid NVE
+// loop (skip after a halt; the FIRE state is not looked at).
+enum Gate { G_NORMAL = 0, G_RESUME = 1, G_ALWAYS = 2, G_STEP = 3 };
 
 // ---- control-block helpers shared by the loop kernels ----
 constexpr long long STAMP_STRIDE = 8192;  // > any chunk length
@@ -210,7 +211,9 @@ int bumpy_adam_update(dpm_system* s, double alpha, double b1, double b2, double 
 int bumpy_mix(dpm_system* s, double alpha);
 int bumpy_stress(dpm_system* s);
 int bumpy_contacts(dpm_system* s);
-int bumpy_nve_run(dpm_system* s, double dt, int64_t n);
+int bumpy_nve_step(dpm_system* s, double dt);
+void bumpy_enqueue_nve_steps(dpm_system* s, double dt, int64_t c);
+void bumpy_enqueue_nve_resume(dpm_system* s, double dt);
 void bumpy_enqueue_fire_forces(dpm_system* s, int kick, int gate, int check_pos = -1);
 void bumpy_enqueue_fire_step(dpm_system* s, int pos);
 int bumpy_snapshot(dpm_system* s, bool save);
