@@ -696,12 +696,6 @@ __global__ void k_fill_int(int* a, int v, int64_t n, const Ctl* gate, int gated)
     if (i < n) a[i] = v;
 }
 
-__device__ __forceinline__ int cell_coord(double pos, double cs, int n) {
-    // getPBCCellIndex, include/particles/base/kernels.cuh:285-301
-    long long idx = (long long)floor(pos / cs);
-    return (int)(idx >= 0 ? idx % n : (idx % n + n) % n);
-}
-
 // kernelGetCellIndexForParticle (base/kernels.cu:309-330) + counting-sort histogram
 __global__ void k_cell_bin(Dev d, NbrParams nb, int gated) {
     GATE_CELL;
@@ -1252,11 +1246,6 @@ __global__ __launch_bounds__(BLOCK) void k_fire_force(Dev d, PairParams p, int p
     if (threadIdx.x == 0) P[3 * nc + blockIdx.x] = b;
 }
 
-__device__ __forceinline__ void fire_finish(const Dev& d, FireCtl* F) {
-    F->done = 1;
-    d.ctl->done = 1;
-}
-
 // init: 1 = minimizeFire's prologue (records the first average energy)
 __global__ void k_fire_ctl(Dev d, int init, int pos, int gate) {
     Ctl* c = d.ctl;
@@ -1291,57 +1280,9 @@ __global__ void k_fire_ctl(Dev d, int init, int pos, int gate) {
         if (gate == G_RESUME) c->progress += 1;  // the finished halted step
         else c->progress = pos + 1;
     }
-    double avg = pe / F->dof;
-    F->fmax_sq = fm;
-    F->avg_pe = avg;
-    if (init) {
-        F->last_avg_pe = avg;
-        if (F->max_steps <= 0) {
-            fire_finish(d, F);
-            return;
-        }
-    } else {
-        // minimizeFire stop test (src/routines/minimization.cu:99-105)
-        double diff = fabs(avg / F->last_avg_pe - 1);
-        F->last_avg_pe = avg;
-        bool fok = F->fmax_target_sq > 0.0 && fm < F->fmax_target_sq;
-        F->step += 1;
-        if (diff < F->avg_pe_diff_target || avg < F->avg_pe_target || fok) {
-            F->converged = 1;
-            fire_finish(d, F);
-            return;
-        }
-        if (F->step >= F->max_steps) {
-            fire_finish(d, F);
-            return;
-        }
-    }
-    // Fire::step decision for the next iteration (src/integrator/fire.cu:14-33);
-    // RigidBumpy::getPowerFire adds sum(tau*w) (rigid_bumpy.cu:1181-1191)
-    double power = px + py;
-    if (d.vpos) power = power + ptw;
-    F->power = power;
-    if (power > 0) {
-        F->n_good++;
-        F->n_bad = 0;
-        if (F->n_good > 5) {
-            F->dt = fmin(F->dt * 1.1, F->dt_max);
-            F->alpha *= 0.99;
-        }
-        F->uphill = 0;
-    } else {
-        F->n_good = 0;
-        F->n_bad++;
-        if (F->n_bad > 10) {
-            F->stopped = 1;
-            F->step += 1;  // the stopped step counts as executed
-            fire_finish(d, F);
-            return;
-        }
-        F->dt = fmax(F->dt * 0.5, F->dt_min);
-        F->alpha = F->alpha_init;
-        F->uphill = 1;
-    }
+    const bool done = init ? fire_begin(*F, px, py, pe, fm, d.vpos ? &ptw : nullptr)
+                           : fire_advance(*F, px, py, pe, fm, d.vpos ? &ptw : nullptr);
+    if (done) c->done = 1;
 }
 
 }  // namespace dpm
@@ -1838,6 +1779,23 @@ static void bumpy_nve_chunk(dpm_system* s, double dt, int64_t c) {
     enqueue_chain(s, 4, dt);
 }
 
+// Resident loops: one launch runs the chunk's steps, k_chunk_end publishes their outcome.
+// RESIDENT_CHUNK launches' worth of the configured chunk at once: a launch reads the system's
+// state and near rows in about the time of a few steps.
+constexpr int64_t RESIDENT_CHUNK = 8;
+
+static void resident_nve_chunk(dpm_system* s, double dt, int64_t c) {
+    Timed t(s, DPM_K_FORCE);
+    resident_nve(s, dt, c);
+    hipLaunchKernelGGL(k_chunk_end, dim3(1), dim3(WAVE), 0, s->stream, s->d);
+}
+
+static void resident_fire_chunk(dpm_system* s, double, int64_t c) {
+    Timed t(s, DPM_K_FORCE);
+    resident_fire(s, c);
+    hipLaunchKernelGGL(k_chunk_end, dim3(1), dim3(WAVE), 0, s->stream, s->d);
+}
+
 static void recovery_fill(dpm_system* s, double dt, int64_t) { enqueue_chain(s, 1, dt); }
 
 // The closing force + kick of an NVE run (the last step's second half); it records in
@@ -1902,9 +1860,11 @@ static int ensure_all_graphs(dpm_system* s, std::map<int64_t, Graph>& cache, dou
 // reports it applied (`closed`).  A tail launched behind a halted step does nothing and
 // is enqueued again after the recovery; a tail that halts itself is finished by the
 // recovery chain, which then closes the run.
+//
+// `direct`: chunks of that many steps, launched without a graph (the resident loops).
 static int run_chunks(dpm_system* s, int64_t total, double dt, int resume, ChunkFn chunk_fn,
                       std::map<int64_t, Graph>& cache, bool stop_on_done, bool host_recovery,
-                      TailFn tail = nullptr) {
+                      TailFn tail = nullptr, int64_t direct = 0) {
     enum { U_CHUNK = 0, U_RECOVERY = 1, U_TAIL = 2 };
     struct Unit {
         int64_t c;       // steps planned (0 for a recovery or tail unit)
@@ -1912,14 +1872,15 @@ static int run_chunks(dpm_system* s, int64_t total, double dt, int resume, Chunk
         int kind;
         bool covered;    // launched before a recovery that finishes its halted step
     };
-    const bool graphs = s->use_graph && s->timing != 1;
+    const bool graphs = s->use_graph && s->timing != 1 && direct == 0;
+    const int64_t longest = direct ? direct : s->chunk;
     if (graphs && tail && ensure_all_graphs(s, cache, dt, chunk_fn)) return -1;
     std::deque<Unit> q;
     int64_t done = 0, planned = 0;
     int next_slot = 0;  // publication sequence of the next unit (k_ctl_reset starts it at 0)
     bool need_recovery = false;
     bool closed = tail == nullptr, tail_queued = false;
-    int64_t cur = s->chunk;
+    int64_t cur = longest;
     auto recovering = [&q] {
         for (auto& x : q)
             if (x.kind == U_RECOVERY) return true;
@@ -2021,9 +1982,9 @@ static int run_chunks(dpm_system* s, int64_t total, double dt, int resume, Chunk
         if (stop_on_done && hc.done) break;
         if (f.kind == U_CHUNK && f.c > 0) {
             if (hc.last_progress < f.c)
-                cur = std::min<int64_t>(s->chunk, pow2_at_least(2 * (hc.last_progress + 1)));
+                cur = std::min<int64_t>(longest, pow2_at_least(2 * (hc.last_progress + 1)));
             else
-                cur = std::min<int64_t>(s->chunk, 2 * cur);
+                cur = std::min<int64_t>(longest, 2 * cur);
             cur = std::max<int64_t>(cur, 2);
         }
     }
@@ -2050,6 +2011,11 @@ int nve_run(dpm_system* s, double dt, int64_t n) {
         if (check_launch()) return -1;
         if (run_chunks(s, n - 1, dt, 4, bumpy_nve_chunk, s->nve_graphs, false, false)) return -1;
         return bumpy_nve_step(s, dt);
+    }
+    if (n >= RESIDENT_MIN_STEPS && resident_ok(s)) {
+        if (check_launch()) return -1;
+        return run_chunks(s, n, dt, 1, resident_nve_chunk, s->nve_graphs, false, true, nullptr,
+                          RESIDENT_CHUNK * s->chunk);
     }
     {  // opening kick + drift of the first step; its request is checked at position 0
         Timed t(s, DPM_K_DRIFT);
@@ -2094,7 +2060,11 @@ int minimize_fire(dpm_system* s, const dpm_fire_params* prm, dpm_fire_result* ou
     }
     hipLaunchKernelGGL(k_fire_ctl, dim3(1), dim3(WAVE), 0, st, d, 1, 0, (int)G_ALWAYS);
     if (check_launch()) return -1;
-    if (prm->max_steps > 0 &&
+    if (prm->max_steps >= RESIDENT_MIN_STEPS && resident_ok(s)) {
+        if (run_chunks(s, prm->max_steps, 0.0, 2, resident_fire_chunk, s->fire_graphs, true, true,
+                       nullptr, RESIDENT_CHUNK * s->chunk))
+            return -1;
+    } else if (prm->max_steps > 0 &&
         run_chunks(s, prm->max_steps, 0.0, rigid ? 3 : 2, rigid ? bumpy_fire_chunk : fire_chunk,
                    s->fire_graphs, true, false))
         return -1;

@@ -209,6 +209,56 @@ __device__ __forceinline__ double wave_max(double v) {
     return fmax(v, lane_down<1>(v));
 }
 
+// One stage of a reduction in all four rows of 16 lanes, a sum in rows 0 to 2 and a maximum in
+// row 3
+template <int S>
+__device__ __forceinline__ double rows_down(double v) {
+    const double o = lane_down<S>(v), s = v + o, m = fmax(v, o);
+    return (threadIdx.x % WAVE) < 48 ? s : m;
+}
+
+__device__ __forceinline__ double rows_reduce(double v) {
+    return rows_down<1>(rows_down<2>(rows_down<4>(rows_down<8>(v))));
+}
+
+// wave_tree_sum of a, b and c and wave_max of d in one pass: the row swaps put the halves of two
+// trees side by side, so that 14 moves and 7 additions do for three sums and a maximum (48 and
+// 18 one by one).  Lanes 0, 16, 32 and 48 receive a, c, b and d's results.
+__device__ __forceinline__ double wave_reduce4(double a, double b, double c, double d) {
+    auto swap32 = [](double x, double y, double& lo, double& hi) {
+        const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(y),
+                                                        false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(y),
+                                                        false, false);
+        lo = __hiloint2double(h[0], l[0]);  // the lower halves of x, y
+        hi = __hiloint2double(h[1], l[1]);  // the upper halves
+    };
+    auto swap16 = [](double x, double y, double& even, double& odd) {
+        const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(x), __double2loint(y),
+                                                        false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(x), __double2hiint(y),
+                                                        false, false);
+        even = __hiloint2double(h[0], l[0]);
+        odd = __hiloint2double(h[1], l[1]);
+    };
+    const int lane = threadIdx.x % WAVE;
+    double p, q, ab, cd;
+    swap32(a, b, p, q);
+    ab = p + q;
+    swap32(c, d, p, q);
+    cd = p + q;
+    const double m = fmax(p, q);
+    cd = lane < 32 ? cd : m;
+    swap16(ab, cd, p, q);  // rows: a, c, b, d
+    const double s = p + q, t = fmax(p, q);
+    return rows_reduce(lane < 48 ? s : t);
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
 __device__ __forceinline__ int wave_max_i(int v) {
     v = max(v, lane_down<32>(v));
     v = max(v, lane_down<16>(v));

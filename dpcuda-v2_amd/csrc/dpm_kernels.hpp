@@ -156,6 +156,94 @@ __device__ __forceinline__ void mix_one(double2& v, double2 f, double alpha) {
     v.y = v.y * (1 - alpha) + f.y * mr;
 }
 
+__device__ __forceinline__ int cell_coord(double pos, double cs, int n) {
+    // getPBCCellIndex, include/particles/base/kernels.cuh:285-301
+    long long idx = (long long)floor(pos / cs);
+    return (int)(idx >= 0 ? idx % n : (idx % n + n) % n);
+}
+
+// Fire::step's decision for the next iteration (src/integrator/fire.cu:14-33);
+// RigidBumpy::getPowerFire adds sum(tau*w) (rigid_bumpy.cu:1181-1191; null for disks).  True
+// when the loop has ended.
+__device__ __forceinline__ bool fire_decide(FireCtl& F, double px, double py,
+                                            const double* spin) {
+    double power = px + py;
+    if (spin) power = power + *spin;
+    F.power = power;
+    if (power > 0) {
+        F.n_good++;
+        F.n_bad = 0;
+        if (F.n_good > 5) {
+            F.dt = fmin(F.dt * 1.1, F.dt_max);
+            F.alpha *= 0.99;
+        }
+        F.uphill = 0;
+    } else {
+        F.n_good = 0;
+        F.n_bad++;
+        if (F.n_bad > 10) {
+            F.stopped = 1;
+            F.step += 1;  // the stopped step counts as executed
+            F.done = 1;
+            return true;
+        }
+        F.dt = fmax(F.dt * 0.5, F.dt_min);
+        F.alpha = F.alpha_init;
+        F.uphill = 1;
+    }
+    return false;
+}
+
+// minimizeFire's prologue: records the first average energy
+__device__ __forceinline__ bool fire_begin(FireCtl& F, double px, double py, double pe,
+                                           double fm, const double* spin) {
+    F.fmax_sq = fm;
+    F.avg_pe = pe / F.dof;
+    F.last_avg_pe = F.avg_pe;
+    if (F.max_steps <= 0) {
+        F.done = 1;
+        return true;
+    }
+    return fire_decide(F, px, py, spin);
+}
+
+// The end of a step: minimizeFire's stop test (src/routines/minimization.cu:99-105), then the
+// decision for the next step.  One thread calls these.
+__device__ __forceinline__ bool fire_advance(FireCtl& F, double px, double py, double pe,
+                                             double fm, const double* spin) {
+    const double avg = pe / F.dof;
+    F.fmax_sq = fm;
+    F.avg_pe = avg;
+    const double diff = fabs(avg / F.last_avg_pe - 1);
+    F.last_avg_pe = avg;
+    const bool fok = F.fmax_target_sq > 0.0 && fm < F.fmax_target_sq;
+    F.step += 1;
+    if (diff < F.avg_pe_diff_target || avg < F.avg_pe_target || fok) {
+        F.converged = 1;
+        F.done = 1;
+        return true;
+    }
+    if (F.step >= F.max_steps) {
+        F.done = 1;
+        return true;
+    }
+    return fire_decide(F, px, py, spin);
+}
+
+// mix_one by the short square root and quotient sequences: the same bits, for squared norms in
+// the range that they cover; other lanes take the general form.
+__device__ __forceinline__ void mix_hot(double2& v, double2 f, double alpha) {
+    const double f2 = f.x * f.x + f.y * f.y, v2 = v.x * v.x + v.y * v.y;
+    if (f2 > 0x1p-100 && f2 < 0x1p500 && v2 > 0x1p-600 && v2 < 0x1p500) {  // (fn > 1e-16)
+        const double fn = sqrt_rn_normal(f2), vn = sqrt_rn_normal(v2);
+        const double mr = div_rn_normal(vn, fn) * alpha;
+        v.x = v.x * (1 - alpha) + f.x * mr;
+        v.y = v.y * (1 - alpha) + f.y * mr;
+    } else {
+        mix_one(v, f, alpha);
+    }
+}
+
 // ---- host helpers (dpm_core.hip) ----
 std::mutex& capture_mutex();
 int dalloc_bytes(dpm_system* s, void** p, size_t bytes);
@@ -197,6 +285,18 @@ struct Timed {
     Timed(dpm_system* s_, int cls_);
     ~Timed();
 };
+
+// ---- small disk systems (dpm_resident.hip) ----
+// Loops of up to RESIDENT_MAX_N particles run in one workgroup, from RESIDENT_MIN_STEPS steps.
+// Measured against the chunked loops, us a step of 1,000: NVE 1.5 and 4.5 at 128 particles, 3.3
+// and 5.9 at 1,000; FIRE 3.4 and 14 at 128, 6.9 and 19.5 at 1,000; NVE in runs of 16 steps 5.0
+// and 7.2 at 1,000.  One CU's vector pipe bounds it: two particles a thread (2,000) took 11 us
+// for an NVE step that the chunked loop does in 6.1.
+constexpr int64_t RESIDENT_MAX_N = 1024;
+constexpr int64_t RESIDENT_MIN_STEPS = 16;
+bool resident_ok(const dpm_system* s);
+void resident_nve(dpm_system* s, double dt, int64_t steps);
+void resident_fire(dpm_system* s, int64_t steps);
 
 // ---- rigid bumpy (dpm_bumpy.hip) ----
 int bumpy_alloc(dpm_system* s);
