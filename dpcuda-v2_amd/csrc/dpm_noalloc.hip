@@ -9,9 +9,10 @@
 // kernelUpdateNeighborList (src/particles/base/kernels.cu:256-293, all pairs within rc in
 // ascending j), then totalPotentialEnergy (src/particles/base/particle.cu:1078-1080) in the
 // library's canonical summation order.  The pairs come from a cell grid (cells at least rc
-// wide; each particle's nine cells merged in ascending index), so the pair order, and every
+// wide; each particle's hits are ranked by index), so the order of a particle's sum, and every
 // result bit, equal the list-based path.
 #include <mutex>
+#include <type_traits>
 
 #include "dpm_kernels.hpp"
 
@@ -21,9 +22,6 @@ namespace dpm {
 __global__ void k_scan_a(Dev d, long long nc, int gated);
 __global__ void k_scan_b(Dev d, long long nb_blocks, int gated);
 __global__ void k_scan_c(Dev d, long long nc, int gated);
-__global__ void k_cell_scatter(Dev d, int gated);
-__global__ void k_cell_sort(Dev d, long long nc, int gated);
-__global__ void k_final_sum(const double* part, int64_t nc, double* out);
 
 // ---- scratch layout -----------------------------------------------------------------------
 constexpr int64_t NA_MAX_N = 1 << 20;      // particles per call
@@ -37,10 +35,10 @@ constexpr size_t NA_OFF_START = NA_OFF_CNT + na_align(sizeof(int) * NA_MAX_CELLS
 constexpr size_t NA_OFF_CUR = NA_OFF_START + na_align(sizeof(int) * (NA_MAX_CELLS + 1));
 constexpr size_t NA_OFF_BSUM = NA_OFF_CUR + na_align(sizeof(int) * NA_MAX_CELLS);
 constexpr size_t NA_OFF_CELL = NA_OFF_BSUM + na_align(sizeof(int) * (NA_MAX_SB + 1));
-constexpr size_t NA_OFF_PERM = NA_OFF_CELL + na_align(sizeof(int) * NA_MAX_N);
-constexpr size_t NA_OFF_PART = NA_OFF_PERM + na_align(sizeof(int) * NA_MAX_N);
+constexpr size_t NA_OFF_REC = NA_OFF_CELL + na_align(sizeof(int) * NA_MAX_N);
+constexpr size_t NA_OFF_PART = NA_OFF_REC + na_align(sizeof(double4) * NA_MAX_N);
 constexpr size_t NA_SCRATCH_BYTES = NA_OFF_PART + na_align(sizeof(double) * (NA_MAX_N / 64 + 1));
-// 20.1 MiB per device
+// 48.1 MiB per device
 
 static __device__ __align__(256) unsigned char scratch[NA_SCRATCH_BYTES];
 
@@ -89,86 +87,306 @@ __device__ __forceinline__ int na_coord(double pos, double cs, int n) {
     return (int)(m < 0 ? m + n : m);
 }
 
-// cell of each particle + counting-sort histogram (non-finite positions go to cell 0)
+// (non-finite positions go to cell 0)
+__device__ __forceinline__ int na_cell(double x, double y, const NaGrid& g) {
+    if (!(isfinite(x) && isfinite(y) && fabs(x) < 1e15 * g.csx && fabs(y) < 1e15 * g.csy)) return 0;
+    return na_coord(x, g.csx, g.ncx) + g.ncx * na_coord(y, g.csy, g.ncy);
+}
+
+// cell of each particle + counting-sort histogram
 __global__ void k_na_bin(const double* x, const double* y, int64_t n, NaGrid g, int* cell,
                          int* cnt) {
     int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     if (i >= n) return;
-    int c = 0;
-    if (g.ncx > 1) {
-        double xi = x[i], yi = y[i];
-        if (isfinite(xi) && isfinite(yi) && fabs(xi) < 1e15 * g.csx && fabs(yi) < 1e15 * g.csy)
-            c = na_coord(xi, g.csx, g.ncx) + g.ncx * na_coord(yi, g.csy, g.ncy);
-    }
+    const int c = na_cell(x[i], y[i], g);
     cell[i] = c;
     atomicAdd(&cnt[c], 1);
 }
 
-// Forces, energies and the closing chunk partials of the canonical PE sum.  One thread per
-// particle; the candidates of the nine cells around i's (every particle, for a 1 x 1 grid,
-// which has no cell lists: perm == nullptr) are taken in ascending index, and a pair
-// counts when its minimum-image separation is within the cutoff (isWithinCutoffSquared,
-// kernels.cuh:249-260), exactly as the listed pairs of the Verlet rows.
-__global__ __launch_bounds__(BLOCK) void k_na_forces(const double* x, const double* y,
-                                                     const double* rad, int64_t n, NaGrid g,
-                                                     PairParams p, double rc2, const int* cell,
-                                                     const int* start, const int* perm,
-                                                     double* fx, double* fy, double* pe,
-                                                     double* part) {
+// The particles in cell order (in no order within a cell): one record each, {x, y, radius, index}
+__global__ void k_na_scatter(const double* x, const double* y, const double* rad, int64_t n,
+                             const int* cell, int* cur, double4* rec) {
     const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= n) return;
+    const double4 q = make_double4(x[i], y[i], rad[i], (double)i);
+    rec[atomicAdd(&cur[cell[i]], 1)] = q;
+}
+
+// Up to NA_LDS_N particles every workgroup forms the whole cell grid in its own LDS, and the call
+// is two launches; beyond, the particles are sorted into records by cell over six launches, so
+// that candidates are neighbours in memory.  Measured, us a call (in LDS, sorted): 26, 31 at
+// 8,192 particles; 42, 34 at 16,400.
+constexpr int NA_LDS_N = 8192;
+constexpr int NA_LDS_CELLS = 8192;
+
+constexpr int NA_T = 1024;            // threads: 16 lanes for each of a chunk's particles
+constexpr int NA_GROUP = NA_T / CHUNK;
+constexpr int NA_HITS = 32;           // pairs of a particle that LDS holds
+
+struct NaForces {
+    double2 f[CHUNK][NA_HITS];  // pair forces and energies in the order of the particle's sum
+    double e[CHUNK][NA_HITS];
+    int hit[CHUNK][NA_HITS];    // partners as they are found, by place
+    int key[CHUNK][NA_HITS];    // and their indices
+    double pe[CHUNK];
+    int wsum[NA_T / WAVE];
+};
+
+struct NaGridLds {
+    int cend[NA_LDS_CELLS];         // end of each cell's list
+    unsigned short lst[NA_LDS_N];   // the lists, in no order within a cell
+};
+
+struct NaNone {};
+
+// The counting sort of all particles into the grid's cells, by one workgroup.
+__device__ __forceinline__ void na_lds_grid(NaGridLds& G, NaForces& L, const double* x,
+                                            const double* y, int n, const NaGrid& g) {
+    const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE, ncell = g.ncx * g.ncy;
+    for (int c = tid; c < ncell; c += NA_T) G.cend[c] = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += NA_T) atomicAdd(&G.cend[na_cell(x[i], y[i], g)], 1);
+    __syncthreads();
+    // exclusive scan of the counts: each thread owns a run of consecutive cells
+    const int per = (ncell + NA_T - 1) / NA_T;
+    const int c0 = min(tid * per, ncell), c1 = min(c0 + per, ncell);
+    int local = 0;
+    for (int c = c0; c < c1; ++c) local += G.cend[c];
+    int incl = local;
+#pragma unroll
+    for (int s = 1; s < WAVE; s <<= 1) {
+        const int o = __shfl_up(incl, s, WAVE);
+        if (lane >= s) incl += o;
+    }
+    if (lane == WAVE - 1) L.wsum[wv] = incl;
+    __syncthreads();
+    int run = incl - local;
+    for (int k = 0; k < wv; ++k) run += L.wsum[k];
+    for (int c = c0; c < c1; ++c) {
+        const int t = G.cend[c];
+        G.cend[c] = run;
+        run += t;
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += NA_T)
+        G.lst[atomicAdd(&G.cend[na_cell(x[i], y[i], g)], 1)] = (unsigned short)i;
+    __syncthreads();
+}
+
+// LDS writes of the wave's lanes before its lanes' later reads
+__device__ __forceinline__ void na_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The total of nc partials in wave_final_sum's order (lane t adds partials t, t + 64, ...): all
+// threads bring a stretch of them to LDS, one wave adds it.
+constexpr int NA_STRETCH = 4096;
+
+__global__ __launch_bounds__(NA_T) void k_na_total(const double* part, int64_t nc,
+                                                   double* total) {
+    __shared__ double stretch[NA_STRETCH];
+    const int tid = threadIdx.x;
+    double s = 0.0;
+    for (int64_t base = 0; base < nc; base += NA_STRETCH) {
+        const int len = (int)min((int64_t)NA_STRETCH, nc - base);
+        __syncthreads();
+        for (int k = tid; k < len; k += NA_T) stretch[k] = part[base + k];
+        __syncthreads();
+        if (tid < WAVE)
+            for (int k = tid; k < len; k += WAVE) s = s + stretch[k];
+    }
+    if (tid >= WAVE) return;
+    s = wave_tree_sum(s);
+    if (tid == 0) *total = s;
+}
+
+// Forces and energies: a workgroup per 64 particles, 16 lanes a particle.  The lanes test the
+// candidates of the nine cells side by side, append the hits, rank them by index and evaluate
+// one pair each; three lanes then add the components in rank order (the ascending order of the
+// Verlet rows).  A serial walk that merged the nine lists in order spent some 60 instructions
+// and a dependent load on each of 27 candidates.
+// LDS: the grid is the workgroup's own, the particles are the caller's arrays in their order, and
+// the workgroup is a chunk of the energy sum.  Otherwise `rec` holds the particles in cell order
+// and `start` the cells' first records: reading the caller's arrays at random costs a cache line
+// for each coordinate of each candidate (1,010 us at 1,048,576 particles).
+// What bounds it: at a thousand particles the host's launches, at a million the records' scatter
+// and the candidates.  Measured, us a call (before, now): 1,500 particles 70, 13; 16,400 75, 34;
+// 1,048,576 1,013, 537.
+template <bool LDS>
+__global__ __launch_bounds__(NA_T) void k_na_forces(const double* x, const double* y,
+                                                    const double* rad, int64_t n, NaGrid g,
+                                                    PairParams p, double rc2, const int* start,
+                                                    const double4* rec, double* fx, double* fy,
+                                                    double* pe, double* part) {
+    __shared__ NaForces L;
+    __shared__ typename std::conditional<LDS, NaGridLds, NaNone>::type G;
+    const int tid = threadIdx.x, lane = tid % WAVE, sub = lane % NA_GROUP, k = tid / NA_GROUP;
+    if constexpr (LDS) na_lds_grid(G, L, x, y, (int)n, g);
+    // a particle's place: its index, or its record's
+    const int tile = LDS ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
+    const int64_t me = (int64_t)tile * CHUNK + k;
+    const bool live = me < n;
+    auto load = [&](int64_t u) {
+        if constexpr (LDS) return make_double4(x[u], y[u], rad[u], 0.0);
+        else return rec[u];
+    };
+    auto key_of = [&](int u, const double4& q) {
+        if constexpr (LDS) return u;
+        else return (int)q.w;
+    };
+    const double4 q = load(live ? me : 0);
+    // the runs of list entries in the three rows of cells: one each, two where a row wraps
+    auto range = [&](int c0, int c1, int& a, int& b) {
+        if constexpr (LDS) {
+            a = c0 == 0 ? 0 : G.cend[c0 - 1];
+            b = G.cend[c1];
+        } else {
+            a = start[c0];
+            b = start[c1 + 1];
+        }
+    };
+    int a[6], m[6];
+    {
+        const int cid = na_cell(q.x, q.y, g);
+        const int cx = cid % g.ncx, cy = cid / g.ncx;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const int yy = cy + r - 1 < 0 ? g.ncy - 1 : (cy + r - 1 >= g.ncy ? 0 : cy + r - 1);
+            const int c = yy * g.ncx;
+            int e;
+            range(c + max(cx - 1, 0), c + min(cx + 1, g.ncx - 1), a[2 * r], e);
+            m[2 * r] = live ? e - a[2 * r] : 0;
+            a[2 * r + 1] = 0;
+            m[2 * r + 1] = 0;
+            if (cx == 0 || cx == g.ncx - 1) {
+                const int w = c + (cx == 0 ? g.ncx - 1 : 0);
+                range(w, w, a[2 * r + 1], e);
+                m[2 * r + 1] = live ? e - a[2 * r + 1] : 0;
+            }
+        }
+    }
+    const int cand = m[0] + m[1] + m[2] + m[3] + m[4] + m[5];
+    auto candidate = [&](int t) {  // the place of candidate t
+        int u = a[0] + t, base = m[0];
+#pragma unroll
+        for (int r = 1; r < 6; ++r) {
+            if (t >= base) u = a[r] + (t - base);
+            base += m[r];
+        }
+        if constexpr (LDS) return (int)G.lst[u];
+        else return u;
+    };
+    auto listed = [&](const double4& o) {
+        const double dx = pbc(q.x, o.x, p.Lx, p.invLx, p.halfLx, 1);
+        const double dy = pbc(q.y, o.y, p.Ly, p.invLy, p.halfLy, 1);
+        return dx * dx + dy * dy < rc2;
+    };
+    const int shift = lane - sub;
+    int cnt = 0;
+    for (int t = sub; __builtin_amdgcn_ballot_w64(t < cand) != 0; t += NA_GROUP) {
+        int u = -1, key = 0;
+        bool hit = false;
+        if (t < cand) {
+            u = candidate(t);
+            const double4 o = load(u);
+            key = key_of(u, o);
+            hit = u != (int)me && listed(o);
+        }
+        const unsigned mask =
+            (unsigned)(__builtin_amdgcn_ballot_w64(hit) >> shift) & ((1u << NA_GROUP) - 1);
+        const int pos = cnt + __popc(mask & ((1u << sub) - 1));
+        if (hit && pos < NA_HITS) {
+            L.hit[k][pos] = u;
+            L.key[k][pos] = key;
+        }
+        cnt += __popc(mask);
+    }
+    na_wave_sync();
+    auto pair = [&](int u, double& px, double& py) {
+        const double4 o = load(u);
+        const double rs = q.z + o.z;
+        PairParams w = p;  // the short sequences, where they give the same bits
+        w.fastdiv = p.fastdiv && rs >= 0x1p-99 && rs <= 0x1p99;
+        return pair_law(q.x, q.y, q.z, o.x, o.y, o.z, w, px, py);
+    };
+    double acc = 0.0;
+    if (cnt <= NA_HITS) {
+        for (int h = sub; h < cnt; h += NA_GROUP) {
+            const int key = L.key[k][h];
+            int rank = 0;
+            for (int v = 0; v < cnt; ++v) rank += L.key[k][v] < key ? 1 : 0;
+            double px, py;
+            const double e = pair(L.hit[k][h], px, py);
+            L.f[k][rank] = make_double2(px, py);
+            L.e[k][rank] = e;
+        }
+        na_wave_sync();
+        if (sub < 3) {
+            for (int v = 0; v < cnt; ++v)
+                acc += sub == 0 ? L.f[k][v].x : (sub == 1 ? L.f[k][v].y : L.e[k][v]);
+        }
+    } else if (sub < 3) {  // more hits than LDS holds: found again in ascending order
+        for (int v = 0, lo = -1; v < cnt; ++v) {
+            int next = INT_MAX, at = 0;
+            for (int t = 0; t < cand; ++t) {
+                const int u = candidate(t);
+                const double4 o = load(u);
+                const int key = key_of(u, o);
+                if (key > lo && key < next && u != (int)me && listed(o)) {
+                    next = key;
+                    at = u;
+                }
+            }
+            lo = next;
+            double px, py;
+            const double e = pair(at, px, py);
+            acc += sub == 0 ? px : (sub == 1 ? py : e);
+        }
+    }
+    acc = 0.0 + acc;
+    const int i = key_of((int)me, q);
+    if (live) {
+        if (sub == 0) fx[i] = acc;
+        if (sub == 1) fy[i] = acc;
+        if (sub == 2) pe[i] = acc;
+    }
+    if constexpr (LDS) {  // the chunk's partial of the energy sum (k_chunk_sum's tree)
+        if (sub == 2) L.pe[k] = live ? acc : 0.0;
+        __syncthreads();
+        if (tid >= WAVE) return;
+        const double v = wave_tree_sum(L.pe[tid]);
+        if (tid == 0) part[blockIdx.x] = v;
+    }
+}
+
+// The chunk partials of the energy sum
+__global__ __launch_bounds__(BLOCK) void k_na_chunks(const double* pe, int64_t n, double* part) {
+    const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    const double v = wave_tree_sum(i < n ? pe[i] : 0.0);
+    if (threadIdx.x % WAVE == 0 && i < n) part[i / CHUNK] = v;
+}
+
+// The same for a box under three cutoffs a side: every particle is a candidate, in ascending
+// order; a thread per particle, a chunk per workgroup.
+__global__ __launch_bounds__(CHUNK) void k_na_forces_all(const double* x, const double* y,
+                                                         const double* rad, int64_t n,
+                                                         PairParams p, double rc2, double* fx,
+                                                         double* fy, double* pe, double* part) {
+    const int64_t i = (int64_t)blockIdx.x * CHUNK + threadIdx.x;
     double e = 0.0;
     if (i < n) {
         const double xi = x[i], yi = y[i], ri = rad[i];
-        int s[9], en[9], h[9];
-        const int nl = g.ncx > 1 ? 9 : 1;
-        if (nl == 9) {
-            const int cid = cell[i];
-            const int cx = cid % g.ncx, cy = cid / g.ncx;
-#pragma unroll
-            for (int oy = -1; oy <= 1; ++oy) {
-                const int yy = cy + oy < 0 ? cy + oy + g.ncy : (cy + oy >= g.ncy ? cy + oy - g.ncy : cy + oy);
-#pragma unroll
-                for (int ox = -1; ox <= 1; ++ox) {
-                    const int xx = cx + ox < 0 ? cx + ox + g.ncx : (cx + ox >= g.ncx ? cx + ox - g.ncx : cx + ox);
-                    const int c = xx + yy * g.ncx;
-                    const int t = (oy + 1) * 3 + (ox + 1);
-                    s[t] = start[c];
-                    en[t] = start[c + 1];
-                }
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < 9; ++t) s[t] = en[t] = 0;
-            en[0] = (int)n;
-        }
-        auto at = [perm](int k) { return perm ? perm[k] : k; };
-#pragma unroll
-        for (int t = 0; t < 9; ++t) h[t] = s[t] < en[t] ? at(s[t]) : INT_MAX;
         double ax = 0.0, ay = 0.0;
-        for (;;) {
-            int best = INT_MAX, bt = -1;
-#pragma unroll
-            for (int t = 0; t < 9; ++t)
-                if (h[t] < best) {
-                    best = h[t];
-                    bt = t;
-                }
-            if (bt < 0) break;
-#pragma unroll
-            for (int t = 0; t < 9; ++t)
-                if (t == bt) {
-                    s[t]++;
-                    h[t] = s[t] < en[t] ? at(s[t]) : INT_MAX;
-                }
-            if (best == i) continue;
-            const double xj = x[best], yj = y[best];
-            const double dx = pbc(xi, xj, p.Lx, p.invLx, p.halfLx, 0);
-            const double dy = pbc(yi, yj, p.Ly, p.invLy, p.halfLy, 0);
+        for (int64_t j = 0; j < n; ++j) {
+            if (j == i) continue;
+            const double dx = pbc(xi, x[j], p.Lx, p.invLx, p.halfLx, 0);
+            const double dy = pbc(yi, y[j], p.Ly, p.invLy, p.halfLy, 0);
             if (dx * dx + dy * dy < rc2) {
-                double fpx, fpy;
-                const double ie = pair_law(xi, yi, ri, xj, yj, rad[best], p, fpx, fpy);
-                ax += fpx;
-                ay += fpy;
+                double px, py;
+                const double ie = pair_law(xi, yi, ri, x[j], y[j], rad[j], p, px, py);
+                ax += px;
+                ay += py;
                 e += ie;
             }
         }
@@ -177,10 +395,8 @@ __global__ __launch_bounds__(BLOCK) void k_na_forces(const double* x, const doub
         e = 0.0 + e;
         pe[i] = e;
     }
-    // chunk partial of the canonical sum (k_chunk_sum's tree over 64 consecutive particles)
-    const double v = wave_tree_sum(i < n ? e : 0.0);
-    const int64_t c = i / CHUNK;
-    if ((threadIdx.x % WAVE) == 0 && c * CHUNK < n) part[c] = v;
+    const double v = wave_tree_sum(e);
+    if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
 }  // namespace dpm
@@ -208,11 +424,20 @@ int dpm_disk_forces_noalloc(const double* x, const double* y, const double* radi
     unsigned char* base = nullptr;
     if (scratch_of_current_device(&base)) return -1;
     hipStream_t st = (hipStream_t)stream;
-    // the grid: cells at least cutoff (1 + 1e-9) wide, at most NA_MAX_CELLS and about two
-    // per particle; under three a side, one cell holds every particle
+    const bool lds = n <= NA_LDS_N;
+    // the grid: cells at least cutoff (1 + 1e-9) wide, at most about two per particle and
+    // what the cell arrays hold; under three a side, one cell holds every particle
     const double cw = cutoff * (1.0 + 1e-9);
     double fx_c = std::floor(lx / cw), fy_c = std::floor(ly / cw);
-    const double cap = std::min<double>((double)NA_MAX_CELLS, std::max(9.0, 2.0 * (double)n));
+    const double cap = std::min<double>(lds ? (double)NA_LDS_CELLS : (double)NA_MAX_CELLS,
+                                        std::max(9.0, 2.0 * (double)n));
+    if (fx_c * fy_c > cap) {  // shrunk in proportion, then to the limit
+        const double f = std::sqrt(fx_c * fy_c / cap);
+        if (std::min(fx_c, fy_c) > 3.0 * f) {
+            fx_c = std::floor(fx_c / f) + 1.0;
+            fy_c = std::floor(fy_c / f) + 1.0;
+        }
+    }
     while (fx_c * fy_c > cap) {
         if (fx_c >= fy_c) fx_c -= 1.0;
         else fy_c -= 1.0;
@@ -233,7 +458,7 @@ int dpm_disk_forces_noalloc(const double* x, const double* y, const double* radi
     d.cell_cur = (int*)(base + NA_OFF_CUR);
     d.scan_bsum = (int*)(base + NA_OFF_BSUM);
     d.cell_tmp = (int*)(base + NA_OFF_CELL);
-    d.perm = (int*)(base + NA_OFF_PERM);
+    double4* rec = (double4*)(base + NA_OFF_REC);
     double* part = (double*)(base + NA_OFF_PART);
     // the pair law's parameters (pair_params without a system)
     PairParams p{};
@@ -250,24 +475,34 @@ int dpm_disk_forces_noalloc(const double* x, const double* y, const double* radi
     int ex;
     p.inv2nc = (std::frexp(p.two_nc, &ex) == 0.5) ? 1.0 / p.two_nc : 0.0;
     p.fast = 0;
-    p.fastdiv = 0;
+    p.fastdiv = n_c == 2.0 && e_c >= 0x1p-100 && e_c <= 0x1p100;  // (radii: the kernels)
     const int64_t nsb = (nc + NA_SCAN_TILE - 1) / NA_SCAN_TILE;
-    const bool grid = g.ncx > 1;
-    if (grid) {  // counting sort into the cells (cells cleared by a kernel: no memset node,
-                 // so a captured graph replays correctly)
+    const double rc2 = cutoff * cutoff;
+    const dim3 chunks((unsigned)((n + CHUNK - 1) / CHUNK)), threads(NA_T);
+    if (g.ncx == 1) {
+        p.fastdiv = 0;
+        hipLaunchKernelGGL(k_na_forces_all, chunks, dim3(CHUNK), 0, st, x, y, radius, n, p, rc2,
+                           fx, fy, pe, part);
+    } else if (lds) {
+        p.fast = 1;  // half a side exceeds the cutoff, and only pairs within it count
+        hipLaunchKernelGGL(k_na_forces<true>, chunks, threads, 0, st, x, y, radius, n, g, p, rc2,
+                           nullptr, nullptr, fx, fy, pe, part);
+    } else {  // counting sort into the cells (cells cleared by a kernel: no memset node, so a
+              // captured graph replays correctly)
+        p.fast = 1;
         hipLaunchKernelGGL(k_na_fill, pgrid(nc), dim3(BLOCK), 0, st, d.cell_cnt, nc);
         hipLaunchKernelGGL(k_na_bin, pgrid(n), dim3(BLOCK), 0, st, x, y, n, g, d.cell_tmp,
                            d.cell_cnt);
         hipLaunchKernelGGL(k_scan_a, dim3((unsigned)nsb), dim3(BLOCK), 0, st, d, (long long)nc, 0);
         hipLaunchKernelGGL(k_scan_b, dim3(1), dim3(1024), 0, st, d, (long long)nsb, 0);
         hipLaunchKernelGGL(k_scan_c, dim3((unsigned)nsb), dim3(BLOCK), 0, st, d, (long long)nc, 0);
-        hipLaunchKernelGGL(k_cell_scatter, pgrid(n), dim3(BLOCK), 0, st, d, 0);
-        hipLaunchKernelGGL(k_cell_sort, pgrid(nc), dim3(BLOCK), 0, st, d, (long long)nc, 0);
+        hipLaunchKernelGGL(k_na_scatter, pgrid(n), dim3(BLOCK), 0, st, x, y, radius, n,
+                           d.cell_tmp, d.cell_cur, rec);
+        hipLaunchKernelGGL(k_na_forces<false>, chunks, threads, 0, st, x, y, radius, n, g, p, rc2,
+                           d.cell_start, rec, fx, fy, pe, part);
+        hipLaunchKernelGGL(k_na_chunks, pgrid(n), dim3(BLOCK), 0, st, pe, n, part);
     }
-    hipLaunchKernelGGL(k_na_forces, pgrid(n), dim3(BLOCK), 0, st, x, y, radius, n, g, p,
-                       cutoff * cutoff, d.cell_tmp, d.cell_start, grid ? d.perm : nullptr, fx,
-                       fy, pe, part);
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(WAVE), 0, st, part, (n + CHUNK - 1) / CHUNK,
+    hipLaunchKernelGGL(k_na_total, dim3(1), threads, 0, st, part, (n + CHUNK - 1) / CHUNK,
                        pe_total);
     return check_launch();
 }

@@ -357,7 +357,7 @@ int dpm_server_release(dpm_server* s, int64_t id);
  * disk system with the Verlet method and this cutoff returns from dpm_neighbor_init +
  * dpm_zero_forces + dpm_compute_forces + dpm_reduce(DPM_RED_PE), bit for bit.  Kernels are
  * enqueued on `stream` (a hipStream_t; null for the null stream) and the call returns
- * without waiting.  The working memory is a 20 MiB array of the library, resident on each
+ * without waiting.  The working memory is a 48 MiB array of the library, resident on each
  * device it runs on until the process ends; the call allocates nothing.  Limits: n <=
  * 1,048,576; a box under three cutoffs a side takes n <= 4,096.  Calls on one device share
  * that array: calls that overlap in time on one device (other streams, other threads)
