@@ -37,42 +37,86 @@ void set_error(const std::string& m) { g_err = m; }
 
 __device__ __forceinline__ int wrap_cell(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
 
-// The list row of particle i (kernelUpdateCellNeighborList, base/kernels.cu:440-505):
-// 3x3 stencil, dy outer, dx inner, ascending sorted index within a cell, written to
-// the column-major ELL.  `pos(j)` supplies the positions the list is built from.
-template <class Pos>
-__device__ __forceinline__ int stencil_build(const Dev& d, const NbrParams& nb, int64_t i,
-                                             double2 xi, Pos pos) {
+// The particles of the 3 x 3 cells around particle i's in the reference's order (dy outer, dx
+// inner, ascending sorted index within a cell).  Particles are in cell order, so the cells of a
+// row of the stencil are one run of indices, except where the row wraps.
+template <class Visit>
+__device__ __forceinline__ void stencil_runs(const Dev& d, const NbrParams& nb, int64_t i,
+                                             Visit visit) {
     const int ncd = nb.ncd;
-    int cid = d.cell_of[i];
-    int cx = cid % ncd, cy = cid / ncd;
-    int s[9], e[9];
+    const int cid = d.cell_of[i];
+    const int cx = cid % ncd, cy = cid / ncd;
+    int a[9], b[9];  // per row: the run before a wrap, the row's, the run after one
+    const bool runs = ncd >= 3;
 #pragma unroll
-    for (int oy = -1; oy <= 1; ++oy) {
-        int yy = wrap_cell(cy + oy, ncd);
+    for (int r = 0; r < 3; ++r) {
+        const int c = wrap_cell(cy + r - 1, ncd) * ncd;
+        const int* s = d.cell_start + c;
+        if (runs) {
+            a[3 * r] = a[3 * r + 2] = b[3 * r] = b[3 * r + 2] = 0;
+            a[3 * r + 1] = s[max(cx - 1, 0)];
+            b[3 * r + 1] = s[min(cx + 1, ncd - 1) + 1];
+            if (cx == 0) {
+                a[3 * r] = s[ncd - 1];
+                b[3 * r] = s[ncd];
+            }
+            if (cx == ncd - 1) {
+                a[3 * r + 2] = s[0];
+                b[3 * r + 2] = s[1];
+            }
+        } else {  // cells repeat
 #pragma unroll
-        for (int ox = -1; ox <= 1; ++ox) {
-            int c = wrap_cell(cx + ox, ncd) + yy * ncd;
-            int t = (oy + 1) * 3 + (ox + 1);
-            s[t] = d.cell_start[c];
-            e[t] = d.cell_start[c + 1];
-        }
-    }
-    int cnt = 0;
-    const int cap = d.cap;
-#pragma unroll
-    for (int t = 0; t < 9; ++t) {
-        for (int j = s[t]; j < e[t]; ++j) {
-            if (j == i) continue;
-            double2 xj = pos(j);
-            double dx = pbc(xi.x, xj.x, nb.Lx, nb.invLx, nb.halfLx, nb.fast);
-            double dy = pbc(xi.y, xj.y, nb.Ly, nb.invLy, nb.halfLy, nb.fast);
-            if (dx * dx + dy * dy < nb.rc2) {  // isWithinCutoffSquared, kernels.cuh:249-260
-                if (cnt < cap) d.nbr[(int64_t)cnt * d.N + i] = j;
-                cnt++;
+            for (int t = 0; t < 3; ++t) {
+                const int x = wrap_cell(cx + t - 1, ncd);
+                a[3 * r + t] = s[x];
+                b[3 * r + t] = s[x + 1];
             }
         }
     }
+#pragma unroll
+    for (int t = 0; t < 9; ++t) visit(a[t], b[t]);
+}
+
+template <class Visit>
+__device__ __forceinline__ void stencil_visit(const Dev& d, const NbrParams& nb, int64_t i,
+                                              Visit visit) {
+    stencil_runs(d, nb, i, [&](int a, int b) {
+        for (int j = a; j < b; ++j)
+            if (j != i) visit(j);
+    });
+}
+
+// isWithinCutoffSquared, include/particles/base/kernels.cuh:249-260
+__device__ __forceinline__ bool within(double ax, double ay, double bx, double by,
+                                       const NbrParams& nb, double c2) {
+    double dx = pbc(ax, bx, nb.Lx, nb.invLx, nb.halfLx, nb.fast);
+    double dy = pbc(ay, by, nb.Ly, nb.invLy, nb.halfLy, nb.fast);
+    return dx * dx + dy * dy < c2;
+}
+
+// The list row of particle i (kernelUpdateCellNeighborList, base/kernels.cu:440-505), written to
+// the column-major ELL.  `pos(j)` supplies the positions the list is built from; the positions
+// of BATCH candidates are loaded together.
+template <int BATCH = 1, class Pos>
+__device__ __forceinline__ int stencil_build(const Dev& d, const NbrParams& nb, int64_t i,
+                                             double2 xi, Pos pos) {
+    int cnt = 0;
+    const int cap = d.cap;
+    stencil_runs(d, nb, i, [&](int a, int b) {
+        for (int j = a; j < b; j += BATCH) {
+            double2 xj[BATCH];
+#pragma unroll
+            for (int t = 0; t < BATCH; ++t) xj[t] = pos(min(j + t, b - 1));
+#pragma unroll
+            for (int t = 0; t < BATCH; ++t) {
+                if (j + t >= b || j + t == i) continue;
+                if (within(xi.x, xi.y, xj[t].x, xj[t].y, nb, nb.rc2)) {
+                    if (cnt < cap) d.nbr[(int64_t)cnt * d.N + i] = j + t;
+                    cnt++;
+                }
+            }
+        }
+    });
     d.nnum[i] = cnt;
     return cnt;
 }
@@ -130,7 +174,7 @@ __device__ __forceinline__ void row_forces(const Dev& d, const double4* P, const
     }
 }
 
-// row_forces for the fused NVE step, with the first ROW_PF index columns loaded by
+// row_forces for the loops' steps, with the first ROW_PF index columns loaded by
 // the caller ahead of everything that waits on the control block, batches of ROW_PF
 // records gathered together, and the wave's slot bound taken from ballots instead of
 // a shuffle reduction.  Same slots, same order, same arithmetic as row_forces.
@@ -140,15 +184,16 @@ __device__ __forceinline__ bool wave_any(bool x) {
     return __builtin_amdgcn_ballot_w64(x) != 0;
 }
 
-template <bool HOT>
+template <bool ENERGY, bool HOT>
 __device__ __forceinline__ void row_forces_pf(const Dev& d, const double4* P, const PairParams& p,
                                               int64_t il, double4 qi, int nn, int (&jn)[ROW_PF],
-                                              double& ax, double& ay) {
+                                              double& ax, double& ay, double& e) {
     const int cap = d.cap;
     const int* col = d.nbr + il;
     const int64_t N = d.N;
     ax = 0.0;
     ay = 0.0;
+    e = 0.0;
     for (int k = 0; wave_any(k < nn); k += ROW_PF) {
         double4 q[ROW_PF];
 #pragma unroll
@@ -161,14 +206,15 @@ __device__ __forceinline__ void row_forces_pf(const Dev& d, const double4* P, co
         for (int t = 0; t < ROW_PF; ++t) {
             if (wave_any(k + t < nn)) {
                 const bool valid = k + t < nn;
-                double fx = 0.0, fy = 0.0;
+                double fx = 0.0, fy = 0.0, ie = 0.0;
                 if (HOT) {
-                    pair_hot<false>(qi, q[t], valid, p, fx, fy);
+                    ie = pair_hot<ENERGY>(qi, q[t], valid, p, fx, fy);
                 } else if (valid) {
-                    pair_law(qi.x, qi.y, qi.z, q[t].x, q[t].y, q[t].z, p, fx, fy);
+                    ie = pair_law(qi.x, qi.y, qi.z, q[t].x, q[t].y, q[t].z, p, fx, fy);
                 }
                 ax += fx;
                 ay += fy;
+                if (ENERGY) e += ie;
             }
         }
     }
@@ -242,8 +288,8 @@ __global__ __launch_bounds__(BLOCK) void k_nve_fused(Dev d, PairParams p, NbrPar
         }
     }
     const int nn = live ? min(nraw, d.cap) : 0;
-    double ax, ay;
-    row_forces_pf<HOT>(d, Pc, p, il, qi, nn, jn, ax, ay);
+    double ax, ay, e0;
+    row_forces_pf<false, HOT>(d, Pc, p, il, qi, nn, jn, ax, ay, e0);
     double nd = 0.0, cd = 0.0;
     if (live) {
         double fx = 0.0 + ax, fy = 0.0 + ay;
@@ -866,14 +912,6 @@ __global__ __launch_bounds__(BLOCK) void k_reorder_copyback(Dev d, Spare sp, int
     }
 }
 
-__device__ __forceinline__ bool within(double ax, double ay, double bx, double by,
-                                       const NbrParams& nb, double c2) {
-    // isWithinCutoffSquared, include/particles/base/kernels.cuh:249-260
-    double dx = pbc(ax, bx, nb.Lx, nb.invLx, nb.halfLx, nb.fast);
-    double dy = pbc(ay, by, nb.Ly, nb.invLy, nb.halfLy, nb.fast);
-    return dx * dx + dy * dy < c2;
-}
-
 // kernelUpdateCellNeighborList, base/kernels.cu:440-505: 3x3 stencil in the
 // reference's order (dy outer, dx inner, ascending sorted index), written to the
 // column-major ELL.  The nine cell ranges are loaded up front.
@@ -889,11 +927,11 @@ __global__ __launch_bounds__(BLOCK) void k_build_cell(Dev d, NbrParams nb, int g
     int cnt = 0;
     if (i < d.N) {
         if (from_ref) {
-            cnt = stencil_build(d, nb, i, d.lref[i], [&](int j) { return d.lref[j]; });
+            cnt = stencil_build<4>(d, nb, i, d.lref[i], [&](int j) { return d.lref[j]; });
         } else {
             double4 q = d.P0[i];
             double2 xi = make_double2(q.x, q.y);
-            cnt = stencil_build(d, nb, i, xi, [&](int j) {
+            cnt = stencil_build<4>(d, nb, i, xi, [&](int j) {
                 double4 qj = d.P0[j];
                 return make_double2(qj.x, qj.y);
             });
@@ -1150,20 +1188,24 @@ __global__ void k_ctl_reset(Dev d, int config) {
 //   k_fire_force  : zero + forces + kick(dt/2) + chunk partials of P, PE, |F|max
 //   k_fire_ctl    : canonical sums, minimizeFire's stop test for this step and
 //                   Fire::step's decision for the next (one wave)
+// (Every load goes out before the control block is looked at, as in k_nve_fused.)
 __global__ __launch_bounds__(BLOCK) void k_fire_move(Dev d, NbrParams nb, int pos) {
     Ctl* c = d.ctl;
-    if (c->halt) return;
     const FireCtl* F = d.fire;
-    if (F->done) return;
-    long long e = c->epoch;
-    double dt = F->dt, alpha = F->alpha;
-    int uphill = F->uphill;
+    const int halted = c->halt, done = F->done, uphill = F->uphill;
+    const long long e = c->epoch;
+    const double dt = F->dt, alpha = F->alpha;
     int tile;
-    int64_t i = particle_of_thread(tile);
+    const int64_t i = particle_of_thread(tile);
+    const bool live = i < d.N;
+    const int64_t il = live ? i : 0;
+    double4 q = d.P0[il];
+    double2 v = d.vel[il];
+    const double2 f = d.frc[il], ln = d.lref[il], lc = d.cref[il];
+    __asm__ __volatile__("" ::: "memory");
+    if (halted || done) return;
     double nd = 0.0, cd = 0.0;
-    if (i < d.N) {
-        double4 q = d.P0[i];
-        double2 v = d.vel[i], f = d.frc[i];
+    if (live) {
         if (uphill) {  // updatePositions(-dt/2) with the decreased dt; setVelocitiesToZero
             double bdt = -dt / 2.0;
             q.x += v.x * bdt;
@@ -1174,27 +1216,50 @@ __global__ __launch_bounds__(BLOCK) void k_fire_move(Dev d, NbrParams nb, int po
         double dtm = (dt / 2.0) / q.w;
         v.x += f.x * dtm;
         v.y += f.y * dtm;
-        mix_one(v, f, alpha);
+        mix_hot(v, f, alpha);
         q.x += v.x * dt;
         q.y += v.y * dt;
         d.P0[i] = q;
         d.vel[i] = v;
-        disp_of(d, i, q.x, q.y, nd, cd);
+        const double dxn = q.x - ln.x, dyn = q.y - ln.y, dxc = q.x - lc.x, dyc = q.y - lc.y;
+        nd = dxn * dxn + dyn * dyn;
+        cd = dxc * dxc + dyc * dyc;
     }
-    (void)tile;
     disp_flags(d, nb, nd, cd, pos & 1, stamp(e, pos));  // maxima: k_disp_partials at the end
 }
 
-// kick: 0 = forces only (minimizeFire's initial evaluation), 1 = + closing kick
+// kick: 0 = forces only (minimizeFire's initial evaluation), 1 = + closing kick.  A list rebuild
+// that a cell list needs is done here, before the particle's forces (rows are independent and
+// the positions rest): halting for it cost a chain of gated launches and the chunk's remaining
+// steps, 57 times in 500 steps of 65,537 disks.
 template <bool HOT>
-__global__ __launch_bounds__(BLOCK) void k_fire_force(Dev d, PairParams p, int pos, int kick,
-                                                      int gate) {
+__global__ __launch_bounds__(BLOCK) void k_fire_force(Dev d, PairParams p, NbrParams nb, int pos,
+                                                      int kick, int gate) {
     Ctl* c = d.ctl;
     const FireCtl* F = d.fire;
+    // the control words and every load that does not depend on them, all at once
+    const int halted = c->halt, done = F->done;
+    const long long epoch = c->epoch;
+    const double half = F->dt / 2.0;
+    int tile;
+    const int64_t i = particle_of_thread(tile);
+    const bool live = i < d.N;
+    const int64_t il = live ? i : 0;
+    const double4 qi = d.P0[il];
+    int cnt = d.nnum[il];
+    double2 v = d.vel[il];
+    int jn[ROW_PF];
+#pragma unroll
+    for (int t = 0; t < ROW_PF; ++t) jn[t] = d.nbr[(int64_t)min(t, d.cap - 1) * d.N + il];
+    __asm__ __volatile__("" ::: "memory");
+    bool in_kernel = false;
+    const long long st = stamp(epoch, pos);
     if (gate == G_NORMAL) {
-        if (c->halt || F->done) return;
-        int need = pending_rebuild(c, c->epoch, pos);
-        if (need) {
+        if (halted || done) return;
+        int need = pending_rebuild(c, epoch, pos);
+        // list rebuilds of a cell list are done here, row by row; the rest halts the chunk
+        in_kernel = need == 1 && nb.method == DPM_NBR_CELL && !ovf_pending(c, st);
+        if (need && !in_kernel) {
             if (threadIdx.x == 0) {
                 c->halt = 1;
                 c->halt_pos = pos;
@@ -1204,23 +1269,45 @@ __global__ __launch_bounds__(BLOCK) void k_fire_force(Dev d, PairParams p, int p
             return;
         }
     } else if (gate == G_RESUME) {
-        if (!c->halt || !resumable(d) || c->halt_mode != H_FIRE) return;
+        if (!halted || !resumable(d) || c->halt_mode != H_FIRE) return;
     }
-    double half = F->dt / 2.0;
-    const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    const bool live = i < d.N;
-    const int64_t il = live ? i : 0;
-    const double4 qi = d.P0[il];
-    const int nn = live ? min(d.nnum[il], d.cap) : 0;
+    if (in_kernel && live) {
+        const double2 xi = make_double2(qi.x, qi.y);
+        cnt = stencil_build<4>(d, nb, i, xi, [&](int j) {
+            const double4 q = d.P0[j];
+            return make_double2(q.x, q.y);
+        });
+        d.lref[i] = xi;
+        if (cnt > d.cap) c->ovf = st;
+#pragma unroll
+        for (int t = 0; t < ROW_PF; ++t) jn[t] = d.nbr[(int64_t)min(t, d.cap - 1) * d.N + il];
+    }
+    const int nn = live ? min(cnt, d.cap) : 0;
     double ax, ay, e;
-    row_forces<true, HOT>(d, d.P0, p, il, qi, nn, ax, ay, e);
+    row_forces_pf<true, HOT>(d, d.P0, p, il, qi, nn, jn, ax, ay, e);
+    if (in_kernel && live && cnt > d.cap) {  // the rest of a row that the ELL does not hold yet
+        int k = 0;
+        stencil_visit(d, nb, i, [&](int j) {
+            const double4 q = d.P0[j];
+            if (!within(qi.x, qi.y, q.x, q.y, nb, nb.rc2) || k++ < d.cap) return;
+            double fx, fy;
+            e += HOT ? pair_hot<true>(qi, q, true, p, fx, fy)
+                     : pair_law(qi.x, qi.y, qi.z, q.x, q.y, q.z, p, fx, fy);
+            ax += fx;
+            ay += fy;
+        });
+    }
+    if (in_kernel) {  // row-length statistics of the rebuild, one atomic per block
+        const int m = block_max_int(live ? cnt : 0);
+        if (threadIdx.x == 0) atomicMax(&c->max_nnum_all, m);
+        if (blockIdx.x == 0 && threadIdx.x == 0) c->n_rebuilds += 1;
+    }
     double pxv = 0.0, pyv = 0.0, pe = 0.0, f2 = 0.0;
     if (live) {
         double fx = 0.0 + ax, fy = 0.0 + ay;
         d.frc[i] = make_double2(fx, fy);
         pe = 0.0 + e;
         d.pe[i] = pe;
-        double2 v = d.vel[i];
         if (kick) {
             double dtm = half / qi.w;
             v.x += fx * dtm;
@@ -1233,56 +1320,78 @@ __global__ __launch_bounds__(BLOCK) void k_fire_force(Dev d, PairParams p, int p
     }
     int64_t nc = (d.N + CHUNK - 1) / CHUNK;
     double* P = d.part;
-    double s0 = wave_tree_sum(pxv);
-    double s1 = wave_tree_sum(pyv);
-    double s2 = wave_tree_sum(pe);
-    int64_t ch = i / CHUNK;
-    if ((threadIdx.x % WAVE) == 0 && ch < nc) {
-        P[ch] = s0;
-        P[nc + ch] = s1;
-        P[2 * nc + ch] = s2;
-    }
-    double b = block_max(f2);
-    if (threadIdx.x == 0) P[3 * nc + blockIdx.x] = b;
+    const double s = wave_reduce4(pxv, pe, pyv, f2);  // rows: F_x v_x, F_y v_y, PE, F^2
+    const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
+    const int64_t ch = i / CHUNK;
+    if (lane % 16 == 0 && lane < 48 && ch < nc) P[(lane / 16) * nc + ch] = s;
+    __shared__ double top[BLOCK / WAVE];
+    if (lane == 48) top[wv] = s;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        P[3 * nc + tile] = fmax(fmax(top[0], top[1]), fmax(top[2], top[3]));
 }
 
-// init: 1 = minimizeFire's prologue (records the first average energy)
-__global__ void k_fire_ctl(Dev d, int init, int pos, int gate) {
+// The canonical sums of a step's chunk partials, then fire_advance (init: fire_begin).  One
+// workgroup: all threads bring a stretch of the four partial arrays to LDS with their loads in
+// flight together, and one wave an array adds it in wave_final_sum's order.  (One wave that did
+// all of it waited for memory once per 256 partials: 33 us at 1,000,003 particles.)
+constexpr int CTL_T = 1024, CTL_STRETCH = 2048;
+
+__global__ __launch_bounds__(CTL_T) void k_fire_ctl(Dev d, int init, int pos, int gate) {
+    __shared__ double st[4][CTL_STRETCH];
+    __shared__ double res[4], top[CTL_T / WAVE];
     Ctl* c = d.ctl;
     FireCtl* F = d.fire;
+    const int T = (int)blockDim.x;
+    static_assert(sizeof(FireCtl) / sizeof(int) <= 4 * WAVE, "copied by words, one a thread");
+    __shared__ FireCtl S;
+    if (threadIdx.x < sizeof(FireCtl) / sizeof(int))
+        ((int*)&S)[threadIdx.x] = ((const int*)F)[threadIdx.x];
     if (gate == G_NORMAL) {
         if (c->halt || F->done) return;
     } else if (gate == G_RESUME) {
         if (!c->halt || !resumable(d) || c->halt_mode != H_FIRE) return;
     }
-    int64_t nc = (d.N + CHUNK - 1) / CHUNK;
-    int64_t nblk = (d.N + BLOCK - 1) / BLOCK;
+    const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
+    const int64_t nc = (d.N + CHUNK - 1) / CHUNK;
+    const int64_t nblk = (d.N + BLOCK - 1) / BLOCK;
     const double* P = d.part;
-    double px, py, pe, ptw;
-    // (the fourth array is the rigid spin power; a disk system sums px's array again)
-    wave_final_sum4(P, P + nc, P + 2 * nc, d.vpos ? P + 3 * nc + nblk : P, nc, px, py, pe, ptw);
-    if (!d.vpos) ptw = 0.0;
     double fm = 0.0;
-    {
-        int64_t k = threadIdx.x;
-        for (; k + (FS_ROWS - 1) * WAVE < nblk; k += FS_ROWS * WAVE) {
-            double v[FS_ROWS];
+    for (int64_t k = tid; k < nblk; k += T) fm = fmax(fm, P[3 * nc + k]);
+    const int arrays = d.vpos ? 4 : 3;  // the fourth is the rigid spin power
+    double s = 0.0;
+    for (int64_t base = 0; base < nc; base += CTL_STRETCH) {
+        const int len = (int)min((int64_t)CTL_STRETCH, nc - base);
+        if (base > 0) __syncthreads();
 #pragma unroll
-            for (int u = 0; u < FS_ROWS; ++u) v[u] = P[3 * nc + k + u * WAVE];
-#pragma unroll
-            for (int u = 0; u < FS_ROWS; ++u) fm = fmax(fm, v[u]);
-        }
-        for (; k < nblk; k += WAVE) fm = fmax(fm, P[3 * nc + k]);
+        for (int q = 0; q < 4; ++q)
+            if (q < arrays)
+                for (int k = tid; k < len; k += T)
+                    st[q][k] = P[q * nc + (q == 3 ? nblk : 0) + base + k];
+        __syncthreads();
+        if (wv < arrays)
+            for (int k = lane; k < len; k += WAVE) s = s + st[wv][k];
     }
     fm = wave_max(fm);
-    if (threadIdx.x != 0) return;
-    if (!init) {
-        if (gate == G_RESUME) c->progress += 1;  // the finished halted step
-        else c->progress = pos + 1;
+    if (lane == 0) top[wv] = fm;
+    if (wv < 4) {
+        s = wave_tree_sum(s);
+        if (lane == 0) res[wv] = s;
     }
-    const bool done = init ? fire_begin(*F, px, py, pe, fm, d.vpos ? &ptw : nullptr)
-                           : fire_advance(*F, px, py, pe, fm, d.vpos ? &ptw : nullptr);
-    if (done) c->done = 1;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < T / WAVE; ++w) fm = fmax(fm, top[w]);
+        if (!init) {
+            if (gate == G_RESUME) c->progress += 1;  // the finished halted step
+            else c->progress = pos + 1;
+        }
+        const double* spin = d.vpos ? &res[3] : nullptr;
+        const bool done = init ? fire_begin(S, res[0], res[1], res[2], fm, spin)
+                               : fire_advance(S, res[0], res[1], res[2], fm, spin);
+        if (done) c->done = 1;
+    }
+    __syncthreads();
+    if (tid < (int)(sizeof(FireCtl) / sizeof(int))) ((int*)F)[tid] = ((const int*)&S)[tid];
 }
 
 }  // namespace dpm
@@ -1604,6 +1713,10 @@ static void enqueue_rebuild(dpm_system* s, int gated) {
     if (s->kind == DPM_BUMPY) bumpy_enqueue_vertex_build(s, gated);
 }
 
+static dim3 ctl_threads(const dpm_system* s) {  // a wave an array, more where they are long
+    return dim3(s->nchunk <= 512 ? 4 * WAVE : CTL_T);
+}
+
 // The halted step's remaining work. resume: 0 none, 1 NVE, 2 FIRE, 3 rigid bumpy FIRE, 4 rigid
 // bumpy NVE.
 static void enqueue_resume(dpm_system* s, int resume, double dt) {
@@ -1617,12 +1730,12 @@ static void enqueue_resume(dpm_system* s, int resume, double dt) {
         hipLaunchKernelGGL(k_nve_kick_drift, pgrid(s->N), dim3(BLOCK), 0, st, d, nb, 0.5 * dt, dt,
                            0, 1, -1, (int)G_RESUME);
     } else if (resume == 2) {
-        LAUNCH_HOT(k_fire_force, dim3((unsigned)s->nblk), dim3(BLOCK), 0, st, d, p, 0, 1,
+        LAUNCH_HOT(k_fire_force, dim3((unsigned)s->nblk), dim3(BLOCK), 0, st, d, p, nb, 0, 1,
                            (int)G_RESUME);
-        hipLaunchKernelGGL(k_fire_ctl, dim3(1), dim3(WAVE), 0, st, d, 0, 0, (int)G_RESUME);
+        hipLaunchKernelGGL(k_fire_ctl, dim3(1), ctl_threads(s), 0, st, d, 0, 0, (int)G_RESUME);
     } else if (resume == 3) {  // rigid bumpy FIRE
         bumpy_enqueue_fire_forces(s, 1, G_RESUME);
-        hipLaunchKernelGGL(k_fire_ctl, dim3(1), dim3(WAVE), 0, st, d, 0, 0, (int)G_RESUME);
+        hipLaunchKernelGGL(k_fire_ctl, dim3(1), ctl_threads(s), 0, st, d, 0, 0, (int)G_RESUME);
     } else if (resume == 4) {
         bumpy_enqueue_nve_resume(s, dt);
     }
@@ -1757,10 +1870,10 @@ static void fire_chunk(dpm_system* s, double, int64_t c) {
         }
         {
             Timed t(s, DPM_K_FORCE);
-            LAUNCH_HOT(k_fire_force, dim3((unsigned)s->nblk), dim3(BLOCK), 0, st, d, p,
+            LAUNCH_HOT(k_fire_force, dim3((unsigned)s->nblk), dim3(BLOCK), 0, st, d, p, nb,
                                (int)k, 1, (int)G_NORMAL);
         }
-        hipLaunchKernelGGL(k_fire_ctl, dim3(1), dim3(WAVE), 0, st, d, 0, (int)k, (int)G_NORMAL);
+        hipLaunchKernelGGL(k_fire_ctl, dim3(1), ctl_threads(s), 0, st, d, 0, (int)k, (int)G_NORMAL);
     }
     enqueue_chain(s, 2, 0.0);
 }
@@ -1768,7 +1881,7 @@ static void fire_chunk(dpm_system* s, double, int64_t c) {
 static void bumpy_fire_chunk(dpm_system* s, double, int64_t c) {
     for (int64_t k = 0; k < c; ++k) {
         bumpy_enqueue_fire_step(s, (int)k);
-        hipLaunchKernelGGL(k_fire_ctl, dim3(1), dim3(WAVE), 0, s->stream, s->d, 0, (int)k,
+        hipLaunchKernelGGL(k_fire_ctl, dim3(1), ctl_threads(s), 0, s->stream, s->d, 0, (int)k,
                            (int)G_NORMAL);
     }
     enqueue_chain(s, 3, 0.0);
@@ -2055,10 +2168,10 @@ int minimize_fire(dpm_system* s, const dpm_fire_params* prm, dpm_fire_result* ou
     if (rigid) {
         bumpy_enqueue_fire_forces(s, 0, G_ALWAYS);
     } else {
-        LAUNCH_HOT(k_fire_force, dim3((unsigned)s->nblk), dim3(BLOCK), 0, st, d, p, 0, 0,
-                   (int)G_ALWAYS);
+        LAUNCH_HOT(k_fire_force, dim3((unsigned)s->nblk), dim3(BLOCK), 0, st, d, p,
+                   nbr_params(s), 0, 0, (int)G_ALWAYS);
     }
-    hipLaunchKernelGGL(k_fire_ctl, dim3(1), dim3(WAVE), 0, st, d, 1, 0, (int)G_ALWAYS);
+    hipLaunchKernelGGL(k_fire_ctl, dim3(1), ctl_threads(s), 0, st, d, 1, 0, (int)G_ALWAYS);
     if (check_launch()) return -1;
     if (prm->max_steps >= RESIDENT_MIN_STEPS && resident_ok(s)) {
         if (run_chunks(s, prm->max_steps, 0.0, 2, resident_fire_chunk, s->fire_graphs, true, true,

@@ -63,7 +63,6 @@ struct FireCtl {
     double last_avg_pe, avg_pe, power, fmax_sq;
     long long n_good, n_bad, step, max_steps;
     int stopped, done, converged, uphill;
-    int pad[4];
 };
 
 constexpr int HSCAL = 4;  // reductions whose results one wait collects
