@@ -53,8 +53,8 @@
 //               the closing kick and the chunk partials
 //   k_rb_eval   per particle (a half-wave over its vertices), before k_b_eval: the
 //               stress and contacts of a rigid system that finished a minimisation
-// Disk systems of up to RES_MAX_N particles take none of these launches: k_b_resident
-// (dpm_batch_resident.hpp) runs all their phases in one workgroup, many steps a launch.
+// Disk systems of up to RES_MAX_N particles take none of these launches: k_b_pairs or
+// k_b_resident (dpm_batch_resident.hpp) runs all their phases in one workgroup, many steps a launch.
 #include <algorithm>
 #include <chrono>
 #include <climits>
@@ -63,6 +63,7 @@
 #include <vector>
 
 #include "dpm_kernels.hpp"
+#include "dpm_resident.hpp"
 #include "dpm_rigid.hpp"
 
 namespace dpm {
@@ -1472,6 +1473,8 @@ struct dpm_batch {
     // resident systems (k_b_resident): their ids by size class, on the device; the launches of
     // the classes run side by side on streams of their own, forked from and joined to `stream`
     int* rids = nullptr;
+    unsigned short* rrows = nullptr;  // k_b_pairs' rows of the systems of two particles a thread
+    int rrows_for = 0;                // how many such systems it holds
     int rcount[dpm::RES_CLASSES] = {};
     bool phased = true;  // some system is advanced by the per-phase kernels
     hipStream_t rstream[dpm::RES_CLASSES] = {};
@@ -1739,7 +1742,7 @@ static void enqueue_batch_step(dpm_batch* b) {
 // Whether a system of n particles is advanced by k_b_resident: disks that fit a workgroup,
 // with a pair law of the short sequences (fastdiv), and no timing of the force pass asked for.
 // The line lies where the LDS ends: up to there one workgroup's step beats seven launches
-// (384 systems of 64 to 2,048 particles: 210 ms against 708 ms).
+// (384 systems of 64 to 2,048 particles: 157 ms against 708 ms).
 static bool resident_size(const dpm_batch* b, int64_t n, bool rigid, bool fastdiv) {
     return !rigid && fastdiv && !b->timing && n <= RES_MAX_N;
 }
@@ -1755,6 +1758,18 @@ static int resident_table(dpm_batch* b, const std::vector<std::pair<int, int64_t
             if (e.second <= RES_LIMIT[c] && (c == 0 || e.second > RES_LIMIT[c - 1]))
                 ids.push_back(e.first);
         b->rcount[c] = (int)(ids.size() - before);
+    }
+    if (b->rcount[RES_PAIRS_BIG] > b->rrows_for) {
+        if (b->rrows) {
+            b->allocs.erase(std::find(b->allocs.begin(), b->allocs.end(), (void*)b->rrows));
+            std::lock_guard<std::mutex> lk(capture_mutex());
+            (void)hipFree(b->rrows);
+        }
+        b->rrows = nullptr;
+        b->rrows_for = 0;
+        const int hold = (int)pow2_at_least(b->rcount[RES_PAIRS_BIG]);
+        if (balloc_n(b, &b->rrows, (long long)hold * RES_LC * RES_LIMIT[RES_PAIRS_BIG])) return -1;
+        b->rrows_for = hold;
     }
     if (!ids.empty()) BCOPY(b->rids, ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice);
     return 0;
@@ -1783,14 +1798,15 @@ static int resident_launch(dpm_batch* b, int64_t base, int64_t steps) {
         const long long b0 = base;
         const int k = (int)steps;
         switch (c) {
-            case 0: hipLaunchKernelGGL((k_b_resident<256, 1, 32>), grid, dim3(256), 0, st, b->d,
-                                       ids, b0, k); break;
-            case 1: hipLaunchKernelGGL((k_b_resident<512, 1, 32>), grid, dim3(512), 0, st, b->d,
-                                       ids, b0, k); break;
-            case 2: hipLaunchKernelGGL((k_b_resident<1024, 1, 24>), grid, dim3(1024), 0, st,
-                                       b->d, ids, b0, k); break;
-            case 3: hipLaunchKernelGGL((k_b_resident<1024, 2, 16>), grid, dim3(1024), 0, st,
-                                       b->d, ids, b0, k); break;
+            case 0: hipLaunchKernelGGL((k_b_pairs<512, 256>), grid, dim3(512), 0, st, b->d, ids,
+                                       b0, k, nullptr); break;
+            case 1: hipLaunchKernelGGL((k_b_pairs<1024, 512>), grid, dim3(1024), 0, st, b->d, ids,
+                                       b0, k, nullptr); break;
+            case 2: hipLaunchKernelGGL((k_b_pairs<1024, 1024>), grid, dim3(1024), 0, st, b->d,
+                                       ids, b0, k, nullptr); break;
+            case RES_PAIRS_BIG:
+                hipLaunchKernelGGL((k_b_pairs<1024, 2048>), grid, dim3(1024), 0, st, b->d, ids,
+                                   b0, k, b->rrows); break;
             default: hipLaunchKernelGGL((k_b_resident<1024, 4, 0>), grid, dim3(1024), 0, st,
                                         b->d, ids, b0, k);
         }

@@ -2125,8 +2125,8 @@ int nve_run(dpm_system* s, double dt, int64_t n) {
         if (run_chunks(s, n - 1, dt, 4, bumpy_nve_chunk, s->nve_graphs, false, false)) return -1;
         return bumpy_nve_step(s, dt);
     }
-    if (n >= RESIDENT_MIN_STEPS && resident_ok(s)) {
-        if (check_launch()) return -1;
+    if (n >= RESIDENT_MIN_STEPS && resident_ok(s, false)) {
+        if (check_launch() || resident_prepare(s)) return -1;
         return run_chunks(s, n, dt, 1, resident_nve_chunk, s->nve_graphs, false, true, nullptr,
                           RESIDENT_CHUNK * s->chunk);
     }
@@ -2173,8 +2173,9 @@ int minimize_fire(dpm_system* s, const dpm_fire_params* prm, dpm_fire_result* ou
     }
     hipLaunchKernelGGL(k_fire_ctl, dim3(1), ctl_threads(s), 0, st, d, 1, 0, (int)G_ALWAYS);
     if (check_launch()) return -1;
-    if (prm->max_steps >= RESIDENT_MIN_STEPS && resident_ok(s)) {
-        if (run_chunks(s, prm->max_steps, 0.0, 2, resident_fire_chunk, s->fire_graphs, true, true,
+    if (prm->max_steps >= RESIDENT_MIN_STEPS && resident_ok(s, true)) {
+        if (resident_prepare(s) ||
+            run_chunks(s, prm->max_steps, 0.0, 2, resident_fire_chunk, s->fire_graphs, true, true,
                        nullptr, RESIDENT_CHUNK * s->chunk))
             return -1;
     } else if (prm->max_steps > 0 &&

@@ -181,6 +181,7 @@ struct dpm_system {
     std::map<int64_t, dpm::Graph> nve_graphs, fire_graphs;
     dpm::Ctl* hctl = nullptr;   // pinned host mirror of the control block (4 slots),
                                 // written by the kernel that ends each launch unit
+    unsigned short* res_rows = nullptr;  // resident loops of two particles a thread (first use)
     double *hscal = nullptr, *hscal_dev = nullptr;  // pinned: reduction results (HSCAL)
     void* hstage = nullptr;     // pinned staging of small transfers (first use)
     double ktime_ms[3] = {0, 0, 0};

@@ -287,16 +287,17 @@ struct Timed {
 };
 
 // ---- small disk systems (dpm_resident.hip) ----
-// Loops of up to RESIDENT_MAX_N particles run in one workgroup, from RESIDENT_MIN_STEPS steps.
-// Measured against the chunked loops, us a step of 1,000: NVE 1.5 and 4.5 at 128 particles, 3.3
-// and 5.9 at 1,000; FIRE 3.4 and 14 at 128, 6.9 and 19.5 at 1,000; NVE in runs of 16 steps 5.0
-// and 7.2 at 1,000.  One CU's vector pipe bounds it: two particles a thread (2,000) took 11 us
-// for an NVE step that the chunked loop does in 6.1.
-constexpr int64_t RESIDENT_MAX_N = 1024;
+// Loops of up to RESIDENT_MAX_* particles run in one workgroup, from RESIDENT_MIN_STEPS steps.
+// Measured against the chunked loops, us a step of 1,000 (chunked, resident): NVE 4.5, 1.5 at
+// 128 particles; 5.9, 3.4 at 1,000; 6.1, 5.1 at 1,500; 6.1, 6.3 at 2,040; FIRE 14, 3.4 at 128;
+// 20, 7.2 at 1,000; 20, 14.4 at 2,040; NVE in runs of 16 steps 7.2, 5.0 at 1,000.  One CU's LDS
+// and vector pipe bound it, where the chunked step is launch gaps.
+constexpr int64_t RESIDENT_MAX_NVE = 1536, RESIDENT_MAX_FIRE = 2048;
 constexpr int64_t RESIDENT_MIN_STEPS = 16;
-bool resident_ok(const dpm_system* s);
-void resident_nve(dpm_system* s, double dt, int64_t steps);
-void resident_fire(dpm_system* s, int64_t steps);
+bool resident_ok(const dpm_system* s, bool fire);
+int resident_prepare(dpm_system* s);
+int resident_nve(dpm_system* s, double dt, int64_t steps);
+int resident_fire(dpm_system* s, int64_t steps);
 
 // ---- rigid bumpy (dpm_bumpy.hip) ----
 int bumpy_alloc(dpm_system* s);

@@ -1,6 +1,7 @@
-// dpm_resident.hpp -- a disk system of up to 1,024 particles held in one workgroup: positions,
+// dpm_resident.hpp -- a disk system of up to 2,048 particles held in one workgroup: positions,
 // radii and the list of pairs in LDS, the rest of a particle's state in the registers of its
-// thread.  Included by dpm_resident.hip.
+// thread.  Shared by the single-system loops (dpm_resident.hip) and the batched engine
+// (dpm_batch_resident.hpp).
 //
 // Near pairs.  The full rows (every particle within the list cutoff, what queries and the other
 // kernels read) go to the ELL in HBM; LDS holds the pairs that can touch before the list is next
@@ -27,6 +28,30 @@ __device__ __forceinline__ double uniform_d(double v) {
                             __builtin_amdgcn_readfirstlane(__double2loint(v)));
 }
 
+// The final stage of three chunk sums and a maximum (wave_final_sum), in part's rows 0 to 3:
+// lanes 0, 16, 32 and 48 receive them.  Up to 16 partials take the last four stages only; more
+// (up to 64) are halved first, lane t adding partial t + 32, then t + 16 (a sum that starts
+// from 0.0 has no negative zero, so a missing partial's 0.0 changes nothing).
+template <int NC>
+__device__ __forceinline__ double res_final(const double (&part)[4][NC], int nc) {
+    const int lane = threadIdx.x % WAVE, row = lane / 16, k = lane % 16;
+    auto at = [&](int t) { return t < nc ? 0.0 + part[row][t] : 0.0; };
+    double v = at(k);
+    auto join = [&](double a, double b) { return row < 3 ? a + b : fmax(a, b); };
+    if constexpr (NC > 32) v = join(join(v, at(k + 32)), join(at(k + 16), at(k + 48)));
+    else if constexpr (NC > 16) v = join(v, at(k + 16));
+    return rows_reduce(v);
+}
+
+// The thread's number, for the rare parts of a step loop (list builds): addresses formed from
+// threadIdx.x there are loop invariants, and the compiler kept some hundred registers of them
+// alive through the steps, which spilled.
+__device__ __forceinline__ int res_tid() {
+    int t = threadIdx.x;
+    __asm__ __volatile__("" : "+v"(t));
+    return t;
+}
+
 // Where the full rows are: entry k of slot i at nbr[k * stride + base + i], holding base + j
 struct ResRows {
     int* nbr;
@@ -34,33 +59,67 @@ struct ResRows {
     int cap;
 };
 
-// T threads, NP <= T particles at most, a cell grid of at most NP cells.  Rows of more than
-// RES_LC near entries or more than MP pairs (a mean of six near entries) make the system
-// "dense": its forces are then summed over the full rows.
+// Rows of more than RES_LC near entries or more than 3 NP pairs (a mean of six near entries), and
+// boxes too small for the branch-free minimum image, make a system "dense": its forces are then
+// summed over the full rows.
 constexpr int RES_LC = 16;
 constexpr unsigned short RES_FLIP = 0x8000;  // the particle is its pair's upper one
 
-template <int T, int NP_>
-struct ResCore {
-    static constexpr int NP = NP_, MP = 3 * NP_;
-    static_assert(NP <= T && MP < RES_FLIP, "a thread per particle, 15-bit pair numbers");
-    double2 x[NP];
-    double2 pf[MP + 1];  // force on the pair's lower particle; the last one stays zero
-    double pe[MP + 1];   // half pair energy
-    double r[NP];
-    unsigned pij[MP];                 // lower particle | upper particle << 16
-    unsigned short row[RES_LC][NP];   // near row: pair number (RES_FLIP), MP past its end
+// What a list build works on
+template <int NP>
+struct ResBuild {
+    unsigned pij[3 * NP];             // lower particle | upper particle << 16
+    unsigned short row[RES_LC][NP];   // near row: particles, then pair numbers (RES_FLIP), 3 NP
+                                      // past its end
     unsigned short first[NP];         // the particle's first pair (as the lower one)
     int cend[NP];                     // end of each cell's list
     unsigned short lst[NP];           // the cells' lists
+};
+
+// Build arrays and the pairs' results (force on the lower particle, half pair energy; the last
+// entry stays zero).  With two particles a thread LDS holds one of the three at a time: the
+// energies follow in the forces' place once those are summed, and after a build a thread keeps
+// its pairs in registers and the rows lie in HBM (read in order).
+template <int NP, bool BIG>
+struct ResPairs {
+    ResBuild<NP> b;
+    double2 f[3 * NP + 1];
+    double e[3 * NP + 1];
+};
+template <int NP>
+struct ResPairs<NP, true> {
+    union {
+        ResBuild<NP> b;
+        double2 f[3 * NP + 1];
+        double e[3 * NP + 1];
+    };
+};
+
+// T threads, NP particles at most (PPT a thread: tid, tid + T), a cell grid of at most NP cells
+template <int T_, int NP_>
+struct ResCore {
+    static constexpr int T = T_, NP = NP_, MP = 3 * NP, PPT = NP > T ? NP / T : 1;
+    static constexpr bool BIG = NP > T;
+    static constexpr int PAIRS = (MP + T - 1) / T;  // a thread's pairs
+    static_assert(MP < RES_FLIP, "15-bit pair numbers");
+    double2 x[NP];
+    ResPairs<NP, BIG> p;
+    double r[NP];
     int wsum[T / WAVE];
     int pairs, dense;
+};
+
+// A thread's pairs and the rows' place in HBM (BIG only; NP entries a column)
+template <int T, int NP>
+struct ResKept {
+    unsigned ij[ResCore<T, NP>::BIG ? ResCore<T, NP>::PAIRS : 1];
+    unsigned short* row;
 };
 
 // Exclusive prefix sum of v over the workgroup's threads; total receives the sum.  Two barriers.
 template <int T, int NP>
 __device__ __forceinline__ int res_scan(ResCore<T, NP>& L, int v, int& total) {
-    const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
+    const int tid = res_tid(), lane = tid % WAVE, wv = tid / WAVE;
     int incl = v;
 #pragma unroll
     for (int d = 1; d < WAVE; d <<= 1) {
@@ -81,30 +140,47 @@ __device__ __forceinline__ int res_scan(ResCore<T, NP>& L, int v, int& total) {
 }
 
 // Counting sort of the n particles into ncell <= NP cells, each list in ascending index: the
-// lists in L.lst, their ends in L.cend.  mine: the cell of the thread's particle.
+// lists in b.lst, their ends in b.cend.  mine: the cells of the thread's particles.
 template <int T, int NP>
-__device__ __forceinline__ void res_sort(ResCore<T, NP>& L, int n, int ncell, int mine) {
-    const int tid = threadIdx.x;
-    if (tid < ncell) L.cend[tid] = 0;
+__device__ __forceinline__ void res_sort(ResCore<T, NP>& L, int n, int ncell,
+                                         const int (&mine)[ResCore<T, NP>::PPT]) {
+    constexpr int PPT = ResCore<T, NP>::PPT;
+    ResBuild<NP>& B = L.p.b;
+    const int tid = res_tid();
+    for (int c = tid; c < ncell; c += T) B.cend[c] = 0;
     __syncthreads();
-    if (tid < n) atomicAdd(&L.cend[mine], 1);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m)
+        if (tid + m * T < n) atomicAdd(&B.cend[mine[m]], 1);
     __syncthreads();
-    int total;
-    const int run = res_scan(L, tid < ncell ? L.cend[tid] : 0, total);
-    if (tid < ncell) L.cend[tid] = run;
+    // each thread owns a run of consecutive cells
+    const int per = (ncell + T - 1) / T;
+    const int c0 = min(tid * per, ncell), c1 = min(c0 + per, ncell);
+    int local = 0, total;
+    for (int c = c0; c < c1; ++c) local += B.cend[c];
+    int run = res_scan(L, local, total);
+    for (int c = c0; c < c1; ++c) {
+        const int t = B.cend[c];
+        B.cend[c] = run;
+        run += t;
+    }
     __syncthreads();
-    if (tid < n) L.lst[atomicAdd(&L.cend[mine], 1)] = (unsigned short)tid;
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+        const int i = tid + m * T;
+        if (i < n) B.lst[atomicAdd(&B.cend[mine[m]], 1)] = (unsigned short)i;
+    }
     __syncthreads();
-    if (tid < ncell) {  // ascending members (a few per cell)
-        const int a = tid == 0 ? 0 : L.cend[tid - 1], e = L.cend[tid];
+    for (int c = tid; c < ncell; c += T) {  // ascending members (a few per cell)
+        const int a = c == 0 ? 0 : B.cend[c - 1], e = B.cend[c];
         for (int u = a + 1; u < e; ++u) {
-            const unsigned short v = L.lst[u];
+            const unsigned short v = B.lst[u];
             int k = u - 1;
-            while (k >= a && L.lst[k] > v) {
-                L.lst[k + 1] = L.lst[k];
+            while (k >= a && B.lst[k] > v) {
+                B.lst[k + 1] = B.lst[k];
                 --k;
             }
-            L.lst[k + 1] = v;
+            B.lst[k + 1] = v;
         }
     }
     __syncthreads();
@@ -124,29 +200,41 @@ __device__ __forceinline__ bool res_near(double2 a, double2 b, double rs, double
 
 __device__ __forceinline__ bool res_listed(double2 a, double2 b, double rc2,
                                            const PairParams& p) {
-    const double dx = pbc_rint(a.x, b.x, p.Lx, p.invLx);
-    const double dy = pbc_rint(a.y, b.y, p.Ly, p.invLy);
+    double dx, dy;
+    if (p.fast) {
+        dx = pbc_rint(a.x, b.x, p.Lx, p.invLx);
+        dy = pbc_rint(a.y, b.y, p.Ly, p.invLy);
+    } else {
+        dx = pbc(a.x, b.x, p.Lx, p.invLx, p.halfLx, 0);
+        dy = pbc(a.y, b.y, p.Ly, p.invLy, p.halfLy, 0);
+    }
     return dx * dx + dy * dy < rc2;
 }
 
-// The three runs of particles in the 3 x 3 cells around (cx, cy), lower row first: the cells of
-// a row are neighbours in L.lst, except where it wraps.  visit(a, b) takes list entries [a, b).
+// The runs of list entries in the 3 x 3 cells around (cx, cy), lower row first: the cells of
+// a row are neighbours in b.lst, except where it wraps.  visit(a, b) takes entries [a, b).
 template <int T, int NP, class Visit>
 __device__ __forceinline__ void res_stencil(const ResCore<T, NP>& L, int cx, int cy, int nx,
                                             int ny, Visit visit) {
-    auto start = [&](int c) { return c == 0 ? 0 : L.cend[c - 1]; };
-    for (int oy = -1; oy <= 1; ++oy) {
+    const int* cend = L.p.b.cend;
+    auto start = [&](int c) { return c == 0 ? 0 : cend[c - 1]; };
+    const bool wraps = cx == 0 || cx == nx - 1;
+    // (one copy of visit: unrolled, the build took the registers of the step loop around it)
+#pragma unroll 1
+    for (int t = 0; t < 6; ++t) {  // two parts a row; the second is empty without a wrap
+        const int oy = t / 2 - 1;
         const int y = cy + oy < 0 ? cy + oy + ny : (cy + oy >= ny ? cy + oy - ny : cy + oy);
-        const int c = y * nx;
-        if (cx == 0) visit(start(c + nx - 1), L.cend[c + nx - 1]);
-        visit(start(c + max(cx - 1, 0)), L.cend[c + min(cx + 1, nx - 1)]);
-        if (cx == nx - 1) visit(start(c), L.cend[c]);
+        const bool far = wraps && (t % 2 == 0) == (cx == 0);  // the part across the boundary
+        if (t % 2 == 1 && !wraps) continue;
+        const int c0 = y * nx + (far ? (cx == 0 ? nx - 1 : 0) : max(cx - 1, 0));
+        const int c1 = y * nx + (far ? (cx == 0 ? nx - 1 : 0) : min(cx + 1, nx - 1));
+        visit(start(c0), cend[c1]);
     }
 }
 
-// The row of the thread's particle under the cell method (stencil_build's order; the particles
-// are in cell order, so list entry j is particle j): the full row in HBM, the near row's
-// particles in L.row.  Returns the full length; near receives the near row's.
+// The row of particle i under the cell method (stencil_build's order; the particles are in cell
+// order, so list entry j is particle j): the full row in HBM, the near row's particles in b.row.
+// Returns the full length; near receives the near row's.
 template <int T, int NP>
 __device__ __forceinline__ int res_row_cell(ResCore<T, NP>& L, const ResRows& R, int i, int cell,
                                             int nc, double rc2, double delta2,
@@ -155,13 +243,14 @@ __device__ __forceinline__ int res_row_cell(ResCore<T, NP>& L, const ResRows& R,
     const double ri = L.r[i];
     int cnt = 0, nr = 0;
     res_stencil(L, cell % nc, cell / nc, nc, nc, [&](int a, int b) {
+#pragma unroll 1
         for (int j = a; j < b; ++j) {
             const double2 xj = L.x[j];
             if (j == i || !res_listed(xi, xj, rc2, p)) continue;
             if (cnt < R.cap) R.nbr[(long long)cnt * R.stride + R.base + i] = (int)(R.base + j);
             cnt++;
             if (!res_near(xi, xj, ri + L.r[j], delta2, p)) continue;
-            if (nr < RES_LC) L.row[nr][i] = (unsigned short)j;
+            if (nr < RES_LC) L.p.b.row[nr][i] = (unsigned short)j;
             nr++;
         }
     });
@@ -171,7 +260,7 @@ __device__ __forceinline__ int res_row_cell(ResCore<T, NP>& L, const ResRows& R,
 
 // The same under the Verlet method: the particles within the cutoff in ascending index, from
 // the lists of a cell grid (cells at least the cutoff wide) or, without one, from all pairs.
-// Hits are kept sorted in L.row; a row that does not fit there is found by increasing index,
+// Hits are kept sorted in b.row; a row that does not fit there is found by increasing index,
 // one pass over the candidates an entry.
 template <int T, int NP>
 __device__ __forceinline__ int res_row_verlet(ResCore<T, NP>& L, const ResRows& R, int i, int n,
@@ -180,47 +269,54 @@ __device__ __forceinline__ int res_row_verlet(ResCore<T, NP>& L, const ResRows& 
                                               int& near) {
     const double2 xi = L.x[i];
     const double ri = L.r[i];
+    auto& row = L.p.b.row;
+    const unsigned short* lst = L.p.b.lst;
     int cnt = 0, nr = 0;
     auto put = [&](int k, int j) {
         if (k < R.cap) R.nbr[(long long)k * R.stride + R.base + i] = (int)(R.base + j);
     };
     if (!grid) {
+#pragma unroll 1
         for (int j = 0; j < n; ++j) {
             const double2 xj = L.x[j];
             if (j == i || !res_listed(xi, xj, rc2, p)) continue;
             put(cnt++, j);
             if (!res_near(xi, xj, ri + L.r[j], delta2, p)) continue;
-            if (nr < RES_LC) L.row[nr][i] = (unsigned short)j;
+            if (nr < RES_LC) row[nr][i] = (unsigned short)j;
             nr++;
         }
         near = nr;
         return cnt;
     }
     res_stencil(L, cx, cy, nx, ny, [&](int a, int b) {
+#pragma unroll 1
         for (int u = a; u < b; ++u) {
-            const int j = L.lst[u];
+            const int j = lst[u];
             if (j == i || !res_listed(xi, L.x[j], rc2, p)) continue;
             if (cnt < RES_LC) {
                 int k = cnt;
-                for (; k > 0 && L.row[k - 1][i] > j; --k) L.row[k][i] = L.row[k - 1][i];
-                L.row[k][i] = (unsigned short)j;
+                for (; k > 0 && row[k - 1][i] > j; --k) row[k][i] = row[k - 1][i];
+                row[k][i] = (unsigned short)j;
             }
             cnt++;
         }
     });
     if (cnt <= RES_LC) {
+#pragma unroll 1
         for (int k = 0; k < cnt; ++k) {
-            const int j = L.row[k][i];
+            const int j = row[k][i];
             put(k, j);
-            if (res_near(xi, L.x[j], ri + L.r[j], delta2, p)) L.row[nr++][i] = (unsigned short)j;
+            if (res_near(xi, L.x[j], ri + L.r[j], delta2, p)) row[nr++][i] = (unsigned short)j;
         }
     } else {
         nr = cnt;  // dense: the forces walk the full rows
+#pragma unroll 1
         for (int k = 0, last = -1; k < cnt; ++k) {
             int next = n;
             res_stencil(L, cx, cy, nx, ny, [&](int a, int b) {
+#pragma unroll 1
                 for (int u = a; u < b; ++u) {
-                    const int j = L.lst[u];
+                    const int j = lst[u];
                     if (j > last && j < next && j != i && res_listed(xi, L.x[j], rc2, p)) next = j;
                 }
             });
@@ -232,7 +328,8 @@ __device__ __forceinline__ int res_row_verlet(ResCore<T, NP>& L, const ResRows& 
     return cnt;
 }
 
-// The near row of a list that an earlier launch built (reference positions ref[base + j]).
+// The near row of a list that was built before (reference positions ref[base + j]), in the
+// present box.
 template <int T, int NP>
 __device__ __forceinline__ int res_load_row(ResCore<T, NP>& L, const ResRows& R,
                                             const double2* ref, int i, int full, double delta2,
@@ -241,73 +338,89 @@ __device__ __forceinline__ int res_load_row(ResCore<T, NP>& L, const ResRows& R,
     const double ri = L.r[i];
     const int nn = min(full, R.cap);
     int near = 0;
+#pragma unroll 1
     for (int k = 0; k < nn; ++k) {
         const int j = (int)(R.nbr[(long long)k * R.stride + R.base + i] - R.base);
         if (!res_near(xi, ref[R.base + j], ri + L.r[j], delta2, p)) continue;
-        if (near < RES_LC) L.row[near][i] = (unsigned short)j;
+        if (near < RES_LC) L.p.b.row[near][i] = (unsigned short)j;
         near++;
     }
     return near;
 }
 
-// The pairs of the near rows (particle numbers in L.row, `near` of the thread's particle; 0
-// without one): numbered by lower particle, then in its row's order; L.row receives the pair
-// numbers.  Returns the length of the force sum's row.  Ends with a barrier.
+// The pairs of the near rows (particle numbers in b.row; near[m]: their lengths, 0 without a
+// particle): numbered by lower particle, then in its row's order; b.row receives the pair
+// numbers (BIG: K, which outlives the build arrays).  len[m]: the lengths of the force sums.
+// Ends with a barrier.
 template <int T, int NP>
-__device__ __forceinline__ int res_pairs(ResCore<T, NP>& L, int n, int near) {
-    const int i = threadIdx.x;
-    const int nr = min(near, RES_LC);
-    int own = 0;
-    for (int k = 0; k < nr; ++k) own += (int)L.row[k][i] > i ? 1 : 0;
-    if (i == 0) L.dense = 0;
-    int total;
-    const int first = res_scan(L, own, total);  // (its barriers order the write above)
-    if (near > RES_LC || total > L.MP) L.dense = 1;
-    if (i < n) L.first[i] = (unsigned short)min(first, L.MP);
-    if (i == 0) {
-        L.pairs = min(total, L.MP);
-        L.pf[L.MP] = make_double2(0.0, 0.0);
-        L.pe[L.MP] = 0.0;
+__device__ __forceinline__ void res_pairs(ResCore<T, NP>& L, ResKept<T, NP>& K, int n, bool fast,
+                                          const int (&near)[ResCore<T, NP>::PPT],
+                                          int (&len)[ResCore<T, NP>::PPT]) {
+    constexpr int PPT = ResCore<T, NP>::PPT, MP = ResCore<T, NP>::MP;
+    ResBuild<NP>& B = L.p.b;
+    const int tid = res_tid();
+    if (tid == 0) L.dense = fast ? 0 : 1;
+    int total = 0, first[PPT];
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+        const int i = tid + m * T, nr = min(near[m], RES_LC);
+        int own = 0, sum;
+#pragma unroll 1
+        for (int k = 0; k < nr; ++k) own += (int)B.row[k][i] > i ? 1 : 0;
+        first[m] = total + res_scan(L, own, sum);  // (its barriers order the write above)
+        total += sum;
+        len[m] = nr;
     }
-    for (int k = 0, s = first; k < nr; ++k) {
-        const int j = L.row[k][i];
-        if (j > i && s < L.MP) L.pij[s++] = (unsigned)i | (unsigned)j << 16;
-    }
-    __syncthreads();
-    if (i < n && !L.dense) {
-        for (int k = 0, s = first; k < nr; ++k) {
-            const int j = L.row[k][i];
-            unsigned short e;
-            if (j > i) {
-                e = (unsigned short)s++;
-            } else {  // listed by j, whose pairs are consecutive
-                int t = L.first[j];
-                while (t < L.pairs && (int)(L.pij[t] >> 16) != i) ++t;
-                if (t == L.pairs) L.dense = 1;  // (rows that are not symmetric)
-                e = (unsigned short)t | RES_FLIP;
-            }
-            L.row[k][i] = e;
+    bool over = total > MP;
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+        const int i = tid + m * T;
+        over = over || near[m] > RES_LC;
+        if (i >= n) continue;
+        B.first[i] = (unsigned short)min(first[m], MP);
+#pragma unroll 1
+        for (int k = 0, s = first[m]; k < len[m]; ++k) {
+            const int j = B.row[k][i];
+            if (j > i && s < MP) B.pij[s++] = (unsigned)i | (unsigned)j << 16;
         }
-        for (int k = nr; k < RES_LC; ++k) L.row[k][i] = (unsigned short)L.MP;
+    }
+    if (over) L.dense = 1;
+    if (tid == 0) L.pairs = min(total, MP);
+    __syncthreads();
+    if (!L.dense) {
+#pragma unroll
+        for (int m = 0; m < PPT; ++m) {
+            const int i = tid + m * T;
+            if (i >= NP) continue;
+#pragma unroll 1
+            for (int k = 0, s = first[m]; k < len[m]; ++k) {
+                const int j = B.row[k][i];
+                unsigned short e;
+                if (j > i) {
+                    e = (unsigned short)s++;
+                } else {  // listed by j, whose pairs are consecutive
+                    int t = B.first[j];
+                    while (t < L.pairs && (int)(B.pij[t] >> 16) != i) ++t;
+                    if (t == L.pairs) L.dense = 1;  // (rows that are not symmetric)
+                    e = (unsigned short)t | RES_FLIP;
+                }
+                B.row[k][i] = e;
+            }
+            for (int k = len[m]; k < RES_LC; ++k) B.row[k][i] = (unsigned short)MP;
+        }
+    }
+    if constexpr (ResCore<T, NP>::BIG) {
+#pragma unroll
+        for (int k = 0; k < ResCore<T, NP>::PAIRS; ++k) {
+            const int t = tid + k * T;
+            K.ij[k] = t < MP ? B.pij[t] : 0u;
+        }
+#pragma unroll
+        for (int m = 0; m < PPT; ++m)
+            for (int k = 0; k < RES_LC; ++k)
+                K.row[k * NP + tid + m * T] = B.row[k][tid + m * T];
     }
     __syncthreads();
-    return nr;
-}
-
-// Every pair's force and energy (no barrier at either end)
-template <bool ENERGY, int T, int NP>
-__device__ __forceinline__ void res_pair_forces(ResCore<T, NP>& L, const PairParams& p) {
-    const int np = L.pairs;
-    for (int t = threadIdx.x; t < np; t += T) {
-        const unsigned ij = L.pij[t];
-        const int i = (int)(ij & 0xffff), j = (int)(ij >> 16);
-        const double2 a = L.x[i], b = L.x[j];
-        double fx, fy;
-        const double e = pair_hot<ENERGY>(make_double4(a.x, a.y, L.r[i], 0.0),
-                                          make_double4(b.x, b.y, L.r[j], 0.0), true, p, fx, fy);
-        L.pf[t] = make_double2(fx, fy);
-        if (ENERGY) L.pe[t] = e;
-    }
 }
 
 // v with its sign flipped where the entry is the pair's upper particle
@@ -316,35 +429,102 @@ __device__ __forceinline__ double res_flip(double v, unsigned e) {
     return __hiloint2double((int)((unsigned)__double2hiint(v) ^ s), __double2loint(v));
 }
 
-// The sums of the thread's particle over its row of nn pairs, in row order; the wave walks its
-// longest row, four entries at a time (entries past the end are the zero pair)
+// Forces (and energies) of the thread's particles: every pair once, then the sums over the rows
+// of len[m] pairs in row order (the wave walks its longest row, four entries at a time; entries
+// past the end are the zero pair).  Every position has been written behind a barrier; no thread
+// reads a position or writes a pair's result after the last barrier in here.
 template <bool ENERGY, int T, int NP>
-__device__ __forceinline__ void res_sum(const ResCore<T, NP>& L, int i, int nn, double& ax,
-                                        double& ay, double& e) {
-    ax = 0.0;
-    ay = 0.0;
-    e = 0.0;
-    for (int k = 0; __builtin_amdgcn_ballot_w64(k < nn) != 0; k += 4) {
-        unsigned s[4];
-        double2 f[4];
-        double w[4];
+__device__ __forceinline__ void res_forces(ResCore<T, NP>& L, const ResKept<T, NP>& K,
+                                           const PairParams& p, int nc,
+                                           const int (&len)[ResCore<T, NP>::PPT],
+                                           double (&ax)[ResCore<T, NP>::PPT],
+                                           double (&ay)[ResCore<T, NP>::PPT],
+                                           double (&e)[ResCore<T, NP>::PPT]) {
+    using C = ResCore<T, NP>;
+    constexpr int PPT = C::PPT, MP = C::MP;
+    const int tid = threadIdx.x, np = L.pairs;
+    double keep[C::BIG ? C::PAIRS : 1];
+    auto pair = [&](int t, unsigned ij) {
+        const int i = (int)(ij & 0xffff), j = (int)(ij >> 16);
+        const double2 a = L.x[i], b = L.x[j];
+        double fx, fy;
+        const double w = pair_hot<ENERGY>(make_double4(a.x, a.y, L.r[i], 0.0),
+                                          make_double4(b.x, b.y, L.r[j], 0.0), true, p, fx, fy);
+        L.p.f[t] = make_double2(fx, fy);
+        return w;
+    };
+    if constexpr (C::BIG) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) s[t] = L.row[k + t][i];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            f[t] = L.pf[s[t] & (RES_FLIP - 1)];
-            if (ENERGY) w[t] = L.pe[s[t] & (RES_FLIP - 1)];
+        for (int k = 0; k < C::PAIRS; ++k) {
+            const int t = tid + k * T;
+            keep[k] = 0.0;
+            if (t < np) keep[k] = pair(t, K.ij[k]);
+            if (k % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // (six at once spill)
         }
+    } else {
+        for (int t = tid; t < np; t += T) {
+            const double w = pair(t, L.p.b.pij[t]);
+            if (ENERGY) L.p.e[t] = w;
+        }
+    }
+    if (tid == 0) {
+        L.p.f[MP] = make_double2(0.0, 0.0);
+        if (ENERGY && !C::BIG) L.p.e[MP] = 0.0;
+    }
+    __syncthreads();
+    auto entry = [&](int k, int i) -> unsigned {
+        if constexpr (C::BIG) return K.row[k * NP + i];
+        else return L.p.b.row[k][i];
+    };
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            ax += res_flip(f[t].x, s[t]);
-            ay += res_flip(f[t].y, s[t]);
-            if (ENERGY) e += w[t];
+    for (int m = 0; m < PPT; ++m) {
+        ax[m] = ay[m] = e[m] = 0.0;
+        const int i = tid + m * T;
+        if (i / WAVE >= nc) continue;  // uniform over the wave
+#pragma unroll 1
+        for (int k = 0; __builtin_amdgcn_ballot_w64(k < len[m]) != 0; k += 4) {
+            unsigned s[4];
+            double2 f[4];
+            double w[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) s[t] = entry(k + t, i);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                f[t] = L.p.f[s[t] & (RES_FLIP - 1)];
+                if (ENERGY && !C::BIG) w[t] = L.p.e[s[t] & (RES_FLIP - 1)];
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                ax[m] += res_flip(f[t].x, s[t]);
+                ay[m] += res_flip(f[t].y, s[t]);
+                if (ENERGY && !C::BIG) e[m] += w[t];
+            }
+        }
+    }
+    if constexpr (ENERGY && C::BIG) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < C::PAIRS; ++k)
+            if (tid + k * T < np) L.p.e[tid + k * T] = keep[k];
+        if (tid == 0) L.p.e[MP] = 0.0;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < PPT; ++m) {
+            const int i = tid + m * T;
+            if (i / WAVE >= nc) continue;
+            for (int k = 0; __builtin_amdgcn_ballot_w64(k < len[m]) != 0; k += 4) {
+                unsigned s[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) s[t] = entry(k + t, i);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) e[m] += L.p.e[s[t] & (RES_FLIP - 1)];
+            }
         }
     }
 }
 
-// The same over the full row in HBM, pair by pair (dense systems)
+// The same over the full row in HBM, pair by pair (dense systems).  No barrier: the positions
+// must rest until every thread is through.
 template <int T, int NP>
 __device__ __forceinline__ void res_sum_full(const ResCore<T, NP>& L, const ResRows& R,
                                              const PairParams& p, int i, int full, double& ax,
@@ -353,11 +533,13 @@ __device__ __forceinline__ void res_sum_full(const ResCore<T, NP>& L, const ResR
     ax = 0.0;
     ay = 0.0;
     e = 0.0;
+#pragma unroll 1
     for (int k = 0; k < min(full, R.cap); ++k) {
         const int j = (int)(R.nbr[(long long)k * R.stride + R.base + i] - R.base);
+        const double4 qj = make_double4(L.x[j].x, L.x[j].y, L.r[j], 0.0);
         double fx, fy;
-        const double ie = pair_hot<true>(qi, make_double4(L.x[j].x, L.x[j].y, L.r[j], 0.0), true,
-                                         p, fx, fy);
+        const double ie = p.fast ? pair_hot<true>(qi, qj, true, p, fx, fy)
+                                 : pair_hot<true, true>(qi, qj, true, p, fx, fy);
         ax += fx;
         ay += fy;
         e += ie;

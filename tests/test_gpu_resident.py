@@ -55,7 +55,7 @@ def fire(s, steps, fmax=0.0):
 
 
 @pytest.mark.parametrize("method", (CELL, VERLET))
-@pytest.mark.parametrize("n", (30, 64, 65, 256, 257, 512, 513, 1023, 1024, 1025))
+@pytest.mark.parametrize("n", (30, 64, 65, 256, 257, 512, 513, 1023, 1024, 1025, 2048, 2049))
 def test_fire_then_nve(n, method):
     print("[gpu-case] resident", n, method, flush=True)
     g, o = pair(n, 0.84, method, seed=n)
@@ -117,6 +117,7 @@ def test_rows_outgrow_the_ell(method):
     (600, 1.3, CELL, 0.3),    # more pairs than the pair list holds
     (600, 1.3, VERLET, 0.3),
     (200, 0.9, VERLET, 1.5),  # near rows longer than the row table
+    (1500, 1.3, CELL, 0.3),
 ))
 def test_small_boxes_and_dense_systems(n, phi, method, skin):
     g, o = pair(n, phi, method, seed=2, skin=skin)
