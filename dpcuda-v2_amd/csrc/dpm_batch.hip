@@ -53,8 +53,8 @@
 //               the closing kick and the chunk partials
 //   k_rb_eval   per particle (a half-wave over its vertices), before k_b_eval: the
 //               stress and contacts of a rigid system that finished a minimisation
-// Disk systems of up to RES_MAX_N particles take none of these launches: k_b_pairs or
-// k_b_resident (dpm_batch_resident.hpp) runs all their phases in one workgroup, many steps a launch.
+// Disk systems of up to RES_MAX_N particles take none of these launches: k_b_resident
+// (dpm_batch_resident.hpp) runs all their phases in one workgroup, many steps a launch.
 #include <algorithm>
 #include <chrono>
 #include <climits>
@@ -1473,8 +1473,9 @@ struct dpm_batch {
     // resident systems (k_b_resident): their ids by size class, on the device; the launches of
     // the classes run side by side on streams of their own, forked from and joined to `stream`
     int* rids = nullptr;
-    unsigned short* rrows = nullptr;  // k_b_pairs' rows of the systems of two particles a thread
-    int rrows_for = 0;                // how many such systems it holds
+    // near rows of the classes from RES_ROWS on, and how many systems they are for
+    unsigned short* rrows[dpm::RES_CLASSES - dpm::RES_ROWS] = {nullptr, nullptr};
+    int rrows_for[dpm::RES_CLASSES - dpm::RES_ROWS] = {0, 0};
     int rcount[dpm::RES_CLASSES] = {};
     bool phased = true;  // some system is advanced by the per-phase kernels
     hipStream_t rstream[dpm::RES_CLASSES] = {};
@@ -1759,17 +1760,20 @@ static int resident_table(dpm_batch* b, const std::vector<std::pair<int, int64_t
                 ids.push_back(e.first);
         b->rcount[c] = (int)(ids.size() - before);
     }
-    if (b->rcount[RES_PAIRS_BIG] > b->rrows_for) {
-        if (b->rrows) {
-            b->allocs.erase(std::find(b->allocs.begin(), b->allocs.end(), (void*)b->rrows));
+    for (int c = RES_ROWS; c < RES_CLASSES; ++c) {
+        unsigned short*& rows = b->rrows[c - RES_ROWS];
+        int& held = b->rrows_for[c - RES_ROWS];
+        if (b->rcount[c] <= held) continue;
+        if (rows) {
+            b->allocs.erase(std::find(b->allocs.begin(), b->allocs.end(), (void*)rows));
             std::lock_guard<std::mutex> lk(capture_mutex());
-            (void)hipFree(b->rrows);
+            (void)hipFree(rows);
         }
-        b->rrows = nullptr;
-        b->rrows_for = 0;
-        const int hold = (int)pow2_at_least(b->rcount[RES_PAIRS_BIG]);
-        if (balloc_n(b, &b->rrows, (long long)hold * RES_LC * RES_LIMIT[RES_PAIRS_BIG])) return -1;
-        b->rrows_for = hold;
+        rows = nullptr;
+        held = 0;
+        const int hold = (int)pow2_at_least(b->rcount[c]);
+        if (balloc_n(b, &rows, (long long)hold * RES_LC * RES_LIMIT[c])) return -1;
+        held = hold;
     }
     if (!ids.empty()) BCOPY(b->rids, ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice);
     return 0;
@@ -1798,17 +1802,16 @@ static int resident_launch(dpm_batch* b, int64_t base, int64_t steps) {
         const long long b0 = base;
         const int k = (int)steps;
         switch (c) {
-            case 0: hipLaunchKernelGGL((k_b_pairs<512, 256>), grid, dim3(512), 0, st, b->d, ids,
+            case 0: hipLaunchKernelGGL((k_b_resident<512, 256>), grid, dim3(512), 0, st, b->d, ids,
                                        b0, k, nullptr); break;
-            case 1: hipLaunchKernelGGL((k_b_pairs<1024, 512>), grid, dim3(1024), 0, st, b->d, ids,
+            case 1: hipLaunchKernelGGL((k_b_resident<1024, 512>), grid, dim3(1024), 0, st, b->d, ids,
                                        b0, k, nullptr); break;
-            case 2: hipLaunchKernelGGL((k_b_pairs<1024, 1024>), grid, dim3(1024), 0, st, b->d,
+            case 2: hipLaunchKernelGGL((k_b_resident<1024, 1024>), grid, dim3(1024), 0, st, b->d,
                                        ids, b0, k, nullptr); break;
-            case RES_PAIRS_BIG:
-                hipLaunchKernelGGL((k_b_pairs<1024, 2048>), grid, dim3(1024), 0, st, b->d, ids,
-                                   b0, k, b->rrows); break;
-            default: hipLaunchKernelGGL((k_b_resident<1024, 4, 0>), grid, dim3(1024), 0, st,
-                                        b->d, ids, b0, k);
+            case 3: hipLaunchKernelGGL((k_b_resident<1024, 2048>), grid, dim3(1024), 0, st, b->d,
+                                       ids, b0, k, b->rrows[0]); break;
+            default: hipLaunchKernelGGL((k_b_resident<1024, 4096>), grid, dim3(1024), 0, st, b->d,
+                                        ids, b0, k, b->rrows[1]);
         }
         if (check_launch()) return -1;
         DPM_HIP(hipEventRecord(b->rjoin[c], st));

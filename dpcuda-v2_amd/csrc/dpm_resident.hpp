@@ -1,6 +1,6 @@
-// dpm_resident.hpp -- a disk system of up to 2,048 particles held in one workgroup: positions,
-// radii and the list of pairs in LDS, the rest of a particle's state in the registers of its
-// thread.  Shared by the single-system loops (dpm_resident.hip) and the batched engine
+// dpm_resident.hpp -- a disk system of up to 4,096 particles held in one workgroup: positions,
+// radii and (up to 2,048) the list of pairs in LDS, the rest of a particle's state in the
+// registers of its thread.  Shared by the single-system loops (dpm_resident.hip) and the batched engine
 // (dpm_batch_resident.hpp).
 //
 // Near pairs.  The full rows (every particle within the list cutoff, what queries and the other
@@ -65,54 +65,70 @@ struct ResRows {
 constexpr int RES_LC = 16;
 constexpr unsigned short RES_FLIP = 0x8000;  // the particle is its pair's upper one
 
+// How a system of NP particles is held by T threads
+enum ResForm {
+    RES_SMALL,  // a particle a thread: pairs and their results in LDS
+    RES_BIG,    // two: LDS holds the build arrays, the pairs' forces or their energies at a time
+                // (the energies follow in the forces' place once those are summed); after a build
+                // a thread keeps its pairs in registers and the rows lie in HBM (read in order)
+    RES_WALK    // four: LDS holds positions and radii, the near rows lie in HBM and are walked
+                // from both sides
+};
+
 // What a list build works on
-template <int NP>
+template <int NP, int COLS, bool PAIRS>
 struct ResBuild {
-    unsigned pij[3 * NP];             // lower particle | upper particle << 16
-    unsigned short row[RES_LC][NP];   // near row: particles, then pair numbers (RES_FLIP), 3 NP
+    unsigned short row[RES_LC][COLS]; // near row: particles, then pair numbers (RES_FLIP), 3 NP
                                       // past its end
-    unsigned short first[NP];         // the particle's first pair (as the lower one)
     int cend[NP];                     // end of each cell's list
     unsigned short lst[NP];           // the cells' lists
+    unsigned short first[PAIRS ? NP : 1];  // the particle's first pair (as the lower one)
+    unsigned pij[PAIRS ? 3 * NP : 1];      // lower particle | upper particle << 16
 };
 
 // Build arrays and the pairs' results (force on the lower particle, half pair energy; the last
-// entry stays zero).  With two particles a thread LDS holds one of the three at a time: the
-// energies follow in the forces' place once those are summed, and after a build a thread keeps
-// its pairs in registers and the rows lie in HBM (read in order).
-template <int NP, bool BIG>
+// entry stays zero)
+template <int T, int NP, ResForm FORM>
 struct ResPairs {
-    ResBuild<NP> b;
+    ResBuild<NP, NP, true> b;
     double2 f[3 * NP + 1];
     double e[3 * NP + 1];
 };
-template <int NP>
-struct ResPairs<NP, true> {
+template <int T, int NP>
+struct ResPairs<T, NP, RES_BIG> {
     union {
-        ResBuild<NP> b;
+        ResBuild<NP, NP, true> b;
         double2 f[3 * NP + 1];
         double e[3 * NP + 1];
     };
 };
+template <int T, int NP>
+struct ResPairs<T, NP, RES_WALK> {
+    ResBuild<NP, T, false> b;
+};
 
-// T threads, NP particles at most (PPT a thread: tid, tid + T), a cell grid of at most NP cells
+// T threads, NP particles at most (PPT a thread: tid, tid + T, ...), a cell grid of at most NP
+// cells
 template <int T_, int NP_>
 struct ResCore {
     static constexpr int T = T_, NP = NP_, MP = 3 * NP, PPT = NP > T ? NP / T : 1;
-    static constexpr bool BIG = NP > T;
+    static constexpr ResForm FORM = PPT == 1 ? RES_SMALL : (PPT == 2 ? RES_BIG : RES_WALK);
+    static constexpr bool BIG = PPT > 1;
     static constexpr int PAIRS = (MP + T - 1) / T;  // a thread's pairs
-    static_assert(MP < RES_FLIP, "15-bit pair numbers");
+    static_assert(FORM == RES_WALK || MP < RES_FLIP, "15-bit pair numbers");
     double2 x[NP];
-    ResPairs<NP, BIG> p;
+    ResPairs<T, NP, FORM> p;
     double r[NP];
     int wsum[T / WAVE];
     int pairs, dense;
+    // the column of particle i in p.b.row
+    static __device__ __forceinline__ int col(int i) { return FORM == RES_WALK ? i % T : i; }
 };
 
-// A thread's pairs and the rows' place in HBM (BIG only; NP entries a column)
+// A thread's pairs and the rows' place in HBM (not RES_SMALL; NP entries a column)
 template <int T, int NP>
 struct ResKept {
-    unsigned ij[ResCore<T, NP>::BIG ? ResCore<T, NP>::PAIRS : 1];
+    unsigned ij[ResCore<T, NP>::FORM == RES_BIG ? ResCore<T, NP>::PAIRS : 1];
     unsigned short* row;
 };
 
@@ -145,7 +161,7 @@ template <int T, int NP>
 __device__ __forceinline__ void res_sort(ResCore<T, NP>& L, int n, int ncell,
                                          const int (&mine)[ResCore<T, NP>::PPT]) {
     constexpr int PPT = ResCore<T, NP>::PPT;
-    ResBuild<NP>& B = L.p.b;
+    auto& B = L.p.b;
     const int tid = res_tid();
     for (int c = tid; c < ncell; c += T) B.cend[c] = 0;
     __syncthreads();
@@ -250,7 +266,7 @@ __device__ __forceinline__ int res_row_cell(ResCore<T, NP>& L, const ResRows& R,
             if (cnt < R.cap) R.nbr[(long long)cnt * R.stride + R.base + i] = (int)(R.base + j);
             cnt++;
             if (!res_near(xi, xj, ri + L.r[j], delta2, p)) continue;
-            if (nr < RES_LC) L.p.b.row[nr][i] = (unsigned short)j;
+            if (nr < RES_LC) L.p.b.row[nr][L.col(i)] = (unsigned short)j;
             nr++;
         }
     });
@@ -271,6 +287,7 @@ __device__ __forceinline__ int res_row_verlet(ResCore<T, NP>& L, const ResRows& 
     const double ri = L.r[i];
     auto& row = L.p.b.row;
     const unsigned short* lst = L.p.b.lst;
+    const int at = L.col(i);
     int cnt = 0, nr = 0;
     auto put = [&](int k, int j) {
         if (k < R.cap) R.nbr[(long long)k * R.stride + R.base + i] = (int)(R.base + j);
@@ -282,7 +299,7 @@ __device__ __forceinline__ int res_row_verlet(ResCore<T, NP>& L, const ResRows& 
             if (j == i || !res_listed(xi, xj, rc2, p)) continue;
             put(cnt++, j);
             if (!res_near(xi, xj, ri + L.r[j], delta2, p)) continue;
-            if (nr < RES_LC) row[nr][i] = (unsigned short)j;
+            if (nr < RES_LC) row[nr][at] = (unsigned short)j;
             nr++;
         }
         near = nr;
@@ -295,8 +312,8 @@ __device__ __forceinline__ int res_row_verlet(ResCore<T, NP>& L, const ResRows& 
             if (j == i || !res_listed(xi, L.x[j], rc2, p)) continue;
             if (cnt < RES_LC) {
                 int k = cnt;
-                for (; k > 0 && row[k - 1][i] > j; --k) row[k][i] = row[k - 1][i];
-                row[k][i] = (unsigned short)j;
+                for (; k > 0 && row[k - 1][at] > j; --k) row[k][at] = row[k - 1][at];
+                row[k][at] = (unsigned short)j;
             }
             cnt++;
         }
@@ -304,9 +321,9 @@ __device__ __forceinline__ int res_row_verlet(ResCore<T, NP>& L, const ResRows& 
     if (cnt <= RES_LC) {
 #pragma unroll 1
         for (int k = 0; k < cnt; ++k) {
-            const int j = row[k][i];
+            const int j = row[k][at];
             put(k, j);
-            if (res_near(xi, L.x[j], ri + L.r[j], delta2, p)) row[nr++][i] = (unsigned short)j;
+            if (res_near(xi, L.x[j], ri + L.r[j], delta2, p)) row[nr++][at] = (unsigned short)j;
         }
     } else {
         nr = cnt;  // dense: the forces walk the full rows
@@ -342,10 +359,19 @@ __device__ __forceinline__ int res_load_row(ResCore<T, NP>& L, const ResRows& R,
     for (int k = 0; k < nn; ++k) {
         const int j = (int)(R.nbr[(long long)k * R.stride + R.base + i] - R.base);
         if (!res_near(xi, ref[R.base + j], ri + L.r[j], delta2, p)) continue;
-        if (near < RES_LC) L.p.b.row[near][i] = (unsigned short)j;
+        if (near < RES_LC) L.p.b.row[near][L.col(i)] = (unsigned short)j;
         near++;
     }
     return near;
+}
+
+// RES_WALK: particle i's near row out of b.row, which the thread's next particle takes
+template <int T, int NP>
+__device__ __forceinline__ void res_keep_row(const ResCore<T, NP>& L, const ResKept<T, NP>& K,
+                                             int i, int near) {
+    if constexpr (ResCore<T, NP>::FORM == RES_WALK) {
+        for (int k = 0; k < min(near, RES_LC); ++k) K.row[k * NP + i] = L.p.b.row[k][L.col(i)];
+    }
 }
 
 // The pairs of the near rows (particle numbers in b.row; near[m]: their lengths, 0 without a
@@ -357,9 +383,19 @@ __device__ __forceinline__ void res_pairs(ResCore<T, NP>& L, ResKept<T, NP>& K, 
                                           const int (&near)[ResCore<T, NP>::PPT],
                                           int (&len)[ResCore<T, NP>::PPT]) {
     constexpr int PPT = ResCore<T, NP>::PPT, MP = ResCore<T, NP>::MP;
-    ResBuild<NP>& B = L.p.b;
+    auto& B = L.p.b;
     const int tid = res_tid();
     if (tid == 0) L.dense = fast ? 0 : 1;
+    if constexpr (ResCore<T, NP>::FORM == RES_WALK) {
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < PPT; ++m) {
+            len[m] = min(near[m], RES_LC);
+            if (near[m] > RES_LC) L.dense = 1;
+        }
+        __syncthreads();
+        return;
+    }
     int total = 0, first[PPT];
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
@@ -409,7 +445,7 @@ __device__ __forceinline__ void res_pairs(ResCore<T, NP>& L, ResKept<T, NP>& K, 
             for (int k = len[m]; k < RES_LC; ++k) B.row[k][i] = (unsigned short)MP;
         }
     }
-    if constexpr (ResCore<T, NP>::BIG) {
+    if constexpr (ResCore<T, NP>::FORM == RES_BIG) {
 #pragma unroll
         for (int k = 0; k < ResCore<T, NP>::PAIRS; ++k) {
             const int t = tid + k * T;
@@ -429,10 +465,49 @@ __device__ __forceinline__ double res_flip(double v, unsigned e) {
     return __hiloint2double((int)((unsigned)__double2hiint(v) ^ s), __double2loint(v));
 }
 
+// RES_WALK: the near rows in row order, the wave to its longest row, two entries at a time with
+// the next two loaded ahead (entries past a row's end are any particle and add +0.0).  No
+// barrier: the positions must rest until every thread is through.
+template <bool ENERGY, int T, int NP>
+__device__ __forceinline__ void res_walk(const ResCore<T, NP>& L, const ResKept<T, NP>& K,
+                                         const PairParams& p, int nc,
+                                         const int (&len)[ResCore<T, NP>::PPT],
+                                         double (&ax)[ResCore<T, NP>::PPT],
+                                         double (&ay)[ResCore<T, NP>::PPT],
+                                         double (&e)[ResCore<T, NP>::PPT]) {
+#pragma unroll
+    for (int m = 0; m < ResCore<T, NP>::PPT; ++m) {
+        ax[m] = ay[m] = e[m] = 0.0;
+        const int i = threadIdx.x + m * T, nn = len[m];
+        if (i / WAVE >= nc) continue;  // uniform over the wave
+        const double4 qi = make_double4(L.x[i].x, L.x[i].y, L.r[i], 0.0);
+        auto entry = [&](int k) { return k < nn ? (int)K.row[k * NP + i] : 0; };
+        int j0 = entry(0), j1 = entry(1);
+#pragma unroll 1
+        for (int k = 0; __builtin_amdgcn_ballot_w64(k < nn) != 0; k += 2) {
+            const double4 q0 = make_double4(L.x[j0].x, L.x[j0].y, L.r[j0], 0.0);
+            const double4 q1 = make_double4(L.x[j1].x, L.x[j1].y, L.r[j1], 0.0);
+            j0 = entry(k + 2);
+            j1 = entry(k + 3);
+            double fx, fy;
+            double w = pair_hot<ENERGY>(qi, q0, k < nn, p, fx, fy);
+            ax[m] += fx;
+            ay[m] += fy;
+            if (ENERGY) e[m] += w;
+            if (__builtin_amdgcn_ballot_w64(k + 1 < nn) == 0) break;
+            w = pair_hot<ENERGY>(qi, q1, k + 1 < nn, p, fx, fy);
+            ax[m] += fx;
+            ay[m] += fy;
+            if (ENERGY) e[m] += w;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // Forces (and energies) of the thread's particles: every pair once, then the sums over the rows
 // of len[m] pairs in row order (the wave walks its longest row, four entries at a time; entries
 // past the end are the zero pair).  Every position has been written behind a barrier; no thread
-// reads a position or writes a pair's result after the last barrier in here.
+// reads a position or writes a pair's result after the last barrier in here (RES_WALK: has none).
 template <bool ENERGY, int T, int NP>
 __device__ __forceinline__ void res_forces(ResCore<T, NP>& L, const ResKept<T, NP>& K,
                                            const PairParams& p, int nc,
@@ -442,8 +517,12 @@ __device__ __forceinline__ void res_forces(ResCore<T, NP>& L, const ResKept<T, N
                                            double (&e)[ResCore<T, NP>::PPT]) {
     using C = ResCore<T, NP>;
     constexpr int PPT = C::PPT, MP = C::MP;
+    if constexpr (C::FORM == RES_WALK) {
+        res_walk<ENERGY>(L, K, p, nc, len, ax, ay, e);
+        return;
+    } else {
     const int tid = threadIdx.x, np = L.pairs;
-    double keep[C::BIG ? C::PAIRS : 1];
+    double keep[(C::FORM == RES_BIG) ? C::PAIRS : 1];
     auto pair = [&](int t, unsigned ij) {
         const int i = (int)(ij & 0xffff), j = (int)(ij >> 16);
         const double2 a = L.x[i], b = L.x[j];
@@ -453,7 +532,7 @@ __device__ __forceinline__ void res_forces(ResCore<T, NP>& L, const ResKept<T, N
         L.p.f[t] = make_double2(fx, fy);
         return w;
     };
-    if constexpr (C::BIG) {
+    if constexpr ((C::FORM == RES_BIG)) {
 #pragma unroll
         for (int k = 0; k < C::PAIRS; ++k) {
             const int t = tid + k * T;
@@ -469,11 +548,11 @@ __device__ __forceinline__ void res_forces(ResCore<T, NP>& L, const ResKept<T, N
     }
     if (tid == 0) {
         L.p.f[MP] = make_double2(0.0, 0.0);
-        if (ENERGY && !C::BIG) L.p.e[MP] = 0.0;
+        if (ENERGY && !(C::FORM == RES_BIG)) L.p.e[MP] = 0.0;
     }
     __syncthreads();
     auto entry = [&](int k, int i) -> unsigned {
-        if constexpr (C::BIG) return K.row[k * NP + i];
+        if constexpr ((C::FORM == RES_BIG)) return K.row[k * NP + i];
         else return L.p.b.row[k][i];
     };
 #pragma unroll
@@ -491,17 +570,17 @@ __device__ __forceinline__ void res_forces(ResCore<T, NP>& L, const ResKept<T, N
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 f[t] = L.p.f[s[t] & (RES_FLIP - 1)];
-                if (ENERGY && !C::BIG) w[t] = L.p.e[s[t] & (RES_FLIP - 1)];
+                if (ENERGY && !(C::FORM == RES_BIG)) w[t] = L.p.e[s[t] & (RES_FLIP - 1)];
             }
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 ax[m] += res_flip(f[t].x, s[t]);
                 ay[m] += res_flip(f[t].y, s[t]);
-                if (ENERGY && !C::BIG) e[m] += w[t];
+                if (ENERGY && !(C::FORM == RES_BIG)) e[m] += w[t];
             }
         }
     }
-    if constexpr (ENERGY && C::BIG) {
+    if constexpr (ENERGY && (C::FORM == RES_BIG)) {
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < C::PAIRS; ++k)
@@ -520,6 +599,7 @@ __device__ __forceinline__ void res_forces(ResCore<T, NP>& L, const ResKept<T, N
                 for (int t = 0; t < 4; ++t) e[m] += L.p.e[s[t] & (RES_FLIP - 1)];
             }
         }
+    }
     }
 }
 
