@@ -35,9 +35,10 @@
 //               controller (for a rigid particle with its vertices), zero velocities
 //               (minimizeFire prologue); then the FIRE move of systems inside a
 //               minimisation (Fire::step first half) and its displacement flags
-//   k_b_build   per (system, 256-slot tile): O(n^2) row build through LDS tiles, for the
-//               systems whose Verlet test (3 max d^2 > thr^2, b_rebuild_now) asks for it
-//   k_b_build_cells  systems of 128+ particles: the same rows from a cell grid in LDS
+//   k_b_build_cells  the Verlet rows of the systems whose test (3 max d^2 > thr^2,
+//               b_rebuild_now) asks for them, from a cell grid in LDS
+//   k_b_build   the same by an O(n^2) pass for systems of more than 16,384 particles
+//               (launched when the arena holds one)
 //   k_b_force   forces (+ closing kick) and the chunk partials of P, PE, max F^2
 //   k_b_ctl     per system: minimizeFire's stop test and Fire::step's decision; clears
 //               the controller's applied requests and counts the step
@@ -377,19 +378,23 @@ __device__ __forceinline__ bool b_rebuild_now(const BDev& b, const BSys& S) {
     return __builtin_amdgcn_ballot_w64(far) != 0;
 }
 
-// Systems of BC_MIN_N particles and more get their rows from a cell grid instead of the
-// all-pairs scan (one work item per BC_PER particles, listed in ctiles; the workgroup
-// holding an item bins the whole system into its LDS and builds the rows of every
-// parts-th block of 1024 particles).  Cells are at least rc (1 + 1e-9) wide,
-// so every particle within rc of i lies in the 3 x 3 cells around i's, and the rows
-// hold the same indices in the same ascending order as the all-pairs scan.
+// Rows of systems of up to BC_MAX_N particles: one work item per BC_PER particles, listed in
+// ctiles; the workgroup holding an item bins the whole system into its LDS and builds the rows of
+// its part, 16 lanes a particle.  Cells are at least rc (1 + 1e-9) wide, so every particle within
+// rc of i lies in the 3 x 3 cells around i's; systems under BC_MIN_N particles and boxes under
+// three cells a side take every particle as a candidate.  The lanes test candidates side by side
+// and rank the hits by index, so the rows hold the same indices in the same ascending order as
+// the all-pairs scan.
 constexpr int BC_MIN_N = 128;      // systems from this size up use the cell grid
 constexpr int BC_MAX_N = 16384;    // particles per system the LDS lists hold
 constexpr int BC_MAX_D = 96;       // cells per side at most
 constexpr int BC_CELLS = BC_MAX_D * BC_MAX_D;
 constexpr int BC_BLOCK = 1024;
-constexpr int BC_PER = 2048;       // particles per workgroup (each bins the whole system
-                                   // itself, then builds the rows of its part)
+constexpr int BC_GROUP = 16;       // lanes per particle
+constexpr int BC_PER = 256;        // particles per workgroup (four rounds; each workgroup bins
+                                   // the whole system itself).  With 2,048, 48 systems of up to
+                                   // 1,024 particles kept 48 workgroups busy.
+constexpr int BC_HITS = 32;        // entries of a row (the arena's capacity)
 
 struct BCGrid {
     int nx, ny;
@@ -417,118 +422,107 @@ __device__ __forceinline__ int bc_coord(double x, double L, double cs, int n) {
 // One work item (system, part): every early return is uniform over the workgroup.
 // cend: counts, then (after the fill) each cell's end; lst: the system's particles
 // (system-local) grouped by cell.
-__device__ __forceinline__ void bc_build_item(const BDev& b, int2 ct, int* cend, int* lst,
-                                              int* wsum) {
+struct BCLds {
+    int cend[BC_CELLS];
+    unsigned short lst[BC_MAX_N];
+    int wsum[BC_BLOCK / WAVE];
+    unsigned short hit[BC_BLOCK / BC_GROUP][BC_HITS];
+};
+
+__device__ __forceinline__ void bc_build_item(const BDev& b, int2 ct, BCLds& L) {
     const BSys& S = b.sys[ct.x];
     if (!b_rebuild_now(b, S)) return;  // the same verdict in every wave of the workgroup
     BCGrid g;
-    if (!bc_grid(b, S, g)) return;
-    const int part = ct.y, parts = (S.n + BC_PER - 1) / BC_PER;
-    const int tid = threadIdx.x, n = S.n, ncell = g.nx * g.ny;
+    const bool grid = bc_grid(b, S, g);
+    const int tid = threadIdx.x, n = S.n;
     const long long off = S.off;
-    for (int c = tid; c < ncell; c += BC_BLOCK) cend[c] = 0;
-    __syncthreads();
-    for (int i = tid; i < n; i += BC_BLOCK) {
-        double4 q = b.P[off + i];
-        int c = bc_coord(q.x, S.Lx, g.csx, g.nx) + g.nx * bc_coord(q.y, S.Ly, g.csy, g.ny);
-        atomicAdd(&cend[c], 1);
-    }
-    __syncthreads();
-    // exclusive scan of the counts: each thread owns a run of consecutive cells
-    const int per = (ncell + BC_BLOCK - 1) / BC_BLOCK;
-    const int c0 = min(tid * per, ncell), c1 = min(c0 + per, ncell);
-    int local = 0;
-    for (int c = c0; c < c1; ++c) local += cend[c];
     const int lane = tid % WAVE, wv = tid / WAVE;
-    int incl = local;
+    auto cell = [&](double4 q) {
+        return bc_coord(q.x, S.Lx, g.csx, g.nx) + g.nx * bc_coord(q.y, S.Ly, g.csy, g.ny);
+    };
+    if (grid) {
+        const int ncell = g.nx * g.ny;
+        for (int c = tid; c < ncell; c += BC_BLOCK) L.cend[c] = 0;
+        __syncthreads();
+        for (int i = tid; i < n; i += BC_BLOCK) atomicAdd(&L.cend[cell(b.P[off + i])], 1);
+        __syncthreads();
+        // exclusive scan of the counts: each thread owns a run of consecutive cells
+        const int per = (ncell + BC_BLOCK - 1) / BC_BLOCK;
+        const int c0 = min(tid * per, ncell), c1 = min(c0 + per, ncell);
+        int local = 0;
+        for (int c = c0; c < c1; ++c) local += L.cend[c];
+        int incl = local;
 #pragma unroll
-    for (int d = 1; d < WAVE; d <<= 1) {
-        int o = __shfl_up(incl, d, WAVE);
-        if (lane >= d) incl += o;
-    }
-    if (lane == WAVE - 1) wsum[wv] = incl;
-    __syncthreads();
-    int before = 0;
-    for (int w = 0; w < wv; ++w) before += wsum[w];
-    int run = before + incl - local;
-    for (int c = c0; c < c1; ++c) {
-        int t = cend[c];
-        cend[c] = run;
-        run += t;
-    }
-    __syncthreads();
-    for (int i = tid; i < n; i += BC_BLOCK) {
-        double4 q = b.P[off + i];
-        int c = bc_coord(q.x, S.Lx, g.csx, g.nx) + g.nx * bc_coord(q.y, S.Ly, g.csy, g.ny);
-        lst[atomicAdd(&cend[c], 1)] = i;
-    }
-    __syncthreads();
-    // each cell's members in ascending order (a few per cell)
-    for (int c = tid; c < ncell; c += BC_BLOCK) {
-        const int a = c == 0 ? 0 : cend[c - 1], e = cend[c];
-        for (int u = a + 1; u < e; ++u) {
-            int v = lst[u], k = u - 1;
-            while (k >= a && lst[k] > v) {
-                lst[k + 1] = lst[k];
-                --k;
-            }
-            lst[k + 1] = v;
+        for (int d = 1; d < WAVE; d <<= 1) {
+            int o = __shfl_up(incl, d, WAVE);
+            if (lane >= d) incl += o;
         }
+        if (lane == WAVE - 1) L.wsum[wv] = incl;
+        __syncthreads();
+        int run = incl - local;
+        for (int w = 0; w < wv; ++w) run += L.wsum[w];
+        for (int c = c0; c < c1; ++c) {
+            int t = L.cend[c];
+            L.cend[c] = run;
+            run += t;
+        }
+        __syncthreads();
+        for (int i = tid; i < n; i += BC_BLOCK)
+            L.lst[atomicAdd(&L.cend[cell(b.P[off + i])], 1)] = (unsigned short)i;
+        __syncthreads();
     }
-    __syncthreads();
     const PairParams p = bparams(b, S);
-    constexpr int NONE = 0x7fffffff;
+    const double rc2 = S.rc2;
+    const int sub = tid % BC_GROUP, k = tid / BC_GROUP, shift = lane - sub;
+    const int end = min(n, (ct.y + 1) * BC_PER);
     int mx = 0;
-    for (int il = part * BC_BLOCK + tid; il < n; il += parts * BC_BLOCK) {
-        const long long i = off + il;
-        const double4 qi = b.P[i];
-        const int cx = bc_coord(qi.x, S.Lx, g.csx, g.nx), cy = bc_coord(qi.y, S.Ly, g.csy, g.ny);
-        // the nine cells' ranges, merged in ascending particle order
-        int pa[9], pe[9], h[9];
-#pragma unroll
-        for (int t = 0; t < 9; ++t) {
-            int x = cx + t % 3 - 1, y = cy + t / 3 - 1;
-            x = x < 0 ? x + g.nx : (x >= g.nx ? x - g.nx : x);
-            y = y < 0 ? y + g.ny : (y >= g.ny ? y - g.ny : y);
-            const int c = x + g.nx * y;
-            pa[t] = c == 0 ? 0 : cend[c - 1];
-            pe[t] = cend[c];
-            h[t] = pa[t] < pe[t] ? lst[pa[t]] : NONE;
-        }
+    for (int il = ct.y * BC_PER + k; il - k < end; il += BC_BLOCK / BC_GROUP) {
+        const bool live = il < end;
+        const double4 qi = b.P[off + (live ? il : 0)];
+        CellRuns runs;
+        runs.count = live ? n : 0;
+        if (grid)
+            runs.set(bc_coord(qi.x, S.Lx, g.csx, g.nx), bc_coord(qi.y, S.Ly, g.csy, g.ny), g.nx,
+                     g.ny, live, [&](int c0, int c1, int& a, int& e) {
+                         a = c0 == 0 ? 0 : L.cend[c0 - 1];
+                         e = L.cend[c1];
+                     });
         int cnt = 0;
-        while (true) {
-            int best = h[0], bt = 0;
-#pragma unroll
-            for (int t = 1; t < 9; ++t)
-                if (h[t] < best) {
-                    best = h[t];
-                    bt = t;
+        for (int t = sub; __builtin_amdgcn_ballot_w64(t < runs.count) != 0; t += BC_GROUP) {
+            int j = 0;
+            bool hit = false;
+            if (t < runs.count) {
+                j = grid ? (int)L.lst[runs.entry(t)] : t;
+                const double4 qj = b.P[off + j];
+                double dx, dy;
+                if (p.fast) {
+                    dx = pbc_rint(qi.x, qj.x, p.Lx, p.invLx);
+                    dy = pbc_rint(qi.y, qj.y, p.Ly, p.invLy);
+                } else {
+                    dx = pbc(qi.x, qj.x, p.Lx, p.invLx, p.halfLx, 0);
+                    dy = pbc(qi.y, qj.y, p.Ly, p.invLy, p.halfLy, 0);
                 }
-            if (best == NONE) break;
-#pragma unroll
-            for (int t = 0; t < 9; ++t)
-                if (t == bt) {
-                    pa[t]++;
-                    h[t] = pa[t] < pe[t] ? lst[pa[t]] : NONE;
-                }
-            if (best == il) continue;
-            const long long j = off + best;
-            const double4 qj = b.P[j];
-            double dx, dy;
-            if (p.fast) {
-                dx = pbc_rint(qi.x, qj.x, p.Lx, p.invLx);
-                dy = pbc_rint(qi.y, qj.y, p.Ly, p.invLy);
-            } else {
-                dx = pbc(qi.x, qj.x, p.Lx, p.invLx, p.halfLx, 0);
-                dy = pbc(qi.y, qj.y, p.Ly, p.invLy, p.halfLy, 0);
+                hit = j != il && dx * dx + dy * dy < rc2;
             }
-            if (dx * dx + dy * dy < S.rc2) {
-                if (cnt < b.cap) b.nbr[(long long)cnt * b.nslot + i] = (int)j;
-                cnt++;
-            }
+            const unsigned mask = (unsigned)(__builtin_amdgcn_ballot_w64(hit) >> shift) &
+                                  ((1u << BC_GROUP) - 1);
+            const int pos = cnt + __popc(mask & ((1u << sub) - 1));
+            if (hit && pos < BC_HITS) L.hit[k][pos] = (unsigned short)j;
+            cnt += __popc(mask);
         }
-        b.nnum[i] = cnt;
-        b.lref[i] = make_double2(qi.x, qi.y);
+        wave_sync();
+        // (a row of more entries than that ends the run: flags[0])
+        for (int h = sub; h < min(cnt, BC_HITS); h += BC_GROUP) {
+            const int j = L.hit[k][h];
+            int rank = 0;
+            for (int v = 0; v < min(cnt, BC_HITS); ++v) rank += L.hit[k][v] < j ? 1 : 0;
+            if (rank < b.cap) b.nbr[(long long)rank * b.nslot + off + il] = (int)(off + j);
+        }
+        wave_sync();  // the next round's hits take this one's place
+        if (live && sub == 0) {
+            b.nnum[off + il] = cnt;
+            b.lref[off + il] = make_double2(qi.x, qi.y);
+        }
         mx = max(mx, cnt);
     }
     mx = wave_max_i(mx);
@@ -542,26 +536,23 @@ __device__ __forceinline__ void bc_build_item(const BDev& b, int2 ct, int* cend,
 // the graph-baked launch stays small whatever the list's capacity.
 constexpr int BC_GRID = 512;
 __global__ __launch_bounds__(BC_BLOCK) void k_b_build_cells(BDev b) {
-    __shared__ int cend[BC_CELLS];
-    __shared__ int lst[BC_MAX_N];
-    __shared__ int wsum[BC_BLOCK / WAVE];
+    __shared__ BCLds L;
     const int count = b.flags[5];
     for (int w = blockIdx.x; w < count; w += gridDim.x) {
-        bc_build_item(b, b.ctiles[w], cend, lst, wsum);
+        bc_build_item(b, b.ctiles[w], L);
         __syncthreads();  // the next item reuses the LDS
     }
 }
 
-// kernelUpdateNeighborList (base/kernels.cu:256-293) for the systems that need it:
-// every other particle of the system with d^2 < rc^2, ascending index.  One block per
+// kernelUpdateNeighborList (base/kernels.cu:256-293) for the systems of more than BC_MAX_N
+// particles that need it (launched when there is one): every other particle of the system with d^2 < rc^2, ascending index.  One block per
 // 256-slot tile of a system; the system's positions pass through LDS.
 __global__ __launch_bounds__(BLOCK) void k_b_build(BDev b) {
     if ((int)blockIdx.x >= b.flags[4]) return;
     const int2 t = b.tiles[blockIdx.x];
     const BSys& S = b.sys[t.x];
+    if (S.n <= BC_MAX_N) return;   // k_b_build_cells builds this system
     if (!b_rebuild_now(b, S)) return;  // the same verdict in every wave of the block
-    BCGrid g;
-    if (bc_grid(b, S, g)) return;  // k_b_build_cells builds this system
     __shared__ double2 tp[BLOCK];
     const long long i = (long long)t.y + threadIdx.x;
     const long long end = S.off + S.n;
@@ -1440,6 +1431,7 @@ __global__ __launch_bounds__(WAVE) void k_b_jam(BDev b) {
 struct dpm_batch {
     int64_t nsys = 0, nslot = 0, ntiles = 0;
     int nct = 0;  // cell-grid build workgroups of a batch (ctiles entries)
+    bool large = false;  // some system has more than BC_MAX_N particles (k_b_build is launched)
     int device = 0;
     hipStream_t stream = nullptr;
     dpm::BDev d{};
@@ -1490,11 +1482,10 @@ struct dpm_batch {
 
 namespace dpm {
 
-// The cell-grid build workgroups of a system: one per BC_PER particles when the system
-// is in the cell-grid size range (k_b_build_cells re-checks the grid for the box of the
-// step and leaves small boxes to k_b_build).
+// The row build's work items of a system: one per BC_PER particles (k_b_build_cells); larger
+// systems are k_b_build's.
 static void cell_tiles(std::vector<int2>& out, int s, int n) {
-    if (n < BC_MIN_N || n > BC_MAX_N) return;
+    if (n > BC_MAX_N) return;
     for (int part = 0; part < (n + BC_PER - 1) / BC_PER; ++part) out.push_back(make_int2(s, part));
 }
 
@@ -1536,9 +1527,9 @@ static int batch_alloc(dpm_batch* b, int64_t nsys, int64_t nslot, int64_t tiles_
     d.nsys = nsys;
     d.nslot = nslot;
     d.ntiles = tiles_cap;
-    // parts = ceil(n / BC_PER) <= n / BC_PER + n / BC_MIN_N for n >= BC_MIN_N, and the
-    // systems share the nslot slots
-    d.nctiles = nslot / BC_PER + nslot / BC_MIN_N + 1;
+    // parts = ceil(n / BC_PER) <= n / BC_PER + 1, and the systems share the nslot slots, at least
+    // WAVE each
+    d.nctiles = nslot / BC_PER + nslot / WAVE + 1;
     d.cap = 32;  // at most 32: k_rb_vbuild holds a row entry per half-wave lane (and
                  // rb_eval marks row positions in a 64-bit mask)
     DPM_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
@@ -1688,7 +1679,7 @@ static void enqueue_batch_step(dpm_batch* b) {
     dim3 vslots((unsigned)((b->nvslot + BLOCK - 1) / BLOCK));
     hipLaunchKernelGGL(k_b_prep_move, slots, dim3(BLOCK), 0, st, d);
     if (rigid) hipLaunchKernelGGL(k_rb_vmove, vslots, dim3(BLOCK), 0, st, d);
-    hipLaunchKernelGGL(k_b_build, dim3((unsigned)b->ntiles), dim3(BLOCK), 0, st, d);
+    if (b->large) hipLaunchKernelGGL(k_b_build, dim3((unsigned)b->ntiles), dim3(BLOCK), 0, st, d);
     hipLaunchKernelGGL(k_b_build_cells, dim3((unsigned)std::min<long long>(d.nctiles, BC_GRID)),
                        dim3(BC_BLOCK), 0, st, d);
     if (rigid)
@@ -1944,7 +1935,10 @@ static dpm_batch* batch_create(int64_t n_systems, const int64_t* n_particles,
                                          hipMemcpyHostToDevice, b->stream)) == hipSuccess;
         }
         std::vector<int2> ct;
-        for (int64_t s = 0; s < n_systems; ++s) cell_tiles(ct, (int)s, b->n[s]);
+        for (int64_t s = 0; s < n_systems; ++s) {
+            cell_tiles(ct, (int)s, b->n[s]);
+            b->large = b->large || b->n[s] > BC_MAX_N;
+        }
         b->nct = (int)ct.size();
         ok = ok && (long long)ct.size() <= d.nctiles;  // always holds (bound of batch_alloc)
         if (ok && b->nct)
@@ -2633,12 +2627,18 @@ static int serve_upload_tiles(dpm_server* sv) {
     std::vector<int2> ct;
     std::vector<std::pair<int, int64_t>> resident;
     b->phased = false;
+    bool large = false;
     for (size_t s = 0; s < sv->sys_req.size(); ++s) {
         if (!sv->sys_req[s]) continue;
         const dpm_server_req& q = sv->reqs.at(sv->sys_req[s]);
         cell_tiles(ct, (int)s, (int)q.n);
+        large = large || q.n > BC_MAX_N;
         if (resident_size(b, q.n, q.kind == DPM_BUMPY, true)) resident.push_back({(int)s, q.n});
         else b->phased = true;
+    }
+    if (large != b->large) {  // the step's launches change
+        drop_graph(b);
+        b->large = large;
     }
     if (resident_table(b, resident)) return -1;
     // the bound of batch_alloc: ct never exceeds d.nctiles entries

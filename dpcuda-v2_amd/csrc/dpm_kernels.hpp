@@ -162,6 +162,49 @@ __device__ __forceinline__ int cell_coord(double pos, double cs, int n) {
     return (int)(idx >= 0 ? idx % n : (idx % n + n) % n);
 }
 
+// The candidates of a particle in cell (cx, cy) of a grid of nx x ny >= 3 x 3 cells, for lanes
+// that test them side by side: the list entries of the 3 x 3 cells around it, which are one run
+// in each row of cells, or two where the row wraps.  range(c0, c1, a, e) gives the entries
+// [a, e) of cells c0 to c1.
+struct CellRuns {
+    int a[6], m[6], count;
+    template <class Range>
+    __device__ __forceinline__ void set(int cx, int cy, int nx, int ny, bool live, Range range) {
+        count = 0;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const int y = cy + r - 1 < 0 ? ny - 1 : (cy + r - 1 >= ny ? 0 : cy + r - 1);
+            const int c = y * nx;
+            int e;
+            range(c + max(cx - 1, 0), c + min(cx + 1, nx - 1), a[2 * r], e);
+            m[2 * r] = live ? e - a[2 * r] : 0;
+            a[2 * r + 1] = 0;
+            m[2 * r + 1] = 0;
+            if (cx == 0 || cx == nx - 1) {
+                const int w = c + (cx == 0 ? nx - 1 : 0);
+                range(w, w, a[2 * r + 1], e);
+                m[2 * r + 1] = live ? e - a[2 * r + 1] : 0;
+            }
+            count += m[2 * r] + m[2 * r + 1];
+        }
+    }
+    __device__ __forceinline__ int entry(int t) const {  // the list entry of candidate t
+        int u = a[0] + t, base = m[0];
+#pragma unroll
+        for (int r = 1; r < 6; ++r) {
+            if (t >= base) u = a[r] + (t - base);
+            base += m[r];
+        }
+        return u;
+    }
+};
+
+// LDS writes of the wave's lanes before its lanes' later reads
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Fire::step's decision for the next iteration (src/integrator/fire.cu:14-33);
 // RigidBumpy::getPowerFire adds sum(tau*w) (rigid_bumpy.cu:1181-1191; null for disks).  True
 // when the loop has ended.

@@ -173,12 +173,6 @@ __device__ __forceinline__ void na_lds_grid(NaGridLds& G, NaForces& L, const dou
     __syncthreads();
 }
 
-// LDS writes of the wave's lanes before its lanes' later reads
-__device__ __forceinline__ void na_wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // The total of nc partials in wave_final_sum's order (lane t adds partials t, t + 64, ...): all
 // threads bring a stretch of them to LDS, one wave adds it.
 constexpr int NA_STRETCH = 4096;
@@ -246,36 +240,13 @@ __global__ __launch_bounds__(NA_T) void k_na_forces(const double* x, const doubl
             b = start[c1 + 1];
         }
     };
-    int a[6], m[6];
-    {
-        const int cid = na_cell(q.x, q.y, g);
-        const int cx = cid % g.ncx, cy = cid / g.ncx;
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            const int yy = cy + r - 1 < 0 ? g.ncy - 1 : (cy + r - 1 >= g.ncy ? 0 : cy + r - 1);
-            const int c = yy * g.ncx;
-            int e;
-            range(c + max(cx - 1, 0), c + min(cx + 1, g.ncx - 1), a[2 * r], e);
-            m[2 * r] = live ? e - a[2 * r] : 0;
-            a[2 * r + 1] = 0;
-            m[2 * r + 1] = 0;
-            if (cx == 0 || cx == g.ncx - 1) {
-                const int w = c + (cx == 0 ? g.ncx - 1 : 0);
-                range(w, w, a[2 * r + 1], e);
-                m[2 * r + 1] = live ? e - a[2 * r + 1] : 0;
-            }
-        }
-    }
-    const int cand = m[0] + m[1] + m[2] + m[3] + m[4] + m[5];
+    const int cid = na_cell(q.x, q.y, g);
+    CellRuns runs;
+    runs.set(cid % g.ncx, cid / g.ncx, g.ncx, g.ncy, live, range);
+    const int cand = runs.count;
     auto candidate = [&](int t) {  // the place of candidate t
-        int u = a[0] + t, base = m[0];
-#pragma unroll
-        for (int r = 1; r < 6; ++r) {
-            if (t >= base) u = a[r] + (t - base);
-            base += m[r];
-        }
-        if constexpr (LDS) return (int)G.lst[u];
-        else return u;
+        if constexpr (LDS) return (int)G.lst[runs.entry(t)];
+        else return runs.entry(t);
     };
     auto listed = [&](const double4& o) {
         const double dx = pbc(q.x, o.x, p.Lx, p.invLx, p.halfLx, 1);
@@ -302,7 +273,7 @@ __global__ __launch_bounds__(NA_T) void k_na_forces(const double* x, const doubl
         }
         cnt += __popc(mask);
     }
-    na_wave_sync();
+    wave_sync();
     auto pair = [&](int u, double& px, double& py) {
         const double4 o = load(u);
         const double rs = q.z + o.z;
@@ -321,7 +292,7 @@ __global__ __launch_bounds__(NA_T) void k_na_forces(const double* x, const doubl
             L.f[k][rank] = make_double2(px, py);
             L.e[k][rank] = e;
         }
-        na_wave_sync();
+        wave_sync();
         if (sub < 3) {
             for (int v = 0; v < cnt; ++v)
                 acc += sub == 0 ? L.f[k][v].x : (sub == 1 ? L.f[k][v].y : L.e[k][v]);
