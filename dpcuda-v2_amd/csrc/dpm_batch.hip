@@ -702,7 +702,9 @@ __global__ __launch_bounds__(BLOCK) void k_rb_vbuild(BDev b) {
     if (S.kind != BK_RIGID || !b_rebuild_now(b, S)) return;
     const PairParams pp = bparams(b, S);
     const double vc = sqrt(S.vc2);
-    const bool shift = fmin(pp.halfLx, pp.halfLy) > vertex_shift_limit(S.rmax, S.rv, vc);
+    const bool shift = fmin(pp.halfLx, pp.halfLy) > ring_shift_limit(S.rmax, S.rv, vc);
+    __shared__ RingEntry rings[BLOCK / RB_HALF][RB_HALF];
+    RingEntry* ring = rings[threadIdx.x / RB_HALF];
     const int hs = (int)(threadIdx.x % WAVE) / RB_HALF * RB_HALF;  // the half's first lane
     const bool live = i - S.off < S.n;  // uniform over the half-wave
     const int st = live ? b.vst[i] : 0, nv = live ? b.nvt[i] : 0;
@@ -713,12 +715,15 @@ __global__ __launch_bounds__(BLOCK) void k_rb_vbuild(BDev b) {
         const bool has = a0 + lane < nv;
         const long long v = st + a0 + lane;
         const double2 xv = has ? b.vpos[v] : make_double2(0.0, 0.0);
-        const int cnt = vertex_row(
-            pp, b.P, b.vst, b.nvt, b.vpos, S.rv, vc, S.vc2, S.vp2, shift, lane, hs, has, xv, cp,
-            nn, [&](int k) { return b.nbr[(long long)k * b.nslot + i]; },
-            [&](int pos, int u) {
-                if (pos < b.vcap) b.vnbr[(long long)pos * b.nvslot + v] = u;
-            });
+        auto entry = [&](int k) { return b.nbr[(long long)k * b.nslot + i]; };
+        auto emit = [&](int pos, int u) {
+            if (pos < b.vcap) b.vnbr[(long long)pos * b.nvslot + v] = u;
+        };
+        const int cnt =
+            shift ? vertex_row<true>(pp, b.P, b.vst, b.nvt, b.vpos, S.rv, vc, S.vc2, S.vp2, lane,
+                                     hs, has, xv, cp, nn, ring, entry, emit)
+                  : vertex_row<false>(pp, b.P, b.vst, b.nvt, b.vpos, S.rv, vc, S.vc2, S.vp2, lane,
+                                      hs, has, xv, cp, nn, ring, entry, emit);
         if (has) {
             b.vnum[v] = cnt;
             mx = max(mx, cnt);

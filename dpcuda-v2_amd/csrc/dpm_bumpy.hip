@@ -292,7 +292,9 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb
                                                              double rmax, int gated) {
     if (gated && d.ctl->kind < 1) return;
     const double vc = sqrt(nb.vc2);
-    const bool shift = fmin(nb.halfLx, nb.halfLy) > vertex_shift_limit(rmax, rv, vc);
+    const bool shift = fmin(nb.halfLx, nb.halfLy) > ring_shift_limit(rmax, rv, vc);
+    __shared__ RingEntry rings[BLOCK / VB_HALF][VB_HALF];
+    RingEntry* ring = rings[threadIdx.x / VB_HALF];
     const int lane = (int)(threadIdx.x % VB_HALF);
     const int hs = (int)(threadIdx.x % WAVE) / VB_HALF * VB_HALF;
     const int64_t halves = (int64_t)gridDim.x * (BLOCK / VB_HALF);
@@ -309,12 +311,15 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb
             const bool has = a0 + lane < nv;
             const int64_t v = st + a0 + lane;
             const double2 xv = has ? d.vpos[v] : make_double2(0.0, 0.0);
-            const int cnt = vertex_row(
-                nb, d.P0, d.vstart, d.nverts, d.vpos, rv, vc, nb.vc2, nb.vp2, shift, lane, hs,
-                has, xv, cp, nn, [&](int k) { return d.nbr[(int64_t)k * d.N + p]; },
-                [&](int pos, int u) {
-                    if (pos < d.vcap) d.vnbr[(int64_t)pos * d.Nv + v] = u;
-                });
+            auto entry = [&](int k) { return d.nbr[(int64_t)k * d.N + p]; };
+            auto emit = [&](int pos, int u) {
+                if (pos < d.vcap) d.vnbr[(int64_t)pos * d.Nv + v] = u;
+            };
+            const int cnt =
+                shift ? vertex_row<true>(nb, d.P0, d.vstart, d.nverts, d.vpos, rv, vc, nb.vc2,
+                                         nb.vp2, lane, hs, has, xv, cp, nn, ring, entry, emit)
+                      : vertex_row<false>(nb, d.P0, d.vstart, d.nverts, d.vpos, rv, vc, nb.vc2,
+                                          nb.vp2, lane, hs, has, xv, cp, nn, ring, entry, emit);
             if (has) {
                 d.vnum[v] = cnt;
                 mx = max(mx, cnt);

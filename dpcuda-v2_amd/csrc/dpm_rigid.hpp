@@ -2,7 +2,7 @@
 // single-system rigid bumpy kernels (dpm_bumpy.hip) and the batched engine
 // (dpm_batch.hip), so that a rigid system carries the same bits on either path.
 #pragma once
-#include "dpm_device.hpp"
+#include "dpm_kernels.hpp"
 #include "dpm_trig.hpp"
 
 namespace dpm {
@@ -96,113 +96,145 @@ __device__ __host__ inline double vertex_shift_limit(double rmax, double rv, dou
     return (2.0 * rmax - 2.0 * rv + vc) * (1.0 + 1e-6);
 }
 
-// Which vertices of ring q (nq of them, radius R, evenly spaced counterclockwise from vertex 0
-// at r0 from the centre) can lie within vc of a point at (dx, dy) from q's centre: at most
-// asin(vc / R) away from the point's direction, wherever the point is.  The candidates in
-// ascending order are c < wrapped ? c : first + c - wrapped for c in [0, count).  Single
-// precision decides only the window, which is 0.02 of a spacing wider than it has to be on
-// either side (asin(x) < x + x^3/4 up to x = 0.6; the rounding of atan2f, the spacing's
-// tolerance of 1e-6 and the rotations' rounding stay far below that).
-struct RingWindow {
-    int first, count, wrapped;
-};
-__device__ __forceinline__ RingWindow ring_window(double dx, double dy, double2 r0, double R,
-                                                  double vc, int nq) {
-    const float x = (float)vc / (float)R;
-    const float per = (float)nq * 0.15915494f;  // spacings per radian
-    const float half = x < 0.6f ? (x + 0.25f * x * x * x) * per + 0.02f : 1e9f;
-    if (!(2.0f * half + 2.0f < (float)nq)) return {0, nq, 0};
-    const float t = per * atan2f((float)(r0.x * dy - r0.y * dx), (float)(r0.x * dx + r0.y * dy));
-    const int lo = (int)ceilf(t - half), hi = (int)floorf(t + half);
-    const int first = lo < 0 ? lo + nq : lo;
-    return {first, hi - lo + 1, max(0, first + (hi - lo + 1) - nq)};
+// The same for the image of two centres whose rings can reach each other (their distance is at
+// most two ring radii and vc) to serve every vertex of the first.
+__device__ __host__ inline double ring_shift_limit(double rmax, double rv, double vc) {
+    return (3.0 * rmax - 3.0 * rv + vc) * (1.0 + 1e-6);
 }
+
+// atan2(y, x) to 1.2e-5 (an odd polynomial on [0, 1], fitted to the least largest error)
+__device__ __forceinline__ float atan2_coarse(float y, float x) {
+    const float ax = fabsf(x), ay = fabsf(y), hi = fmaxf(ax, ay), lo = fminf(ax, ay);
+    const float t = hi > 0.0f ? lo * __builtin_amdgcn_rcpf(hi) : 0.0f, q = t * t;
+    float r = t * (0.99986631f + q * (-0.33030444f + q * (0.18015778f +
+                  q * (-0.08515398f + q * 0.0208439f))));
+    r = ay > ax ? 1.57079633f - r : r;
+    r = x < 0.0f ? 3.14159265f - r : r;
+    return y < 0.0f ? -r : r;
+}
+
+// A neighbouring particle q of a particle row, as the vertex rows need it: centre, the shift
+// L k of the minimum image of v - x_q, the squared distance below which a vertex looks at its
+// ring (min of the vertex-particle cutoff's square and vertex_ring_near's bound), vertex 0 from
+// the centre, and the window's half width.
+//
+// The window: which vertices of ring q (n of them, radius R, evenly spaced counterclockwise from
+// vertex 0) can lie within vc of a point in the direction (dx, dy) from q's centre: at most
+// asin(vc / R) away from that direction, wherever the point is.  Single precision decides only
+// the window, which is 0.02 of a spacing and the angle's error wider than it has to be on
+// either side (asin(x) < x + x^3/4 up to x = 0.6; the spacing's tolerance of 1e-6 and the
+// rotations' rounding stay far below that).
+struct RingEntry {
+    double cx, cy, sx, sy, lim;
+    float x0, y0;    // vertex 0 from the centre
+    float per, half; // spacings per radian; the window's half width in spacings (-1: all)
+    int first, n;    // vertex range
+};
 
 // The vertex rows of one particle (kernelUpdateVertexNeighborList, rigid_bumpy/kernels.cu:
 // 870-922: for vertex v, over the particle row in order, the particles q whose centre lies
 // within vp of v, then q's vertices in order within vc of v), for evenly spaced rings: a
 // half-wave per particle, lane a0 + lane its vertex xv; the return value is the lane's row
-// length, emit(pos, u) stores entry pos.
-//   1. each lane loads one row entry (q's record, vertex range and first vertex) and drops the
-//      q that no vertex of the particle can reach;
-//   2. every lane tests the remaining centres (vp and vertex_ring_near) into a bit mask;
+// length, emit(pos, u) stores entry pos.  R: 32 entries of LDS of the half-wave's own.
+//   1. each lane loads one row entry and puts it into R if some vertex of the particle can
+//      reach it (in row order);
+//   2. every lane tests the entries (vp and vertex_ring_near) into a bit mask;
 //   3. every lane walks its own mask and tests the window of q's vertices (3 or 4 of 20 to 28)
-//      that can be within vc.
-// A vertex passes the gate of one or two of its particle's neighbours, so the wave takes two
-// or three rounds of step 3.  Before, a gated vertex was tested against all of q's vertices by
-// the 32 lanes, one after another (some 36 rounds a particle, nine cross-lane reads each).
-template <class Box, class Entry, class Emit>
+//      that can be within vc, four loads at a time.
+// SHIFT: the minimum image of x_p - x_q serves every vertex of both rings (ring_shift_limit):
+// pbc(v, u) = (v - u) - L k with one k, the same bits.  It is formed once per row entry; a lane
+// that formed it for every vertex and entry spent most of its instructions on it.
+// What bounds it: the vector pipe (some 450 instructions a wave; the entries' fields came by
+// cross-lane reads before: 82 us, now 70 us a build at 65,536
+// particles of 24 vertices).
+template <bool SHIFT, class Box, class Entry, class Emit>
 __device__ __forceinline__ int vertex_row(const Box& bx, const double4* P, const int* vst,
                                           const int* nvt, const double2* vpos, double rv,
-                                          double vc, double vc2, double vp2, bool shift,
-                                          int lane, int hs, bool has, double2 xv, double4 cp,
-                                          int nn, Entry entry, Emit emit) {
+                                          double vc, double vc2, double vp2, int lane, int hs,
+                                          bool has, double2 xv, double4 cp, int nn,
+                                          RingEntry* R, Entry entry, Emit emit) {
     constexpr int HALF = WAVE / 2;
     int cnt = 0;
-    for (int k0 = 0; k0 < nn; k0 += HALF) {
-        int rf = 0, rn = 0;
-        double rx = 0.0, ry = 0.0, rr = 0.0;
-        double2 r0 = make_double2(0.0, 0.0);
+    auto image = [&](double a, double b, double s, double L, double invL, double halfL) {
+        if constexpr (SHIFT) return (a - b) - s;
+        else return pbc(a, b, L, invL, halfL, bx.fast);
+    };
+    for (int k0 = 0; __builtin_amdgcn_ballot_w64(k0 < nn) != 0; k0 += HALF) {
+        RingEntry e;
         bool near = false;
         if (k0 + lane < nn) {
             const int q = entry(k0 + lane);
             const double4 c = P[q];
-            rx = c.x;
-            ry = c.y;
-            rr = c.z;
-            rf = vst[q];
-            rn = nvt[q];
-            const double2 u = vpos[rf];
-            r0 = make_double2(u.x - c.x, u.y - c.y);
+            e.first = vst[q];
+            e.n = nvt[q];
+            e.cx = c.x;
+            e.cy = c.y;
+            e.sx = e.sy = 0.0;
             near = true;
-            if (shift) {  // both rings' radii and vc, with vertex_ring_near's margin
-                const double ex = pbc(cp.x, c.x, bx.Lx, bx.invLx, bx.halfLx, bx.fast);
-                const double ey = pbc(cp.y, c.y, bx.Ly, bx.invLy, bx.halfLy, bx.fast);
+            if constexpr (SHIFT) {  // both rings' radii and vc, with vertex_ring_near's margin
+                e.sx = bx.Lx * image_index(cp.x - c.x, bx.Lx, bx.invLx, bx.halfLx, bx.fast);
+                e.sy = bx.Ly * image_index(cp.y - c.y, bx.Ly, bx.invLy, bx.halfLy, bx.fast);
+                const double ex = (cp.x - c.x) - e.sx, ey = (cp.y - c.y) - e.sy;
                 const double reach = (cp.z - rv) + (c.z - rv) + vc;
                 near = ex * ex + ey * ey < reach * reach * (1.0 + 1e-6);
             }
+            if (near) {
+                const double2 u = vpos[e.first];
+                const double reach = c.z - rv + vc;
+                e.lim = fmin(vp2, reach * reach * (1.0 + 1e-6));
+                e.x0 = (float)(u.x - c.x);
+                e.y0 = (float)(u.y - c.y);
+                e.per = (float)e.n * 0.15915494f;
+                const float x = (float)vc / (float)(c.z - rv);
+                e.half = (x + 0.25f * x * x * x) * e.per + 0.02f + 2e-5f * e.per;
+                if (!(x < 0.6f && 2.0f * e.half + 2.0f < (float)e.n)) e.half = -1.0f;
+            }
         }
+        const unsigned nm = (unsigned)(__builtin_amdgcn_ballot_w64(near) >> hs);
+        if (near) R[__popc(nm & ((1u << lane) - 1u))] = e;
+        wave_sync();
+        const int entries = __popc(nm);
         unsigned gm = 0;
-        for (unsigned m = (unsigned)(__builtin_amdgcn_ballot_w64(near) >> hs); m; m &= m - 1) {
-            const int k = __builtin_ctz(m);
-            const double cx = __shfl(rx, k, HALF), cy = __shfl(ry, k, HALF);
-            const double cr = __shfl(rr, k, HALF);
-            const double kx = image_index(xv.x - cx, bx.Lx, bx.invLx, bx.halfLx, bx.fast);
-            const double ky = image_index(xv.y - cy, bx.Ly, bx.invLy, bx.halfLy, bx.fast);
-            const double dx = pbc_known(xv.x, cx, bx.Lx, kx, bx.fast);  // = pbc(xv, cq)
-            const double dy = pbc_known(xv.y, cy, bx.Ly, ky, bx.fast);
-            const double d2 = dx * dx + dy * dy;
-            if (has && d2 < vp2 && vertex_ring_near(d2, cr, rv, vc)) gm |= 1u << k;
+        for (int k = 0; k < entries; ++k) {
+            const double dx = image(xv.x, R[k].cx, R[k].sx, bx.Lx, bx.invLx, bx.halfLx);
+            const double dy = image(xv.y, R[k].cy, R[k].sy, bx.Ly, bx.invLy, bx.halfLy);
+            if (has && dx * dx + dy * dy < R[k].lim) gm |= 1u << k;
         }
-        while (__builtin_amdgcn_ballot_w64(gm != 0) != 0) {
-            const bool on = gm != 0;
-            const int k = on ? __builtin_ctz(gm) : 0;
-            const double cx = __shfl(rx, k, HALF), cy = __shfl(ry, k, HALF);
-            const double cr = __shfl(rr, k, HALF);
-            const double2 v0 = make_double2(__shfl(r0.x, k, HALF), __shfl(r0.y, k, HALF));
-            const int f0 = __shfl(rf, k, HALF), nq = __shfl(rn, k, HALF);
-            if (on) {
-                const double kx = image_index(xv.x - cx, bx.Lx, bx.invLx, bx.halfLx, bx.fast);
-                const double ky = image_index(xv.y - cy, bx.Ly, bx.invLy, bx.halfLy, bx.fast);
-                const double dx = pbc_known(xv.x, cx, bx.Lx, kx, bx.fast);
-                const double dy = pbc_known(xv.y, cy, bx.Ly, ky, bx.fast);
-                const RingWindow w = ring_window(dx, dy, v0, cr - rv, vc, nq);
-                for (int c = 0; c < w.count; ++c) {
-                    const int u = f0 + (c < w.wrapped ? c : w.first + c - w.wrapped);
-                    const double2 xu = vpos[u];
-                    double ex, ey;
-                    if (shift) {
-                        ex = pbc_known(xv.x, xu.x, bx.Lx, kx, bx.fast);
-                        ey = pbc_known(xv.y, xu.y, bx.Ly, ky, bx.fast);
-                    } else {
-                        ex = pbc(xv.x, xu.x, bx.Lx, bx.invLx, bx.halfLx, bx.fast);
-                        ey = pbc(xv.y, xu.y, bx.Ly, bx.invLy, bx.halfLy, bx.fast);
-                    }
-                    if (ex * ex + ey * ey < vc2) emit(cnt++, u);
+        while (gm != 0) {
+            const RingEntry& q = R[__builtin_ctz(gm)];
+            gm &= gm - 1;
+            const double sx = q.sx, sy = q.sy;
+            int lo = 0, count = q.n, first = q.first, n = q.n;
+            if (q.half >= 0.0f) {
+                const float dx = (float)image(xv.x, q.cx, sx, bx.Lx, bx.invLx, bx.halfLx);
+                const float dy = (float)image(xv.y, q.cy, sy, bx.Ly, bx.invLy, bx.halfLy);
+                const float t = q.per * atan2_coarse(q.x0 * dy - q.y0 * dx,
+                                                     q.x0 * dx + q.y0 * dy);
+                lo = (int)ceilf(t - q.half);
+                count = (int)floorf(t + q.half) - lo + 1;
+                if (lo < 0) lo += n;
+            }
+            // the candidates in ascending order: those beyond the ring's last vertex first
+            const int wrapped = max(0, lo + count - n);
+            constexpr int LOADS = 4;
+            for (int c0 = 0; c0 < count; c0 += LOADS) {
+                int u[LOADS];
+                double2 xu[LOADS];
+#pragma unroll
+                for (int t = 0; t < LOADS; ++t) {
+                    const int c = min(c0 + t, count - 1);
+                    u[t] = first + (c < wrapped ? c : lo + c - wrapped);
+                    xu[t] = vpos[u[t]];
+                }
+#pragma unroll
+                for (int t = 0; t < LOADS; ++t) {
+                    const double ex = image(xv.x, xu[t].x, sx, bx.Lx, bx.invLx, bx.halfLx);
+                    const double ey = image(xv.y, xu[t].y, sy, bx.Ly, bx.invLy, bx.halfLy);
+                    if (c0 + t < count && ex * ex + ey * ey < vc2) emit(cnt++, u[t]);
                 }
             }
-            gm &= gm - 1;
         }
+        wave_sync();  // the next entries take these ones' place
     }
     return cnt;
 }
