@@ -154,10 +154,16 @@ __device__ __forceinline__ double pair_hot(double4 qi, double4 q, bool valid, co
     double d = sqrt_rn_normal(d2);
     double ov = 1.0 - div_rn_normal(d, rs);
     double fm = div_rn_normal(p.e_c * ov, rs * d);
-    if (contact && d2 < 0x1p-700) {  // separations the short sequences do not cover
-        d = sqrt(d2);
-        ov = 1.0 - (d / rs);
-        fm = p.e_c * ov / (rs * d);
+    // Separations that the short sequences do not cover.  The whole wave branches: as a branch
+    // of the lane the compiler folded it into selects, and every pair paid for the IEEE square
+    // root and two divisions (85 double precision instructions instead of 50).
+    const bool tiny = contact && d2 < 0x1p-700;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(tiny) != 0, 0)) {
+        if (tiny) {
+            d = sqrt(d2);
+            ov = 1.0 - (d / rs);
+            fm = p.e_c * ov / (rs * d);
+        }
     }
     fx = contact ? fm * dx : 0.0;
     fy = contact ? fm * dy : 0.0;
