@@ -287,31 +287,79 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_build(Dev d, NbrParams n
 
 // The same rows for evenly spaced rings (dpm_system::vuniform): a half-wave per particle,
 // lanes over its vertices (vertex_row).  Grid-stride over the particles.
+//
+// LISTS (cell method): the half-wave builds its particle's list row first, as k_build_cell does
+// -- the particles are in cell order, so its lanes read the candidates as runs of records and
+// append the hits in order -- and hands it on through LDS.  A vertex row needs no other
+// particle's list row, so one launch does for both, and a step that rebuilds nothing has one
+// gated launch less (bumpy_fused_lists: for which sizes).
 constexpr int VB_HALF = 32;
+constexpr int VB_LIST = 64;  // row entries that LDS holds; the rest is read back
+template <bool LISTS>
 __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb, double rv,
                                                              double rmax, int gated) {
     if (gated && d.ctl->kind < 1) return;
     const double vc = sqrt(nb.vc2);
     const bool shift = fmin(nb.halfLx, nb.halfLy) > ring_shift_limit(rmax, rv, vc);
     __shared__ RingEntry rings[BLOCK / VB_HALF][VB_HALF];
+    __shared__ int lists[LISTS ? BLOCK / VB_HALF : 1][VB_LIST];
     RingEntry* ring = rings[threadIdx.x / VB_HALF];
+    int* list = lists[LISTS ? threadIdx.x / VB_HALF : 0];
     const int lane = (int)(threadIdx.x % VB_HALF);
     const int hs = (int)(threadIdx.x % WAVE) / VB_HALF * VB_HALF;
     const int64_t halves = (int64_t)gridDim.x * (BLOCK / VB_HALF);
-    int mx = 0;
+    int mx = 0, mn = 0;
     // (whole waves stay in the loop together: the odd half of the last wave has no particle)
     for (int64_t p0 = ((int64_t)blockIdx.x * BLOCK + threadIdx.x - lane - hs) / VB_HALF;
          p0 < d.N; p0 += halves) {
         const int64_t p = p0 + hs / VB_HALF;
         const bool live = p < d.N;
         const int st = live ? d.vstart[p] : 0, nv = live ? d.nverts[p] : 0;
-        const int nn = live ? min(d.nnum[p], d.cap) : 0;
         const double4 cp = d.P0[live ? p : 0];
+        int nn = 0;
+        if constexpr (LISTS) {
+            const int cid = live ? d.cell_of[p] : 0;
+            CellRuns runs;
+            runs.set(cid % nb.ncd, cid / nb.ncd, nb.ncd, nb.ncd, live,
+                     [&](int c0, int c1, int& a, int& e) {
+                         a = d.cell_start[c0];
+                         e = d.cell_start[c1 + 1];
+                     });
+            for (int t = lane; __builtin_amdgcn_ballot_w64(t < runs.count) != 0; t += VB_HALF) {
+                int j = 0;
+                bool hit = false;
+                if (t < runs.count) {
+                    j = runs.entry(t);
+                    const double4 q = d.P0[j];
+                    hit = j != p && within(cp.x, cp.y, q.x, q.y, nb, nb.rc2);
+                }
+                const unsigned m = (unsigned)(__builtin_amdgcn_ballot_w64(hit) >> hs);
+                const int pos = nn + __popc(m & ((1u << lane) - 1u));
+                if (hit && pos < d.cap) d.nbr[(int64_t)pos * d.N + p] = j;
+                if (hit && pos < VB_LIST) list[pos] = j;
+                nn += __popc(m);
+            }
+            if (live && lane == 0) {
+                d.nnum[p] = nn;
+                d.lref[p] = make_double2(cp.x, cp.y);
+                if (p % BLOCK == 0) d.pmax_nd[p / BLOCK] = 0.0;
+            }
+            mn = max(mn, nn);
+            nn = min(nn, d.cap);
+            // the entries, in LDS and beyond it in memory, before other lanes read them
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            nn = live ? min(d.nnum[p], d.cap) : 0;
+        }
+        auto entry = [&](int k) {
+            if (LISTS && k < VB_LIST) return list[k];
+            return d.nbr[(int64_t)k * d.N + p];
+        };
         for (int a0 = 0; __builtin_amdgcn_ballot_w64(a0 < nv) != 0; a0 += VB_HALF) {
             const bool has = a0 + lane < nv;
             const int64_t v = st + a0 + lane;
             const double2 xv = has ? d.vpos[v] : make_double2(0.0, 0.0);
-            auto entry = [&](int k) { return d.nbr[(int64_t)k * d.N + p]; };
             auto emit = [&](int pos, int u) {
                 if (pos < d.vcap) d.vnbr[(int64_t)pos * d.Nv + v] = u;
             };
@@ -325,11 +373,19 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb
                 mx = max(mx, cnt);
             }
         }
+        if (LISTS) wave_sync();  // the next particle's list takes this one's place
     }
     int m = block_max_int(mx);
     if (threadIdx.x == 0) {
         atomicMax(&d.ctl->max_vnum, m);
         atomicMax(&d.ctl->max_vnum_all, m);
+    }
+    if constexpr (LISTS) {
+        m = block_max_int(mn);
+        if (threadIdx.x == 0) {
+            atomicMax(&d.ctl->max_nnum, m);
+            atomicMax(&d.ctl->max_nnum_all, m);
+        }
     }
 }
 
@@ -986,14 +1042,29 @@ int bumpy_ensure_vcap(dpm_system* s, int64_t cap) {
     return 0;
 }
 
+// Whether the vertex rows' launch builds the particle list too: evenly spaced rings, cells that
+// do not repeat in a stencil, and few enough particles that the launch weighs more than the
+// longer chain of each half-wave.  Measured, us a step of 200 (two launches, one): FIRE from
+// overlaps, a rebuild in most steps: 48, 34 at 512 particles; 64, 53 at 4,096; 77, 75 at 8,192;
+// 110, 127 at 16,384; NVE: 20, 18 at 2,048; 26, 25 at 8,192; 37, 37 at 16,384.
+constexpr int64_t FUSED_LISTS_MAX_N = 8192;
+bool bumpy_fused_lists(const dpm_system* s) {
+    return s->kind == DPM_BUMPY && s->method == DPM_NBR_CELL && s->vuniform && s->ncd >= 3 &&
+           s->N <= FUSED_LISTS_MAX_N;
+}
+
 // RigidBumpy::updateVertexVerletList (rigid_bumpy.cu:1198-1212), enqueued after the
 // particle list build; overflow is detected by the chain's end kernel.
 void bumpy_enqueue_vertex_build(dpm_system* s, int gated) {
     // grid-stride: a gated launch that skips stays cheap
     if (s->vuniform) {
         dim3 g(std::min<unsigned>(pgrid(s->N * VB_HALF).x, 2048u));
-        hipLaunchKernelGGL(k_bumpy_vertex_rows, g, dim3(BLOCK), 0, s->stream, s->d,
-                           nbr_params(s), s->rv, s->rmax, gated);
+        if (bumpy_fused_lists(s))
+            hipLaunchKernelGGL(k_bumpy_vertex_rows<true>, g, dim3(BLOCK), 0, s->stream, s->d,
+                               nbr_params(s), s->rv, s->rmax, gated);
+        else
+            hipLaunchKernelGGL(k_bumpy_vertex_rows<false>, g, dim3(BLOCK), 0, s->stream, s->d,
+                               nbr_params(s), s->rv, s->rmax, gated);
         return;
     }
     dim3 g(std::min<unsigned>(pgrid(s->Nv).x, 2048u));

@@ -86,14 +86,6 @@ __device__ __forceinline__ void stencil_visit(const Dev& d, const NbrParams& nb,
     });
 }
 
-// isWithinCutoffSquared, include/particles/base/kernels.cuh:249-260
-__device__ __forceinline__ bool within(double ax, double ay, double bx, double by,
-                                       const NbrParams& nb, double c2) {
-    double dx = pbc(ax, bx, nb.Lx, nb.invLx, nb.halfLx, nb.fast);
-    double dy = pbc(ay, by, nb.Ly, nb.invLy, nb.halfLy, nb.fast);
-    return dx * dx + dy * dy < c2;
-}
-
 // The list row of particle i (kernelUpdateCellNeighborList, base/kernels.cu:440-505), written to
 // the column-major ELL.  `pos(j)` supplies the positions the list is built from; the positions
 // of BATCH candidates are loaded together.
@@ -1687,6 +1679,7 @@ static void enqueue_cell_sort(dpm_system* s, const NbrParams& nb, int cg) {
 
 void enqueue_list_build(dpm_system* s, int gated) {
     NbrParams nb = nbr_params(s);
+    if (bumpy_fused_lists(s)) return;  // with the vertex rows (bumpy_enqueue_vertex_build)
     if (s->method == DPM_NBR_CELL) {
         hipLaunchKernelGGL(k_build_cell, pgrid(s->N), dim3(BLOCK), 0, s->stream, s->d, nb, gated);
     } else if (s->method == DPM_NBR_VERLET && s->vg_ncd >= 3) {

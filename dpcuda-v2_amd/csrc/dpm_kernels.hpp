@@ -162,9 +162,17 @@ __device__ __forceinline__ int cell_coord(double pos, double cs, int n) {
     return (int)(idx >= 0 ? idx % n : (idx % n + n) % n);
 }
 
+// isWithinCutoffSquared, include/particles/base/kernels.cuh:249-260
+__device__ __forceinline__ bool within(double ax, double ay, double bx, double by,
+                                       const NbrParams& nb, double c2) {
+    double dx = pbc(ax, bx, nb.Lx, nb.invLx, nb.halfLx, nb.fast);
+    double dy = pbc(ay, by, nb.Ly, nb.invLy, nb.halfLy, nb.fast);
+    return dx * dx + dy * dy < c2;
+}
+
 // The candidates of a particle in cell (cx, cy) of a grid of nx x ny >= 3 x 3 cells, for lanes
-// that test them side by side: the list entries of the 3 x 3 cells around it, which are one run
-// in each row of cells, or two where the row wraps.  range(c0, c1, a, e) gives the entries
+// that test them side by side: the list entries of the 3 x 3 cells around it, rows and cells of
+// a row in ascending order, which are one run in each row of cells, or two where the row wraps.  range(c0, c1, a, e) gives the entries
 // [a, e) of cells c0 to c1.
 struct CellRuns {
     int a[6], m[6], count;
@@ -175,16 +183,17 @@ struct CellRuns {
         for (int r = 0; r < 3; ++r) {
             const int y = cy + r - 1 < 0 ? ny - 1 : (cy + r - 1 >= ny ? 0 : cy + r - 1);
             const int c = y * nx;
-            int e;
-            range(c + max(cx - 1, 0), c + min(cx + 1, nx - 1), a[2 * r], e);
-            m[2 * r] = live ? e - a[2 * r] : 0;
-            a[2 * r + 1] = 0;
-            m[2 * r + 1] = 0;
+            int b, e, wb = 0, we = 0;
+            range(c + max(cx - 1, 0), c + min(cx + 1, nx - 1), b, e);
             if (cx == 0 || cx == nx - 1) {
                 const int w = c + (cx == 0 ? nx - 1 : 0);
-                range(w, w, a[2 * r + 1], e);
-                m[2 * r + 1] = live ? e - a[2 * r + 1] : 0;
+                range(w, w, wb, we);
             }
+            const bool swap = cx == 0;  // the cell across the boundary comes first
+            a[2 * r] = swap ? wb : b;
+            m[2 * r] = live ? (swap ? we - wb : e - b) : 0;
+            a[2 * r + 1] = swap ? b : wb;
+            m[2 * r + 1] = live ? (swap ? e - b : we - wb) : 0;
             count += m[2 * r] + m[2 * r + 1];
         }
     }
@@ -344,6 +353,7 @@ int resident_fire(dpm_system* s, int64_t steps);
 
 // ---- rigid bumpy (dpm_bumpy.hip) ----
 int bumpy_alloc(dpm_system* s);
+bool bumpy_fused_lists(const dpm_system* s);
 int bumpy_forces(dpm_system* s, int mode);
 void bumpy_enqueue_vertex_build(dpm_system* s, int gated);
 void bumpy_enqueue_vertex_reorder(dpm_system* s, int gated);
