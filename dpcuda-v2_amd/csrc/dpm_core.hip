@@ -170,7 +170,11 @@ __device__ __forceinline__ void row_forces(const Dev& d, const double4* P, const
 // the caller ahead of everything that waits on the control block, batches of ROW_PF
 // records gathered together, and the wave's slot bound taken from ballots instead of
 // a shuffle reduction.  Same slots, same order, same arithmetic as row_forces.
-constexpr int ROW_PF = 2;
+// Four since the pair's range fallback left the lane's path (two before, when a batch of four
+// cost registers that the loads did not earn): 30,011 disks, 400 logged steps 3.72 ms with two,
+// 3.59 with four; 1,000,003 disks, 200 steps 14.3, 14.0; a step of 60,000 disks 6.08, 5.79 us, of
+// 262,144 12.17, 12.24.
+constexpr int ROW_PF = 4;
 
 __device__ __forceinline__ bool wave_any(bool x) {
     return __builtin_amdgcn_ballot_w64(x) != 0;
