@@ -369,7 +369,8 @@ int dpm_disk_forces_noalloc(const double* x, const double* y, const double* radi
 
 /* ---- execution options and measurement (no reference counterpart) -------------------------
  * DPM_OPT_GRAPH: capture the NVE/FIRE chunk in a hipGraph (default 1).
- * DPM_OPT_CHUNK: steps per host poll of the device status (default 32).
+ * DPM_OPT_CHUNK: steps per host poll of the device status (default 32; eight times as many in
+ *   the one-workgroup loops of small disk systems).
  * DPM_OPT_TIMING: 0 off (default); 1 HIP events around every launch of the hot kernels
  *   (disables graph capture); 2 HIP events around every graph-launched chunk of the NVE and
  *   FIRE loops (chunk time is charged to DPM_K_FORCE, recovery chains to DPM_K_REBUILD).
