@@ -1116,6 +1116,7 @@ __global__ __launch_bounds__(WAVE) void k_chain_end(Dev d, int mode) {
         bool over = c->max_nnum > d.cap || (d.vnbr != nullptr && c->max_vnum > d.vcap);
         if (mode != 0) {
             if (c->kind >= 1 && over) c->overflow = 1;
+            else if (c->kind >= 1) c->ovf = 0;
         } else {
             if (c->halt) {
                 if (c->overflow || over) {
@@ -1157,6 +1158,15 @@ __global__ void k_overflow_begin(Dev d) {
     if (c->kind != 3) c->kind = 1;
     c->max_nnum = 0;
     c->max_vnum = 0;
+}
+
+// Rows that the last step of a minimisation rebuilt and the ELL does not hold: an overflow of
+// that list (kind 3), for the host to fix.
+__global__ void k_rows_short(Dev d) {
+    Ctl* c = d.ctl;
+    c->overflow = 1;
+    c->kind = 3;
+    c->max_nnum = c->max_nnum_all;
 }
 
 __global__ void k_ctl_reset(Dev d, int config) {
@@ -1343,6 +1353,7 @@ __global__ __launch_bounds__(CTL_T) void k_fire_ctl(Dev d, int init, int pos, in
     __shared__ FireCtl S;
     if (threadIdx.x < sizeof(FireCtl) / sizeof(int))
         ((int*)&S)[threadIdx.x] = ((const int*)F)[threadIdx.x];
+    const long long ovf = c->ovf;
     if (gate == G_NORMAL) {
         if (c->halt || F->done) return;
     } else if (gate == G_RESUME) {
@@ -1385,6 +1396,7 @@ __global__ __launch_bounds__(CTL_T) void k_fire_ctl(Dev d, int init, int pos, in
         const bool done = init ? fire_begin(S, res[0], res[1], res[2], fm, spin)
                                : fire_advance(S, res[0], res[1], res[2], fm, spin);
         if (done) c->done = 1;
+        S.short_rows = gate == G_NORMAL && ovf != 0;  // (an older overflow would have halted)
     }
     __syncthreads();
     if (tid < (int)(sizeof(FireCtl) / sizeof(int))) ((int*)F)[tid] = ((const int*)&S)[tid];
@@ -2182,6 +2194,13 @@ int minimize_fire(dpm_system* s, const dpm_fire_params* prm, dpm_fire_result* ou
     hipLaunchKernelGGL(k_disp_partials, pgrid(s->N), dim3(BLOCK), 0, st, d, nbr_params(s));
     hipLaunchKernelGGL(k_zero_velocities, pgrid(s->N), dim3(BLOCK), 0, st, d);
     if (scopy(s, &f, d.fire, sizeof(FireCtl), hipMemcpyDeviceToHost)) return -1;
+    if (f.short_rows) {  // the step that would have halted for the rows was not taken
+        hipLaunchKernelGGL(k_rows_short, dim3(1), dim3(1), 0, st, d);
+        if (fix_overflow(s, 0, 0.0)) {
+            s->nbr_ready = false;
+            return -1;
+        }
+    }
     if (out) {
         out->steps = std::min<int64_t>(f.step, prm->max_steps);
         out->stopped = f.stopped;

@@ -38,7 +38,8 @@ struct Ctl {
     long long flag[2];
     long long cflag[2];
     long long epoch;          // bumped by the chain at the end of every chunk
-    long long ovf;            // stamp of a step whose in-kernel list rebuild overflowed
+    long long ovf;            // stamp of a step whose in-kernel list rebuild overflowed (0 once
+                              // the rows are complete; no run ends with it set)
     int halt;                 // a step stopped because it needs the rebuild chain
     int halt_pos;             // chunk position of the halted step
     int halt_mode;            // HaltMode of the halted step
@@ -63,6 +64,7 @@ struct FireCtl {
     double last_avg_pe, avg_pe, power, fmax_sq;
     long long n_good, n_bad, step, max_steps;
     int stopped, done, converged, uphill;
+    int short_rows;           // the last step rebuilt rows that the ELL does not hold yet
 };
 
 constexpr int HSCAL = 4;  // reductions whose results one wait collects
