@@ -339,7 +339,8 @@ __device__ __forceinline__ void nve_force_body(const Dev& d, const PairParams& p
         if (!c->halt || !resumable(d) || c->halt_mode == H_FIRE) return;
         closes = c->halt_mode == H_NVE_FORCE;
     }
-    if (closes && blockIdx.x == 0 && threadIdx.x == 0) c->closed = 1;
+    // (a run's own closing launch is recorded by k_unit_end: its workgroups read the word)
+    if (gate == G_RESUME && closes && blockIdx.x == 0 && threadIdx.x == 0) c->closed = 1;
     int tile;
     const int64_t i = particle_of_thread(tile);
     const bool live = i < d.N;
@@ -365,9 +366,13 @@ __global__ __launch_bounds__(BLOCK) void k_nve_force(Dev d, PairParams p, double
     nve_force_body<HOT>(d, p, hdt, pos, hmode, gate);
 }
 
-// End of a launch unit that changes no loop state (the closing force of a run): publishes
-// the control block (one wave).
-__global__ __launch_bounds__(WAVE) void k_unit_end(Dev d) { publish_ctl(d); }
+// End of the unit that closes a run (one wave): records that the closing force was applied, which
+// it was unless a step has halted, and publishes the control block.
+__global__ __launch_bounds__(WAVE) void k_unit_end(Dev d) {
+    if (threadIdx.x == 0 && !d.ctl->halt) d.ctl->closed = 1;
+    __syncthreads();
+    publish_ctl(d);
+}
 
 // Opening kick(dt/2) + drift(dt) in place on P0.  (wr_pos, epoch + wr_eoff) names
 // the step that must check the rebuild request; progress >= 0 is recorded (a resumed
