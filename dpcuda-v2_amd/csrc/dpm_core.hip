@@ -216,6 +216,25 @@ __device__ __forceinline__ void row_forces_pf(const Dev& d, const double4* P, co
     }
 }
 
+// The rest of a row that was just rebuilt from P and that the ELL does not hold: its entries
+// past the capacity, found again and added in row order.
+template <bool ENERGY, bool HOT>
+__device__ __forceinline__ void row_rest(const Dev& d, const double4* P, const PairParams& p,
+                                         const NbrParams& nb, int64_t i, double4 qi, double& ax,
+                                         double& ay, double& e) {
+    int k = 0;
+    stencil_visit(d, nb, i, [&](int j) {
+        const double4 q = P[j];
+        if (!within(qi.x, qi.y, q.x, q.y, nb, nb.rc2) || k++ < d.cap) return;
+        double fx, fy;
+        const double ie = HOT ? pair_hot<ENERGY>(qi, q, true, p, fx, fy)
+                              : pair_law(qi.x, qi.y, qi.z, q.x, q.y, q.z, p, fx, fy);
+        ax += fx;
+        ay += fy;
+        if (ENERGY) e += ie;
+    });
+}
+
 // ---- NVE (src/integrator/nve.cu:15-25) ---------------------------------------
 // One launch per step: zero + forces + closing kick(dt/2) of step s, then the
 // opening kick(dt/2) + drift(dt) of step s+1 (kernelCalcDiskForces,
@@ -286,6 +305,7 @@ __global__ __launch_bounds__(BLOCK) void k_nve_fused(Dev d, PairParams p, NbrPar
     const int nn = live ? min(nraw, d.cap) : 0;
     double ax, ay, e0;
     row_forces_pf<false, HOT>(d, Pc, p, il, qi, nn, jn, ax, ay, e0);
+    if (in_kernel && live && cnt > d.cap) row_rest<false, HOT>(d, Pc, p, nb, i, qi, ax, ay, e0);
     double nd = 0.0, cd = 0.0;
     if (live) {
         double fx = 0.0 + ax, fy = 0.0 + ay;
@@ -1296,18 +1316,7 @@ __global__ __launch_bounds__(BLOCK) void k_fire_force(Dev d, PairParams p, NbrPa
     const int nn = live ? min(cnt, d.cap) : 0;
     double ax, ay, e;
     row_forces_pf<true, HOT>(d, d.P0, p, il, qi, nn, jn, ax, ay, e);
-    if (in_kernel && live && cnt > d.cap) {  // the rest of a row that the ELL does not hold yet
-        int k = 0;
-        stencil_visit(d, nb, i, [&](int j) {
-            const double4 q = d.P0[j];
-            if (!within(qi.x, qi.y, q.x, q.y, nb, nb.rc2) || k++ < d.cap) return;
-            double fx, fy;
-            e += HOT ? pair_hot<true>(qi, q, true, p, fx, fy)
-                     : pair_law(qi.x, qi.y, qi.z, q.x, q.y, q.z, p, fx, fy);
-            ax += fx;
-            ay += fy;
-        });
-    }
+    if (in_kernel && live && cnt > d.cap) row_rest<true, HOT>(d, d.P0, p, nb, i, qi, ax, ay, e);
     if (in_kernel) {  // row-length statistics of the rebuild, one atomic per block
         const int m = block_max_int(live ? cnt : 0);
         if (threadIdx.x == 0) atomicMax(&c->max_nnum_all, m);

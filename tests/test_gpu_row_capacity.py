@@ -1,6 +1,6 @@
 """GPU test of cell-list rows that outgrow the ELL in a rebuild inside a step kernel, against the
 oracle bit for bit: a minimisation that ends in exactly that step, and what the queries, a following
-run and the pair lists then read.
+run and the pair lists then read; an NVE run through that step on the chunked loop.
 
 A jittered square lattice with a wide skin: its first rows hold 12 entries, so the ELL starts
 with 16 slots, and the first list rebuild (no cell sort) finds rows of more."""
@@ -93,5 +93,30 @@ def test_minimisation_that_ends_in_the_outgrowing_step(g, phi, dt, steps, then):
         q = s.neighbor_stats()
         got.append(out + state(s) + [q["n_rebuilds"], q["n_cell_rebuilds"], q["total_entries"],
                                      q["max_alloc"]])
+        s.close()
+    assert_same(*got)
+
+
+@pytest.mark.parametrize("steps", (35, 36, 37, 38, 70))
+def test_nve_through_the_outgrowing_step(steps):
+    print("[gpu-case] rows outgrow in an NVE step", steps, flush=True)
+    st = lattice(70, 1.0)
+    vx, vy = W.gaussian_velocities(st.n, 0.1, 5)
+
+    def run(s, k):
+        s.upload(P.F_VX, vx)
+        s.upload(P.F_VY, vy)
+        s.zero_forces()
+        s.compute_forces()
+        s.nve_run(0.01, k)
+
+    assert outgrows_in(st, 36, run)
+    got = []
+    for be in (None, oracle()):
+        s = make(st, be)
+        run(s, steps)
+        q = s.neighbor_stats()
+        got.append(state(s) + [q["n_rebuilds"], q["n_cell_rebuilds"], q["total_entries"],
+                               q["max_alloc"]])
         s.close()
     assert_same(*got)
