@@ -144,6 +144,9 @@ struct RingEntry {
 // SHIFT: the minimum image of x_p - x_q serves every vertex of both rings (ring_shift_limit):
 // pbc(v, u) = (v - u) - L k with one k, the same bits.  It is formed once per row entry; a lane
 // that formed it for every vertex and entry spent most of its instructions on it.
+// Without it (boxes of a few diameters) every vertex is tested by its own image, and all of them
+// are candidates: another image of the ring than its centre's nearest may be within vc of v, and
+// the window looks at the nearest alone.
 // What bounds it: the vector pipe (some 450 instructions a wave; the entries' fields came by
 // cross-lane reads before: 82 us, now 70 us a build at 65,536
 // particles of 24 vertices).
@@ -187,7 +190,7 @@ __device__ __forceinline__ int vertex_row(const Box& bx, const double4* P, const
                 e.per = (float)e.n * 0.15915494f;
                 const float x = (float)vc / (float)(c.z - rv);
                 e.half = (x + 0.25f * x * x * x) * e.per + 0.02f + 2e-5f * e.per;
-                if (!(x < 0.6f && 2.0f * e.half + 2.0f < (float)e.n)) e.half = -1.0f;
+                if (!SHIFT || !(x < 0.6f && 2.0f * e.half + 2.0f < (float)e.n)) e.half = -1.0f;
             }
         }
         const unsigned nm = (unsigned)(__builtin_amdgcn_ballot_w64(near) >> hs);
