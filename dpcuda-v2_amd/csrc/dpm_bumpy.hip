@@ -1129,11 +1129,11 @@ int bumpy_stress(dpm_system* s) {
     return check_launch();
 }
 
-// Whether every vertex lies at r - r_v from its particle's centre to a relative 1e-9
-// (vertex_ring_near's assumption), and whether the vertices of each particle are also evenly
-// spaced around it, counterclockwise and in the centre's own image, to 1e-6 (ring_window's):
-// both true after dpm_bumpy_setup, checked again on the host after an upload of positions,
-// radii or vertex positions.
+// Whether every vertex lies at r - r_v from its particle's centre, in the centre's own image, to a
+// relative 1e-9 (what vertex_ring_near and the image that serves a whole ring rest on), and
+// whether the vertices of each particle are also evenly spaced around it, counterclockwise, to
+// 1e-6 (RingEntry's window): both true after dpm_bumpy_setup, checked again on the host after an
+// upload of positions, radii or vertex positions.
 int bumpy_check_ring(dpm_system* s) {
     std::vector<double4> P(s->N);
     std::vector<int> st(s->N), nv(s->N);
@@ -1143,7 +1143,6 @@ int bumpy_check_ring(dpm_system* s) {
         scopy(s, nv.data(), s->d.nverts, sizeof(int) * s->N, hipMemcpyDeviceToHost) ||
         scopy(s, vp.data(), s->d.vpos, sizeof(double2) * s->Nv, hipMemcpyDeviceToHost))
         return -1;
-    auto img = [](double d, double L) { return d - L * std::round(d / L); };
     bool ok = true, even = true;
     int turn_nv = 0;
     double turn_s = 0.0, turn_c = 1.0;
@@ -1164,7 +1163,7 @@ int bumpy_check_ring(dpm_system* s) {
         }
         for (int k = 0; k < nv[p] && ok; ++k) {
             const double2 u = vp[st[p] + k];
-            const double dx = img(u.x - P[p].x, s->box[0]), dy = img(u.y - P[p].y, s->box[1]);
+            const double dx = u.x - P[p].x, dy = u.y - P[p].y;
             ok = inner > 0 && std::fabs(std::sqrt(dx * dx + dy * dy) - inner) <= 1e-9 * inner;
         }
     }

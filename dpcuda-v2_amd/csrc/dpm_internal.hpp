@@ -158,7 +158,8 @@ struct dpm_system {
     int64_t phys_cap = 0;
     int64_t vphys_cap = 0;
     int64_t nv_max = 0;         // most vertices of any particle
-    bool vring = false;         // every vertex at r - r_v from its centre (bumpy_check_ring)
+    bool vring = false;         // every vertex at r - r_v from its centre, in the centre's own
+                                // image (bumpy_check_ring)
     bool vuniform = false;      // and evenly spaced around it
     bool snap_vring = false, snap_vuniform = false;  // the snapshot's
     int64_t ncells_alloc = 0;
