@@ -721,9 +721,9 @@ __global__ __launch_bounds__(BLOCK) void k_rb_vbuild(BDev b) {
         };
         const int cnt =
             shift ? vertex_row<true>(pp, b.P, b.vst, b.nvt, b.vpos, S.rv, vc, S.vc2, S.vp2, lane,
-                                     hs, has, xv, cp, nn, ring, entry, emit)
+                                     hs, has, xv, cp, nn, true, ring, entry, emit)
                   : vertex_row<false>(pp, b.P, b.vst, b.nvt, b.vpos, S.rv, vc, S.vc2, S.vp2, lane,
-                                      hs, has, xv, cp, nn, ring, entry, emit);
+                                      hs, has, xv, cp, nn, true, ring, entry, emit);
         if (has) {
             b.vnum[v] = cnt;
             mx = max(mx, cnt);

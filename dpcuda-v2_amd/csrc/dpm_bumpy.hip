@@ -229,17 +229,11 @@ __device__ __forceinline__ bool within_v(double ax, double ay, double bx, double
     return dx * dx + dy * dy < c2;
 }
 
-// kernelUpdateVertexNeighborList, rigid_bumpy/kernels.cu:870-922
+// kernelUpdateVertexNeighborList, rigid_bumpy/kernels.cu:870-922, for vertices anywhere: a thread per
+// vertex, every pair by its own image.
 // gated: run only when the rebuild chain chose a list rebuild
-// ring: the vertices sit on their rings (dpm_system::vring), so q's vertices are scanned
-// only when v lies within reach of q's centre (vertex_ring_near); the rows are unchanged
-__global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_build(Dev d, NbrParams nb, double rv,
-                                                              double rmax, int ring,
-                                                              int gated) {
+__global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_build(Dev d, NbrParams nb, int gated) {
     if (gated && d.ctl->kind < 1) return;
-    const double vc = sqrt(nb.vc2);
-    // the centre's image serves q's vertices (pbc_known): needs the ring gate
-    const bool shift = ring && fmin(nb.halfLx, nb.halfLy) > vertex_shift_limit(rmax, rv, vc);
     int mx = 0;
     for (int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x; v < d.Nv;
          v += (int64_t)gridDim.x * BLOCK) {
@@ -250,24 +244,11 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_build(Dev d, NbrParams n
         for (int k = 0; k < nn; ++k) {
             int q = d.nbr[(int64_t)k * d.N + p];
             double4 cq = d.P0[q];
-            const double kx = image_index(xv.x - cq.x, nb.Lx, nb.invLx, nb.halfLx, nb.fast);
-            const double ky = image_index(xv.y - cq.y, nb.Ly, nb.invLy, nb.halfLy, nb.fast);
-            const double dx = pbc_known(xv.x, cq.x, nb.Lx, kx, nb.fast);  // = pbc(xv, cq)
-            const double dy = pbc_known(xv.y, cq.y, nb.Ly, ky, nb.fast);
-            const double d2 = dx * dx + dy * dy;
-            if (d2 < nb.vp2 && (!ring || vertex_ring_near(d2, cq.z, rv, vc))) {
+            if (within_v(xv.x, xv.y, cq.x, cq.y, nb, nb.vp2)) {
                 int f0 = d.vstart[q], nv = d.nverts[q];
                 for (int u = f0; u < f0 + nv; ++u) {
                     double2 xu = d.vpos[u];
-                    bool in;
-                    if (shift) {
-                        const double ux = pbc_known(xv.x, xu.x, nb.Lx, kx, nb.fast);
-                        const double uy = pbc_known(xv.y, xu.y, nb.Ly, ky, nb.fast);
-                        in = ux * ux + uy * uy < nb.vc2;
-                    } else {
-                        in = within_v(xv.x, xv.y, xu.x, xu.y, nb, nb.vc2);
-                    }
-                    if (in) {
+                    if (within_v(xv.x, xv.y, xu.x, xu.y, nb, nb.vc2)) {
                         if (cnt < d.vcap) d.vnbr[(int64_t)cnt * d.Nv + v] = u;
                         cnt++;
                     }
@@ -285,8 +266,10 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_build(Dev d, NbrParams n
     }
 }
 
-// The same rows for evenly spaced rings (dpm_system::vuniform): a half-wave per particle,
-// lanes over its vertices (vertex_row).  Grid-stride over the particles.
+// The same rows for vertices on their rings (dpm_system::vring): a half-wave per particle, lanes
+// over its vertices (vertex_row; even: evenly spaced rings, dpm_system::vuniform).  Grid-stride
+// over the particles.  Measured against a thread per vertex, ms for 100 FIRE steps of unevenly
+// spaced rings: 12.8, 7.5 at 4,000 particles; 20.0, 13.5 at 20,000.
 //
 // LISTS (cell method): the half-wave builds its particle's list row first, as k_build_cell does
 // -- the particles are in cell order, so its lanes read the candidates as runs of records and
@@ -297,7 +280,8 @@ constexpr int VB_HALF = 32;
 constexpr int VB_LIST = 64;  // row entries that LDS holds; the rest is read back
 template <bool LISTS>
 __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb, double rv,
-                                                             double rmax, int gated) {
+                                                             double rmax, int even,
+                                                             int gated) {
     if (gated && d.ctl->kind < 1) return;
     const double vc = sqrt(nb.vc2);
     const bool shift = fmin(nb.halfLx, nb.halfLy) > ring_shift_limit(rmax, rv, vc);
@@ -365,9 +349,11 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb
             };
             const int cnt =
                 shift ? vertex_row<true>(nb, d.P0, d.vstart, d.nverts, d.vpos, rv, vc, nb.vc2,
-                                         nb.vp2, lane, hs, has, xv, cp, nn, ring, entry, emit)
+                                         nb.vp2, lane, hs, has, xv, cp, nn, even, ring, entry,
+                                         emit)
                       : vertex_row<false>(nb, d.P0, d.vstart, d.nverts, d.vpos, rv, vc, nb.vc2,
-                                          nb.vp2, lane, hs, has, xv, cp, nn, ring, entry, emit);
+                                          nb.vp2, lane, hs, has, xv, cp, nn, even, ring, entry,
+                                         emit);
             if (has) {
                 d.vnum[v] = cnt;
                 mx = max(mx, cnt);
@@ -1042,14 +1028,14 @@ int bumpy_ensure_vcap(dpm_system* s, int64_t cap) {
     return 0;
 }
 
-// Whether the vertex rows' launch builds the particle list too: evenly spaced rings, cells that
-// do not repeat in a stencil, and few enough particles that the launch weighs more than the
+// Whether the vertex rows' launch builds the particle list too: vertices on their rings, cells
+// that do not repeat in a stencil, and few enough particles that the launch weighs more than the
 // longer chain of each half-wave.  Measured, us a step of 200 (two launches, one): FIRE from
 // overlaps, a rebuild in most steps: 48, 34 at 512 particles; 64, 53 at 4,096; 77, 75 at 8,192;
 // 110, 127 at 16,384; NVE: 20, 18 at 2,048; 26, 25 at 8,192; 37, 37 at 16,384.
 constexpr int64_t FUSED_LISTS_MAX_N = 8192;
 bool bumpy_fused_lists(const dpm_system* s) {
-    return s->kind == DPM_BUMPY && s->method == DPM_NBR_CELL && s->vuniform && s->ncd >= 3 &&
+    return s->kind == DPM_BUMPY && s->method == DPM_NBR_CELL && s->vring && s->ncd >= 3 &&
            s->N <= FUSED_LISTS_MAX_N;
 }
 
@@ -1057,19 +1043,19 @@ bool bumpy_fused_lists(const dpm_system* s) {
 // particle list build; overflow is detected by the chain's end kernel.
 void bumpy_enqueue_vertex_build(dpm_system* s, int gated) {
     // grid-stride: a gated launch that skips stays cheap
-    if (s->vuniform) {
+    if (s->vring) {
         dim3 g(std::min<unsigned>(pgrid(s->N * VB_HALF).x, 2048u));
         if (bumpy_fused_lists(s))
             hipLaunchKernelGGL(k_bumpy_vertex_rows<true>, g, dim3(BLOCK), 0, s->stream, s->d,
-                               nbr_params(s), s->rv, s->rmax, gated);
+                               nbr_params(s), s->rv, s->rmax, (int)s->vuniform, gated);
         else
             hipLaunchKernelGGL(k_bumpy_vertex_rows<false>, g, dim3(BLOCK), 0, s->stream, s->d,
-                               nbr_params(s), s->rv, s->rmax, gated);
+                               nbr_params(s), s->rv, s->rmax, (int)s->vuniform, gated);
         return;
     }
     dim3 g(std::min<unsigned>(pgrid(s->Nv).x, 2048u));
     hipLaunchKernelGGL(k_bumpy_vertex_build, g, dim3(BLOCK), 0, s->stream, s->d, nbr_params(s),
-                       s->rv, s->rmax, (int)s->vring, gated);
+                       gated);
 }
 
 // Vertex half of the cell reorder: new vertex starts from the permuted counts, then
@@ -1130,9 +1116,9 @@ int bumpy_stress(dpm_system* s) {
 }
 
 // Whether every vertex lies at r - r_v from its particle's centre, in the centre's own image, to a
-// relative 1e-9 (what vertex_ring_near and the image that serves a whole ring rest on), and
+// relative 1e-9 (what RingEntry's reach and the image that serves a whole ring rest on), and
 // whether the vertices of each particle are also evenly spaced around it, counterclockwise, to
-// 1e-6 (RingEntry's window): both true after dpm_bumpy_setup, checked again on the host after an
+// 1e-6 (its window): both true after dpm_bumpy_setup, checked again on the host after an
 // upload of positions, radii or vertex positions.
 int bumpy_check_ring(dpm_system* s) {
     std::vector<double4> P(s->N);

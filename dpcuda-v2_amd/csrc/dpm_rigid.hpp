@@ -62,42 +62,23 @@ __device__ __forceinline__ double2 ring_vertex(double2 c, double r, double a, in
     return make_double2(c.x + inner * cv, c.y + inner * sv);
 }
 
-// Whether a vertex v at squared distance d2 from the centre of particle q (radius r_q,
-// vertex radius rv) can have one of q's vertices within vc: every vertex of q lies at
-// r_q - rv from its centre (to rounding of the rotations, far below the margin), so by
-// the triangle inequality none can when d2 >= (r_q - rv + vc)^2; the test keeps a
-// relative margin of 1e-6 and so only skips vertex scans that would list nothing.
-__device__ __forceinline__ bool vertex_ring_near(double d2, double rq, double rv, double vc) {
-    const double reach = rq - rv + vc;
-    return d2 < reach * reach * (1.0 + 1e-6);
-}
+// The ring's reach: every vertex of q (radius r_q, vertex radius rv) lies at r_q - rv from its
+// centre (to rounding of the rotations, far below the margin), so by the triangle inequality a
+// vertex at squared distance d2 from the centre has none of them within vc when d2 >=
+// (r_q - rv + vc)^2.  The tests keep a relative margin of 1e-6 and so only skip scans that would
+// list nothing.
 
-// Vertex rows through the centre's image.  For a vertex v and a particle q that passed
-// vertex_ring_near, every vertex u of q lies within ring reach + (r_q - r_v) of v; when
-// half the box exceeds that bound (vertex_shift_ok), the minimum image of v - u is the
-// image of v - x_q: pbc(v, u) = (v - u) - L k with the same k.  image_index gives that k
-// as pbc forms it (0 when |d| < L/2 on the fast path, where pbc returns d itself), and
-// pbc_known applies it with pbc's own operations, so the bits are pbc's.
+// The image index k of a minimum image, pbc(a, b) = d - L k with d = a - b, as pbc forms it (0
+// when |d| < L/2 on the fast path, where pbc returns d itself).
 __device__ __forceinline__ double image_index(double d, double L, double invL, double halfL,
                                               int fast) {
     if (fast) return fabs(d) < halfL ? 0.0 : round(d * invL);
     return round(d / L);
 }
 
-__device__ __forceinline__ double pbc_known(double a, double b, double L, double k, int fast) {
-    const double d = a - b;
-    if (fast && k == 0.0) return d;
-    return d - L * k;
-}
-
-// The half box a system needs for the image shortcut: ring reach plus ring radius of the
-// largest particle (vertex_ring_near's relative margin included).
-__device__ __host__ inline double vertex_shift_limit(double rmax, double rv, double vc) {
-    return (2.0 * rmax - 2.0 * rv + vc) * (1.0 + 1e-6);
-}
-
-// The same for the image of two centres whose rings can reach each other (their distance is at
-// most two ring radii and vc) to serve every vertex of the first.
+// The half box a system needs for the image of two centres whose rings can reach each other
+// (their distance is at most two ring radii and vc) to serve every vertex of both: the distance
+// of any two of those vertices stays below it.
 __device__ __host__ inline double ring_shift_limit(double rmax, double rv, double vc) {
     return (3.0 * rmax - 3.0 * rv + vc) * (1.0 + 1e-6);
 }
@@ -115,7 +96,7 @@ __device__ __forceinline__ float atan2_coarse(float y, float x) {
 
 // A neighbouring particle q of a particle row, as the vertex rows need it: centre, the shift
 // L k of the minimum image of v - x_q, the squared distance below which a vertex looks at its
-// ring (min of the vertex-particle cutoff's square and vertex_ring_near's bound), vertex 0 from
+// ring (min of the vertex-particle cutoff's square and the ring's reach), vertex 0 from
 // the centre, and the window's half width.
 //
 // The window: which vertices of ring q (n of them, radius R, evenly spaced counterclockwise from
@@ -133,14 +114,15 @@ struct RingEntry {
 
 // The vertex rows of one particle (kernelUpdateVertexNeighborList, rigid_bumpy/kernels.cu:
 // 870-922: for vertex v, over the particle row in order, the particles q whose centre lies
-// within vp of v, then q's vertices in order within vc of v), for evenly spaced rings: a
-// half-wave per particle, lane a0 + lane its vertex xv; the return value is the lane's row
-// length, emit(pos, u) stores entry pos.  R: 32 entries of LDS of the half-wave's own.
+// within vp of v, then q's vertices in order within vc of v), for vertices on their rings (even:
+// evenly spaced ones): a half-wave per particle, lane a0 + lane its vertex xv; the return value
+// is the lane's row length, emit(pos, u) stores entry pos.  R: 32 entries of LDS of the
+// half-wave's own.
 //   1. each lane loads one row entry and puts it into R if some vertex of the particle can
 //      reach it (in row order);
-//   2. every lane tests the entries (vp and vertex_ring_near) into a bit mask;
+//   2. every lane tests the entries (vp and the ring's reach) into a bit mask;
 //   3. every lane walks its own mask and tests the window of q's vertices (3 or 4 of 20 to 28)
-//      that can be within vc, four loads at a time.
+//      that can be within vc, or all of an uneven ring's, four loads at a time.
 // SHIFT: the minimum image of x_p - x_q serves every vertex of both rings (ring_shift_limit):
 // pbc(v, u) = (v - u) - L k with one k, the same bits.  It is formed once per row entry; a lane
 // that formed it for every vertex and entry spent most of its instructions on it.
@@ -154,7 +136,7 @@ template <bool SHIFT, class Box, class Entry, class Emit>
 __device__ __forceinline__ int vertex_row(const Box& bx, const double4* P, const int* vst,
                                           const int* nvt, const double2* vpos, double rv,
                                           double vc, double vc2, double vp2, int lane, int hs,
-                                          bool has, double2 xv, double4 cp, int nn,
+                                          bool has, double2 xv, double4 cp, int nn, bool even,
                                           RingEntry* R, Entry entry, Emit emit) {
     constexpr int HALF = WAVE / 2;
     int cnt = 0;
@@ -174,7 +156,7 @@ __device__ __forceinline__ int vertex_row(const Box& bx, const double4* P, const
             e.cy = c.y;
             e.sx = e.sy = 0.0;
             near = true;
-            if constexpr (SHIFT) {  // both rings' radii and vc, with vertex_ring_near's margin
+            if constexpr (SHIFT) {  // both rings' radii and vc, with the margin
                 e.sx = bx.Lx * image_index(cp.x - c.x, bx.Lx, bx.invLx, bx.halfLx, bx.fast);
                 e.sy = bx.Ly * image_index(cp.y - c.y, bx.Ly, bx.invLy, bx.halfLy, bx.fast);
                 const double ex = (cp.x - c.x) - e.sx, ey = (cp.y - c.y) - e.sy;
@@ -190,7 +172,8 @@ __device__ __forceinline__ int vertex_row(const Box& bx, const double4* P, const
                 e.per = (float)e.n * 0.15915494f;
                 const float x = (float)vc / (float)(c.z - rv);
                 e.half = (x + 0.25f * x * x * x) * e.per + 0.02f + 2e-5f * e.per;
-                if (!SHIFT || !(x < 0.6f && 2.0f * e.half + 2.0f < (float)e.n)) e.half = -1.0f;
+                if (!SHIFT || !even || !(x < 0.6f && 2.0f * e.half + 2.0f < (float)e.n))
+                    e.half = -1.0f;
             }
         }
         const unsigned nm = (unsigned)(__builtin_amdgcn_ballot_w64(near) >> hs);
