@@ -200,6 +200,10 @@ __global__ __launch_bounds__(NA_T) void k_na_total(const double* part, int64_t n
 // one pair each; three lanes then add the components in rank order (the ascending order of the
 // Verlet rows).  A serial walk that merged the nine lists in order spent some 60 instructions
 // and a dependent load on each of 27 candidates.
+// A particle with more hits than LDS holds takes them by windows of the index, each found by all
+// lanes again: 2,000 particles at a cutoff of 3.5 (some 30 to 45 pairs) 43 us a call, 2,077 when
+// three lanes looked for one pair at a time, 211 by the serial walk; 4,000 particles in a cluster
+// (up to 160 pairs) 330, 33,500 and 1,460 us.
 // LDS: the grid is the workgroup's own, the particles are the caller's arrays in their order, and
 // the workgroup is a chunk of the energy sum.  Otherwise `rec` holds the particles in cell order
 // and `start` the cells' first records: reading the caller's arrays at random costs a cache line
@@ -254,26 +258,31 @@ __global__ __launch_bounds__(NA_T) void k_na_forces(const double* x, const doubl
         return dx * dx + dy * dy < rc2;
     };
     const int shift = lane - sub;
-    int cnt = 0;
-    for (int t = sub; __builtin_amdgcn_ballot_w64(t < cand) != 0; t += NA_GROUP) {
-        int u = -1, key = 0;
-        bool hit = false;
-        if (t < cand) {
-            u = candidate(t);
-            const double4 o = load(u);
-            key = key_of(u, o);
-            hit = u != (int)me && listed(o);
+    // the hits (with an index in [lo, lo + width)): as many as LDS holds, and their number
+    auto collect = [&](auto window, int lo, int width) {
+        int cnt = 0;
+        for (int t = sub; __builtin_amdgcn_ballot_w64(t < cand) != 0; t += NA_GROUP) {
+            int u = -1, key = 0;
+            bool hit = false;
+            if (t < cand) {
+                u = candidate(t);
+                const double4 o = load(u);
+                key = key_of(u, o);
+                hit = u != (int)me && listed(o);
+                if constexpr (window.value) hit = hit && key >= lo && key - lo < width;
+            }
+            const unsigned mask =
+                (unsigned)(__builtin_amdgcn_ballot_w64(hit) >> shift) & ((1u << NA_GROUP) - 1);
+            const int pos = cnt + __popc(mask & ((1u << sub) - 1));
+            if (hit && pos < NA_HITS) {
+                L.hit[k][pos] = u;
+                L.key[k][pos] = key;
+            }
+            cnt += __popc(mask);
         }
-        const unsigned mask =
-            (unsigned)(__builtin_amdgcn_ballot_w64(hit) >> shift) & ((1u << NA_GROUP) - 1);
-        const int pos = cnt + __popc(mask & ((1u << sub) - 1));
-        if (hit && pos < NA_HITS) {
-            L.hit[k][pos] = u;
-            L.key[k][pos] = key;
-        }
-        cnt += __popc(mask);
-    }
-    wave_sync();
+        wave_sync();
+        return cnt;
+    };
     auto pair = [&](int u, double& px, double& py) {
         const double4 o = load(u);
         const double rs = q.z + o.z;
@@ -282,7 +291,7 @@ __global__ __launch_bounds__(NA_T) void k_na_forces(const double* x, const doubl
         return pair_law(q.x, q.y, q.z, o.x, o.y, o.z, w, px, py);
     };
     double acc = 0.0;
-    if (cnt <= NA_HITS) {
+    auto add = [&](int cnt) {  // the hits in LDS, in ascending order
         for (int h = sub; h < cnt; h += NA_GROUP) {
             const int key = L.key[k][h];
             int rank = 0;
@@ -297,22 +306,23 @@ __global__ __launch_bounds__(NA_T) void k_na_forces(const double* x, const doubl
             for (int v = 0; v < cnt; ++v)
                 acc += sub == 0 ? L.f[k][v].x : (sub == 1 ? L.f[k][v].y : L.e[k][v]);
         }
-    } else if (sub < 3) {  // more hits than LDS holds: found again in ascending order
-        for (int v = 0, lo = -1; v < cnt; ++v) {
-            int next = INT_MAX, at = 0;
-            for (int t = 0; t < cand; ++t) {
-                const int u = candidate(t);
-                const double4 o = load(u);
-                const int key = key_of(u, o);
-                if (key > lo && key < next && u != (int)me && listed(o)) {
-                    next = key;
-                    at = u;
-                }
+    };
+    const int total = collect(std::false_type{}, 0, 0);
+    if (total <= NA_HITS) {
+        add(total);
+    } else {  // by windows of the index that LDS holds
+        int width = max(1, (int)(n * (NA_HITS * 2 / 3) / total));
+        for (int lo = 0, done = 0; done < total && lo < n;) {
+            const int cnt = collect(std::true_type{}, lo, width);
+            if (cnt > NA_HITS) {
+                width /= 2;
+                continue;
             }
-            lo = next;
-            double px, py;
-            const double e = pair(at, px, py);
-            acc += sub == 0 ? px : (sub == 1 ? py : e);
+            add(cnt);
+            wave_sync();  // the next window's take this one's place
+            done += cnt;
+            lo += width;
+            if (cnt < NA_HITS / 2) width = min(2 * width, (int)n);
         }
     }
     acc = 0.0 + acc;
