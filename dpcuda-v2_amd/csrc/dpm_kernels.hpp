@@ -345,6 +345,11 @@ struct Timed {
 // 20, 7.2 at 1,000; 20, 14.4 at 2,040; NVE in runs of 16 steps 7.2, 5.0 at 1,000.  One CU's LDS
 // and vector pipe bound it, where the chunked step is launch gaps.
 constexpr int64_t RESIDENT_MAX_NVE = 1536, RESIDENT_MAX_FIRE = 2048;
+// Systems that are expected to be dense (dpm_resident.hpp: a wide skin) sum full rows, which one CU
+// takes long over: us a step with a skin of 1.0 (chunked, resident): NVE 6.1, 5.4 at 256
+// particles, 6.4, 8.8 at 384, 7.3, 22 at 1,536; FIRE 14, 9.4 at 384, 14.5, 12 at 700, 15.3, 15.1
+// at 1,000 (1.3: 15.5, 16.8), 15, 29 at 2,000.
+constexpr int64_t RESIDENT_DENSE_NVE = 256, RESIDENT_DENSE_FIRE = 768;
 constexpr int64_t RESIDENT_MIN_STEPS = 16;
 bool resident_ok(const dpm_system* s, bool fire);
 int resident_prepare(dpm_system* s);

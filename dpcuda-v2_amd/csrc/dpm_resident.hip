@@ -352,11 +352,26 @@ __global__ __launch_bounds__(T) void k_resident(Dev d, Spare sp, PairParams p, N
     }
 }
 
+// Whether a system is expected to have near rows and pairs that some class holds.
+constexpr double RES_MOST_PAIRS = 3.0 * 2048;
+static bool resident_sparse(const ResLoad& l) {
+    return l.row <= RES_ROW && l.pairs <= RES_MOST_PAIRS;
+}
+
+// The size class of a system: its particles, its cells and, unless it is dense in every class, its
+// expected pairs must fit (a class that they outgrow costs more than the next).
+static int64_t resident_need(const dpm_system* s) {
+    const ResLoad l(s->N, s->box[0] * s->box[1], s->rmin, s->rmax, s->thr_sq);
+    int64_t need = std::max(s->N, s->method == DPM_NBR_CELL ? s->ncells : (int64_t)0);
+    if (resident_sparse(l)) need = std::max(need, (int64_t)std::ceil(l.pairs / 3.0));
+    return need;
+}
+
 template <bool FIRE>
 static int launch_resident(dpm_system* s, double dt, int steps) {
     const PairParams p = params_of(s);
     const NbrParams nb = nbr_params(s);
-    const int64_t need = std::max(s->N, s->method == DPM_NBR_CELL ? s->ncells : (int64_t)0);
+    const int64_t need = resident_need(s);
     hipStream_t st = s->stream;
     if (need <= 256)
         hipLaunchKernelGGL((k_resident<FIRE, 512, 256>), dim3(1), dim3(512), 0, st, s->d, s->sp,
@@ -382,11 +397,13 @@ bool resident_ok(const dpm_system* s, bool fire) {
         return false;
     }
     const PairParams p = params_of(s);
-    return p.fast && p.fastdiv;
+    if (!p.fast || !p.fastdiv) return false;
+    const ResLoad l(s->N, s->box[0] * s->box[1], s->rmin, s->rmax, s->thr_sq);
+    return resident_sparse(l) || s->N <= (fire ? RESIDENT_DENSE_FIRE : RESIDENT_DENSE_NVE);
 }
 
 int resident_prepare(dpm_system* s) {
-    const bool big = s->N > 1024 || (s->method == DPM_NBR_CELL && s->ncells > 1024);
+    const bool big = resident_need(s) > 1024;
     if (!big || s->res_rows) return 0;
     return dalloc(s, &s->res_rows, (int64_t)RES_LC * 2048);
 }

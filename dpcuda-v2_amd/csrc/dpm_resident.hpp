@@ -19,6 +19,8 @@
 // and symmetric to the bit).  Then each particle's thread adds its pairs in the order of its
 // row, which gives the row walk's sums.
 #pragma once
+#include <cmath>
+
 #include "dpm_kernels.hpp"
 
 namespace dpm {
@@ -63,6 +65,22 @@ struct ResRows {
 // boxes too small for the branch-free minimum image, make a system "dense": its forces are then
 // summed over the full rows.
 constexpr int RES_LC = 16;
+
+// What a system of n particles spread over its box is expected to have (host): the near entries of
+// a large particle and the pairs, from the mean density.  A cluster in a large box has more.
+// Counted on half and half disks of 1 : 1.4 at phi 0.70 to 0.90, skins of 0.3 to 1.0, relaxed:
+// 0.80 to 1.04 of the pairs (above 0.95 only at the narrow end, where every class has room), and
+// rows of up to 13 where 10.7 entries are expected, 16 where 12.0 are (longer ones in motion).
+constexpr double RES_ROW = 11.0, RES_PAIR_SHARE = 0.93;
+struct ResLoad {
+    double row, pairs;
+    ResLoad(double n, double area, double rmin, double rmax, double thr) {
+        const double rho = n / area * 3.141592653589793, mid = 0.5 * (rmin + rmax);
+        const double delta2 = 2.0 * std::sqrt(std::max(thr, 0.0) / 3.0);
+        row = rho * (rmax + mid + delta2) * (rmax + mid + delta2);
+        pairs = RES_PAIR_SHARE * 0.5 * n * rho * (2.0 * mid + delta2) * (2.0 * mid + delta2);
+    }
+};
 constexpr unsigned short RES_FLIP = 0x8000;  // the particle is its pair's upper one
 
 // How a system of NP particles is held by T threads
