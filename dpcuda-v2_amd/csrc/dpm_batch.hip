@@ -1827,20 +1827,15 @@ static int resident_join(dpm_batch* b) {
 }
 
 static void drop_graph(dpm_batch* b) {
-    if (b->exec) {
-        (void)hipGraphExecDestroy(b->exec);
-        (void)hipGraphDestroy(b->graph);
-        b->exec = nullptr;
-    }
+    if (b->exec) (void)hipGraphExecDestroy(b->exec);
+    if (b->graph) (void)hipGraphDestroy(b->graph);
+    b->exec = nullptr;
+    b->graph = nullptr;
 }
 
 static int ensure_batch_graph(dpm_batch* b, int64_t k) {
     if (b->exec && b->graph_steps == k) return 0;
-    if (b->exec) {
-        (void)hipGraphExecDestroy(b->exec);
-        (void)hipGraphDestroy(b->graph);
-        b->exec = nullptr;
-    }
+    drop_graph(b);
     std::lock_guard<std::mutex> lk(capture_mutex());
     DPM_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     for (int64_t s = 0; s < k; ++s) enqueue_batch_step(b);
@@ -1992,8 +1987,7 @@ void dpm_batch_destroy(dpm_batch* b) {
     for (auto st : b->rstream)
         if (st) (void)hipStreamSynchronize(st);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
+    drop_graph(b);
     {
         std::lock_guard<std::mutex> g(capture_mutex());
         for (void* p : b->allocs) (void)hipFree(p);
@@ -2300,11 +2294,7 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
     const int nt[2] = {(int)b->ntiles, b->nct};  // live until the synchronisation below
     DPM_HIP(hipMemcpyAsync(d.flags + 4, nt, 2 * sizeof(int), hipMemcpyHostToDevice, b->stream));
     DPM_HIP(hipStreamSynchronize(b->stream));
-    if (b->exec) {  // the parameters are baked into the graph's kernel arguments
-        (void)hipGraphExecDestroy(b->exec);
-        (void)hipGraphDestroy(b->graph);
-        b->exec = nullptr;
-    }
+    drop_graph(b);  // the parameters are baked into its kernel arguments
     // up to two launch units in flight; each ends with a copy of the flags
     int64_t launched = 0, finished_steps = 0;
     int inflight = 0, slot = 0;
