@@ -1475,6 +1475,7 @@ struct dpm_batch {
     int rrows_for[dpm::RES_CLASSES - dpm::RES_ROWS] = {0, 0};
     int rcount[dpm::RES_CLASSES] = {};
     bool phased = true;  // some system is advanced by the per-phase kernels
+    bool slow_phased = false;  // and is rigid or above RES_MAX_N (serving loop)
     hipStream_t rstream[dpm::RES_CLASSES] = {};
     hipEvent_t rfork = nullptr, rjoin[dpm::RES_CLASSES] = {};
     // DPM_OPT_TIMING: HIP events around every k_b_force launch (eager launches)
@@ -1741,13 +1742,48 @@ static void enqueue_batch_step(dpm_batch* b) {
     hipLaunchKernelGGL(k_b_jam, dim3((unsigned)b->nsys), dim3(WAVE), 0, st, d);
 }
 
-// Whether a system of n particles is advanced by k_b_resident: disks that fit a workgroup,
-// with a pair law of the short sequences (fastdiv), and no timing of the force pass asked for.
-// The line lies where the LDS ends: up to there one workgroup's step beats seven launches
-// (384 systems of 64 to 2,048 particles: 157 ms against 708 ms).
+// Whether a system can be advanced by k_b_resident: disks that fit a workgroup, with a pair law of
+// the short sequences (fastdiv), and no timing of the force pass asked for.
 static bool resident_size(const dpm_batch* b, int64_t n, bool rigid, bool fastdiv) {
     return !rigid && fastdiv && !b->timing && n <= RES_MAX_N;
 }
+
+// And whether it is.  A resident step takes one CU the longer, the larger and denser its system;
+// the per-phase kernels' step hardly depends on a system's size until the chip fills.  Both
+// estimates are fits, in us, of FIRE steps of 1 to 32 equal systems of 256 to 4,096 half and half
+// disks of 1 : 1.4 at phi 0.84, cutoffs of 1.7 to 2.6 (measured per-phase, resident): one system
+// of 1,000 23, 12; of 2,000 24, 23; of 4,096 26, 51; eight of 4,096 38, 54; 32 of 4,096 63, 57;
+// with a cutoff of 2.3 (full rows) one of 2,000 25, 42, one of 4,096 26, 90, 32 of 4,096 55, 102.
+// A batch starts from any state, random ones too, whose longest rows are longer (RES_ROW is for
+// relaxed ones).
+static double resident_us(const dpm_batch* b, int64_t n, double side, double rmin, double rmax) {
+    constexpr double ROW = 9.5;
+    const double area = side * side, k = (double)n;
+    const ResLoad l(k, area, rmin, rmax, b->thr_sq);
+    int c = 0;
+    while (c < RES_CLASSES - 1 && n > RES_LIMIT[c]) ++c;
+    const bool walk = RES_LIMIT[c] > 2048;
+    if (!(l.row <= ROW) || (!walk && !(l.pairs <= 3.0 * RES_LIMIT[c])))
+        return 5.0 + 2.0e-3 * k * (k / area * 3.141592653589793 * b->rc * b->rc);
+    return walk ? 8.5 + (7.0e-3 + 0.57e-3 * l.row) * k : 4.0 + 9.5e-3 * k;
+}
+
+struct PhasedLoad {  // the systems that the per-phase kernels would advance
+    int64_t systems = 0, particles = 0;
+    bool rigid = false;
+    void add(int64_t n, bool is_rigid) {
+        ++systems;
+        particles += n;
+        rigid = rigid || is_rigid;
+    }
+    // (a rigid step has more launches: some 65 us with a few small systems)
+    double us() const {
+        return LEAST + 2.2 * std::log2((double)std::max<int64_t>(systems, 1)) +
+               1.6e-4 * (double)particles + (rigid ? 40.0 : 0.0);
+    }
+    // systems whose resident step takes no longer than this are resident whatever else runs
+    static constexpr double LEAST = 24.0;
+};
 
 // The resident systems' table from (system, particles) pairs: class by class.  The stream is
 // idle with respect to the table's readers.
@@ -2260,6 +2296,8 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
     const BJam J = jam_constants(P);
     // every system starts minimizeFire (decompression phase) with a fresh list
     std::vector<std::pair<int, int64_t>> resident;
+    std::vector<double> cost(b->nsys, -1.0);  // of a resident step (< 0: not resident)
+    PhasedLoad load;
     for (int64_t s = 0; s < b->nsys; ++s) {
         BSys& S = b->hsys[s];
         BSys f{};
@@ -2281,9 +2319,18 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
         f.jphase = min_only ? BJ_MIN : BJ_DECOMP;
         f.status = 1;
         f.L_low = f.L_high = f.L_last = -1;
-        f.res = resident_size(b, f.n, b->nv[s] > 0, fastdiv) ? 1 : 0;
-        if (f.res) resident.push_back({(int)s, f.n});
+        if (!resident_size(b, f.n, b->nv[s] > 0, fastdiv)) {
+            load.add(f.n, b->nv[s] > 0);
+        } else {
+            cost[s] = resident_us(b, f.n, b->box0[s], b->rmin[s], b->rmax[s]);
+            if (!(cost[s] <= PhasedLoad::LEAST)) load.add(f.n, false);
+        }
         S = f;
+    }
+    for (int64_t s = 0; s < b->nsys; ++s) {
+        BSys& S = b->hsys[s];
+        S.res = cost[s] >= 0.0 && cost[s] <= load.us() ? 1 : 0;
+        if (S.res) resident.push_back({(int)s, S.n});
     }
     b->phased = (int64_t)resident.size() < b->nsys;
     if (resident_table(b, resident)) return -1;
@@ -2590,6 +2637,8 @@ struct dpm_server_req {
     int sys = -1;
     long long off = -1, slots = 0, voff = -1, vslots = 0;
     int64_t bytes = 0;
+    double res_us = -1.0;   // its step's cost if resident (< 0: cannot be)
+    bool resident = false;  // it is (running)
 };
 
 // Locking: `mu` guards the request table, the queue and every counter; the batch (arena,
@@ -2626,15 +2675,19 @@ static int serve_upload_tiles(dpm_server* sv) {
     }
     std::vector<int2> ct;
     std::vector<std::pair<int, int64_t>> resident;
-    b->phased = false;
+    b->phased = b->slow_phased = false;
     bool large = false;
     for (size_t s = 0; s < sv->sys_req.size(); ++s) {
         if (!sv->sys_req[s]) continue;
         const dpm_server_req& q = sv->reqs.at(sv->sys_req[s]);
         cell_tiles(ct, (int)s, (int)q.n);
         large = large || q.n > BC_MAX_N;
-        if (resident_size(b, q.n, q.kind == DPM_BUMPY, true)) resident.push_back({(int)s, q.n});
-        else b->phased = true;
+        if (q.resident) {
+            resident.push_back({(int)s, q.n});
+        } else {
+            b->phased = true;
+            b->slow_phased = b->slow_phased || q.res_us < 0.0;
+        }
     }
     if (large != b->large) {  // the step's launches change
         drop_graph(b);
@@ -2799,7 +2852,7 @@ static int serve_place(dpm_server* sv, dpm_server_req& q, int s) {
     f.jphase = q.mode == DPM_REQ_MINIMIZE ? BJ_MIN : BJ_DECOMP;
     f.status = 1;
     f.L_low = f.L_high = f.L_last = -1;
-    f.res = resident_size(b, q.n, rigid, true) ? 1 : 0;
+    f.res = q.resident ? 1 : 0;
     BCOPY(d.sys + s, &f, sizeof(BSys), hipMemcpyHostToDevice);
     return 0;
 }
@@ -2807,6 +2860,15 @@ static int serve_place(dpm_server* sv, dpm_server_req& q, int s) {
 // Queued requests that fit join the arena.
 static int serve_admit(dpm_server* sv) {
     bool tiles_changed = false;
+    PhasedLoad load;  // of what runs and what is queued
+    load.rigid = sv->b->nvslot > 0;  // (the launches are there for a vertex arena)
+    auto count = [&load](const dpm_server_req& q) {
+        if (!(q.res_us >= 0.0 && q.res_us <= PhasedLoad::LEAST))
+            load.add(q.n, q.kind == DPM_BUMPY);
+    };
+    for (int64_t id : sv->sys_req)
+        if (id) count(sv->reqs.at(id));
+    for (int64_t id : sv->queue) count(sv->reqs.at(id));
     for (auto it = sv->queue.begin(); it != sv->queue.end();) {
         dpm_server_req& q = sv->reqs.at(*it);
         if (sv->used + q.bytes > sv->budget || sv->free_sys.empty()) {
@@ -2829,6 +2891,7 @@ static int serve_admit(dpm_server* sv) {
         q.off = off;
         q.voff = voff;
         q.state = 1;
+        q.resident = q.res_us >= 0.0 && q.res_us <= load.us();
         sv->used += q.bytes;
         sv->sys_req[s] = q.id;
         sv->active++;
@@ -2957,6 +3020,9 @@ int64_t dpm_server_submit(dpm_server* sv, const dpm_request* r) try {
             set_error("dpm_server_submit: disk requests share the server's contact energy");
             return -1;
         }
+        const auto r_range = std::minmax_element(q.r.begin(), q.r.end());
+        if (resident_size(sv->b, q.n, false, true))
+            q.res_us = resident_us(sv->b, q.n, q.side, *r_range.first, *r_range.second);
     } else {
         if (!r->angle || !r->vertices_per_particle ||
             !(r->vertex_radius >= 0x1p-100 && r->vertex_radius <= 0x1p100) ||
@@ -3017,9 +3083,9 @@ int dpm_server_progress(dpm_server* sv, int64_t batched_steps, int64_t* finished
         active = sv->active;
     }
     if (active > 0 && batched_steps > 0) {
-        // the resident systems run their steps beside the others', and as a step of theirs is
-        // the shorter one, RES_PACE steps for each
-        const int64_t pace = b->phased ? RES_PACE : 1;
+        // the resident systems run their steps beside the others', RES_PACE steps for each of a
+        // rigid or large system, whose step is the longer one
+        const int64_t pace = b->slow_phased ? RES_PACE : 1;
         if (resident_launch(b, 0, std::min<int64_t>(batched_steps, INT_MAX / pace) * pace))
             return -1;
         int64_t done = b->phased ? 0 : batched_steps;

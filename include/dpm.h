@@ -314,8 +314,8 @@ int dpm_batch_autotune_shape(dpm_batch* b, const dpm_jam_params* p, int64_t tria
  * budget allows -- each joins the running batch of the batched engine, whose arena holds
  * arena_slots particle slots, vertex_slots vertex slots (rigid bumpy requests; 0: the
  * server takes none) and max_systems systems -- advances the batch by batched_steps and
- * collects finished requests.  (Beside rigid systems, a disk system of up to 4,096 particles,
- * whose steps are shorter, may take up to four times as many.)
+ * collects finished requests.  (Beside rigid systems, or disk systems above 4,096 particles, a
+ * smaller disk system, whose steps are shorter, may take up to four times as many.)
  * Disk requests share the server's pair law (e_c = 1, n_c = 2, Verlet cutoff 1.7, rebuild at
  * 3 max d^2 > 3 (0.15)^2); a rigid bumpy request brings its own e_c and follows the rigid
  * rules of dpm_batch_set_rigid_system (rotation on).  A DPM_REQ_JAM request's result
