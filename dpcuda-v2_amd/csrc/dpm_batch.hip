@@ -1644,9 +1644,9 @@ static BJam jam_constants(const dpm_jam_params* P) {
     return J;
 }
 
-// Steps of one launch of resident systems with no other system in the batch: some tens of
-// milliseconds, so that a finished batch is noticed soon and a launch's end, where the large
-// systems run alone, weighs little.
+// Steps of one launch of resident systems, with no other system in the batch or in the serving
+// loop: some tens of milliseconds, so that a finished batch is noticed soon and a launch's end,
+// where the large systems run alone, weighs little.
 constexpr int64_t RES_STEPS = 4096;
 
 // Serving loop: steps of a resident system for each batched step of the systems on the per-phase
@@ -3086,21 +3086,38 @@ int dpm_server_progress(dpm_server* sv, int64_t batched_steps, int64_t* finished
         // the resident systems run their steps beside the others', RES_PACE steps for each of a
         // rigid or large system, whose step is the longer one
         const int64_t pace = b->slow_phased ? RES_PACE : 1;
-        if (resident_launch(b, 0, std::min<int64_t>(batched_steps, INT_MAX / pace) * pace))
-            return -1;
-        int64_t done = b->phased ? 0 : batched_steps;
-        while (done < batched_steps) {
-            int64_t k = std::min<int64_t>(b->steps_per_graph, batched_steps - done);
-            if (b->use_graph && k == b->steps_per_graph) {
-                if (ensure_batch_graph(b, k)) return -1;
-                DPM_HIP(hipGraphLaunch(b->exec, b->stream));
-            } else {
-                for (int64_t s = 0; s < k; ++s) enqueue_batch_step(b);
-                if (check_launch()) return -1;
+        // In pieces, so that no launch holds its CUs for long and a call of many steps ends once
+        // everything has finished: two pieces in flight, each with a copy of the flags.
+        int64_t piece = 0;
+        for (int64_t done = 0; done < batched_steps; ++piece) {
+            if (piece >= 2) {
+                const int ws = (int)(piece % 2);  // the piece before the last
+                DPM_HIP(hipEventSynchronize(b->poll[ws]));
+                const int* f = b->hflags + 4 * ws;
+                if (f[0] || f[2] - sv->seen_done >= active) break;
             }
-            done += k;
+            const int64_t steps = std::min<int64_t>(batched_steps - done, RES_STEPS / pace);
+            if (resident_launch(b, 0, steps * pace)) return -1;
+            for (int64_t sent = 0; b->phased && sent < steps;) {
+                const int64_t k = std::min<int64_t>(b->steps_per_graph, steps - sent);
+                if (b->use_graph && k == b->steps_per_graph) {
+                    if (ensure_batch_graph(b, k)) return -1;
+                    DPM_HIP(hipGraphLaunch(b->exec, b->stream));
+                } else {
+                    for (int64_t s = 0; s < k; ++s) enqueue_batch_step(b);
+                    if (check_launch()) return -1;
+                }
+                sent += k;
+            }
+            if (resident_join(b)) return -1;
+            done += steps;
+            if (done < batched_steps) {
+                const int ws = (int)(piece % 2);
+                DPM_HIP(hipMemcpyAsync(b->hflags + 4 * ws, b->d.flags, 4 * sizeof(int),
+                                       hipMemcpyDeviceToHost, b->stream));
+                DPM_HIP(hipEventRecord(b->poll[ws], b->stream));
+            }
         }
-        if (resident_join(b)) return -1;
         DPM_HIP(hipStreamSynchronize(b->stream));
         std::lock_guard<std::mutex> g(sv->mu);
         if (serve_collect(sv) || serve_admit(sv)) return -1;
