@@ -185,7 +185,7 @@ __global__ __launch_bounds__(T) void k_b_resident(BDev b, const int* ids, long l
     __syncthreads();
     PairParams p = res_params(b, S);
     const double thr2 = uniform_d(S.thr2);
-    const double delta2 = 2.0 * sqrt(fmax(thr2, 0.0) / 3.0);
+    const double delta2 = res_reach(thr2);
     // the near rows of the list that the last launch left, in the present box
     auto load_near = [&](bool any) {
 #pragma unroll

@@ -51,7 +51,7 @@ __global__ __launch_bounds__(T) void k_resident(Dev d, Spare sp, PairParams p, N
     const int n = (int)d.N, nc = (n + WAVE - 1) / WAVE;
     const bool cells = nb.method == DPM_NBR_CELL;
     const int ncell = cells ? (int)nb.ncells : 0;
-    const double delta2 = 2.0 * sqrt(fmax(nb.thr, 0.0) / 3.0);
+    const double delta2 = res_reach(nb.thr);
     const ResRows R{d.nbr, (long long)d.N, 0, d.cap};
     ResKept<T, NP> K;
     K.row = rows;

@@ -220,6 +220,12 @@ __device__ __forceinline__ void res_sort(ResCore<T, NP>& L, int n, int ncell,
     __syncthreads();
 }
 
+// 2 delta: how much nearer two particles can come before 3 d^2 > thr asks for a rebuild (an
+// undefined threshold never does: every listed pair is near)
+__device__ __forceinline__ double res_reach(double thr) {
+    return 2.0 * sqrt((thr < 0.0 ? 0.0 : thr) / 3.0);
+}
+
 // Whether a pair listed at reference positions a, b can touch before the next rebuild.  The
 // bound is widened by the rounding of the coordinates; a NaN keeps the entry.  (a, b) and (b, a)
 // have the same answer to the bit: near rows are symmetric where the full rows are.
