@@ -1475,6 +1475,7 @@ struct dpm_batch {
     int rrows_for[dpm::RES_CLASSES - dpm::RES_ROWS] = {0, 0};
     int rcount[dpm::RES_CLASSES] = {};
     bool phased = true;  // some system is advanced by the per-phase kernels
+    bool phased_disks = true;  // and is a disk system (dpm_batch_jam, dpm_batch_minimize)
     bool slow_phased = false;  // and is rigid or above RES_MAX_N (serving loop)
     hipStream_t rstream[dpm::RES_CLASSES] = {};
     hipEvent_t rfork = nullptr, rjoin[dpm::RES_CLASSES] = {};
@@ -2327,10 +2328,12 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
         }
         S = f;
     }
+    b->phased_disks = false;
     for (int64_t s = 0; s < b->nsys; ++s) {
         BSys& S = b->hsys[s];
         S.res = cost[s] >= 0.0 && cost[s] <= load.us() ? 1 : 0;
         if (S.res) resident.push_back({(int)s, S.n});
+        else if (b->nv[s] == 0) b->phased_disks = true;
     }
     b->phased = (int64_t)resident.size() < b->nsys;
     if (resident_table(b, resident)) return -1;
@@ -2487,7 +2490,7 @@ extern "C" {
 
 // Autotuner: runs `trial_steps` batched steps of the jam from the configured state for
 // every (cutoff, steps per launch) pair, restores the state after each trial, and keeps
-// the fastest pair.  Neither choice changes any result bit (rows only add listed
+// the fastest pair (the first length where every system is resident and none matters).  Neither choice changes any result bit (rows only add listed
 // non-contacts, which contribute +0.0; launch grouping is not visible to the systems).
 int dpm_batch_autotune(dpm_batch* b, const dpm_jam_params* P, int64_t trial_steps,
                        const double* cutoffs, int n_cutoffs, const int64_t* chunks,
@@ -2531,6 +2534,7 @@ int dpm_batch_autotune(dpm_batch* b, const dpm_jam_params* P, int64_t trial_step
                 bc = cutoffs[i];
                 bk = chunks[j];
             }
+            if (!b->phased) break;  // resident systems alone: no launch takes this length
         }
     }
     if (best == 1e300) {
@@ -2553,7 +2557,8 @@ int dpm_batch_autotune(dpm_batch* b, const dpm_jam_params* P, int64_t trial_step
 
 // Launch shape: the force pass's workgroup size (64, 128 or 256 slots) and the cell-grid
 // build's cell width (100, 125 or 150 % of the cutoff), tried one after the other with
-// the current cutoff and steps per launch.  Neither changes a result bit: the force pass
+// the current cutoff and steps per launch.  The workgroup size stays as it is where no disk system
+// takes the force pass.  Neither changes a result bit: the force pass
 // is per slot, and cells at least the cutoff wide give the same rows.
 int dpm_batch_autotune_shape(dpm_batch* b, const dpm_jam_params* P, int64_t trial_steps,
                              int64_t* best_block, int64_t* best_cell_pct,
@@ -2564,25 +2569,29 @@ int dpm_batch_autotune_shape(dpm_batch* b, const dpm_jam_params* P, int64_t tria
     }
     if (tune_begin(b)) return -1;
     double best = 1e300;
-    int bb = b->force_block, bp = b->cell_pct;
-    for (int blk : {64, 128, 256}) {
-        b->force_block = blk;
+    const int block0 = b->force_block;
+    int bb = block0, bp = b->cell_pct;
+    auto trial = [&](int& best_value, int value) {
         double ms;
         if (tune_trial(b, P, trial_steps, &ms)) return -1;
         if (ms < best) {
             best = ms;
-            bb = blk;
+            best_value = value;
         }
+        return 0;
+    };
+    for (int blk : {64, 128, 256}) {
+        b->force_block = blk;
+        if (trial(bb, blk)) return -1;
+        if (b->phased_disks) continue;
+        bb = block0;  // no system takes the force pass: nothing to choose
+        best = 1e300;
+        break;
     }
     b->force_block = bb;
     for (int pct : {100, 125, 150}) {
         b->cell_pct = pct;
-        double ms;
-        if (tune_trial(b, P, trial_steps, &ms)) return -1;
-        if (ms < best) {
-            best = ms;
-            bp = pct;
-        }
+        if (trial(bp, pct)) return -1;
     }
     b->cell_pct = bp;
     if (tune_end(b)) return -1;

@@ -235,7 +235,9 @@ int dpm_bumpy_setup(dpm_system* s, const int64_t* n_vertices_per_particle, doubl
  * result is bit-identical to dpm_jam on a dpm_system holding the same particles with the
  * Verlet method, cutoff and threshold given here.
  * dpm_batch_config: pair law (e_c, n_c), Verlet cutoff and rebuild threshold (3 max d^2 >
- * disp_thresh_sq), common to all systems.  dpm_batch_jam: out[] has n_systems entries;
+ * disp_thresh_sq), common to all systems.  Small disk systems, and many of up to 4,096
+ * particles, are each advanced by one workgroup in launches of many steps ("resident"), the
+ * others by a sequence of kernels per step; results do not depend on it.  dpm_batch_jam: out[] has n_systems entries;
  * status -1 marks a system still running after max_batched_steps; steps_done returns the
  * batched steps executed.  dpm_batch_set_option takes DPM_OPT_GRAPH, DPM_OPT_CHUNK
  * (batched steps per graph launch) and DPM_OPT_TIMING. */
@@ -280,8 +282,8 @@ int dpm_batch_minimize(dpm_batch* b, const dpm_fire_params* p, int64_t max_batch
 /* the batched step (1-based) in which each system finished its last dpm_batch_jam, -1 if
  * it has not */
 int dpm_batch_finish_steps(dpm_batch* b, int64_t* steps_out);
-/* Measurement: with dpm_batch_set_option(b, DPM_OPT_TIMING, 1) every batched step is
- * launched eagerly with HIP events around its force pass (the disk pass k_b_force, or the
+/* Measurement: with dpm_batch_set_option(b, DPM_OPT_TIMING, 1) no system is resident, and every
+ * batched step is launched eagerly with HIP events around its force pass (the disk pass k_b_force, or the
  * rigid pass k_rb_force in a batch of rigid systems only); dpm_batch_kernel_time returns
  * the summed milliseconds and the number of timed passes since the option was set.
  * dpm_batch_row_entries: the stored neighbour-row entries of every system's particles. */
@@ -294,7 +296,8 @@ int dpm_batch_vertex_row_entries(dpm_batch* b, int64_t* total);
 /* Autotuner: times trial_steps batched steps of dpm_batch_jam for every pair of a Verlet
  * cutoff (rebuild threshold: half its skin) and a number of steps per graph launch,
  * restoring the configured state after each trial, and keeps the fastest pair.  Neither
- * choice changes a result bit. */
+ * choice changes a result bit.  Where every system is resident, the number of steps has no
+ * effect and the first candidate is kept. */
 int dpm_batch_autotune(dpm_batch* b, const dpm_jam_params* p, int64_t trial_steps,
                        const double* cutoffs, int n_cutoffs, const int64_t* chunks,
                        int n_chunks, double* best_cutoff, int64_t* best_chunk,
@@ -303,7 +306,8 @@ int dpm_batch_autotune(dpm_batch* b, const dpm_jam_params* p, int64_t trial_step
  * batched steps for each force-pass workgroup size (64, 128, 256), keeps the fastest, then
  * for each cell width of the cell-grid rows (100, 125, 150 % of the cutoff), restoring the
  * configured state after each trial; the choices stay set (DPM_OPT_FORCE_BLOCK,
- * DPM_OPT_CELL_PCT). */
+ * DPM_OPT_CELL_PCT).  Where no disk system takes the force pass (resident or rigid systems
+ * only) its workgroup size stays as set. */
 int dpm_batch_autotune_shape(dpm_batch* b, const dpm_jam_params* p, int64_t trial_steps,
                              int64_t* best_block, int64_t* best_cell_pct,
                              double* best_ms_per_step);
