@@ -54,8 +54,9 @@
 //               the closing kick and the chunk partials
 //   k_rb_eval   per particle (a half-wave over its vertices), before k_b_eval: the
 //               stress and contacts of a rigid system that finished a minimisation
-// Disk systems of up to RES_MAX_N particles take none of these launches: k_b_resident
-// (dpm_batch_resident.hpp) runs all their phases in one workgroup, many steps a launch.
+// Disk systems of up to RES_MAX_N particles for which one CU is fast enough (resident_us) take none
+// of these launches: k_b_resident (dpm_batch_resident.hpp) runs all their phases in one
+// workgroup, many steps a launch.
 #include <algorithm>
 #include <chrono>
 #include <climits>
@@ -545,8 +546,9 @@ __global__ __launch_bounds__(BC_BLOCK) void k_b_build_cells(BDev b) {
 }
 
 // kernelUpdateNeighborList (base/kernels.cu:256-293) for the systems of more than BC_MAX_N
-// particles that need it (launched when there is one): every other particle of the system with d^2 < rc^2, ascending index.  One block per
-// 256-slot tile of a system; the system's positions pass through LDS.
+// particles that need it (launched when there is one): every other particle of the system with
+// d^2 < rc^2, ascending index.  One block per 256-slot tile of a system; the system's positions
+// pass through LDS.
 __global__ __launch_bounds__(BLOCK) void k_b_build(BDev b) {
     if ((int)blockIdx.x >= b.flags[4]) return;
     const int2 t = b.tiles[blockIdx.x];
@@ -1650,9 +1652,11 @@ static BJam jam_constants(const dpm_jam_params* P) {
 // where the large systems run alone, weighs little.
 constexpr int64_t RES_STEPS = 4096;
 
-// Serving loop: steps of a resident system for each batched step of the systems on the per-phase
-// kernels (some 90 us a step; a resident step takes 4 us at 256 particles, 33 us at 4,096).
-// With one for one, a burst's disk jams waited for its rigid minimisations most of their time.
+// Serving loop: steps of a resident system for each batched step of rigid or larger systems on the
+// per-phase kernels (some 90 us a step; a resident step takes 4 us at 256 particles, 33 us of a
+// jam at 4,096).  With one for one, a burst's disk jams waited for its rigid minimisations most
+// of their time (a burst of 24 jams and 8 minimisations 205 ms, 141 with four for one; such a
+// burst spreads, 185 to 250 ms over processes with the seed of its arrivals).
 constexpr int64_t RES_PACE = 4;
 
 static hipEvent_t batch_event(dpm_batch* b) {
@@ -2490,8 +2494,9 @@ extern "C" {
 
 // Autotuner: runs `trial_steps` batched steps of the jam from the configured state for
 // every (cutoff, steps per launch) pair, restores the state after each trial, and keeps
-// the fastest pair (the first length where every system is resident and none matters).  Neither choice changes any result bit (rows only add listed
-// non-contacts, which contribute +0.0; launch grouping is not visible to the systems).
+// the fastest pair (the first length where every system is resident and none matters).
+// Neither choice changes any result bit (rows only add listed non-contacts, which contribute
+// +0.0; launch grouping is not visible to the systems).
 int dpm_batch_autotune(dpm_batch* b, const dpm_jam_params* P, int64_t trial_steps,
                        const double* cutoffs, int n_cutoffs, const int64_t* chunks,
                        int n_chunks, double* best_cutoff, int64_t* best_chunk,

@@ -9,11 +9,13 @@
 // moves no particle data through HBM.
 // Up to 2,048 particles LDS holds the pairs that can touch, each evaluated once; beyond, it holds
 // positions and radii and the near rows are walked (dpm_resident.hpp).
-// What bounds it: LDS gathers and the vector pipe of its CU, and for small systems the chain of
-// a step's phases.
+// What bounds it: the vector pipe of its CU (busy 55 to 58 % of the time from 512 particles up, LDS
+// 7 to 10 %) and the chain of a step's phases, in which waves wait 57 to 74 % of their time.
 // Measured, 64 systems jammed, ms (full rows walked from both sides, as it is now): up to 256
-// particles 48, 35; 512 63, 47; 1,024 95, 64; 2,048 167, 123; 4,096 397, 308.  384 systems of 64 to 2,048 particles
-// (log-uniform): 708 ms on the per-phase kernels (seven launches a step), 203, 157.
+// particles 48, 35; 512 63, 47; 1,024 95, 64; 2,048 167, 123; 4,096 397, 308.  384 systems of 64
+// to 2,048 particles (log-uniform): 708 ms on the per-phase kernels (seven launches a step), 203,
+// 157.  4,096 systems of 16 particles leave most of their threads idle: 200 FIRE steps 10.6 ms,
+// 9.9 on the per-phase kernels.
 constexpr int RES_MAX_N = 4096;
 
 // The size classes: a wave or more per SIMD from 256 particles up; systems of more than 512

@@ -541,11 +541,11 @@ __global__ void k_bumpy_init_vertices(Dev d, double rv) {
 //   k_bfire_vertices  vertices: the rotations of those moves, in the same order; one thread
 //                     makes the neighbour check of the step: a list rebuild runs inside the
 //                     chunk
-//   k_build_cell / k_build_verlet, k_bumpy_vertex_build   (gated on that decision)
+//   k_build_cell / k_build_verlet, k_bumpy_vertex_rows    (gated on that decision)
 //   k_bfire_forces    a step that needs a cell rebuild, or whose rebuilt rows overflowed the
-//                     capacity, halts the loop until the chunk's end; else vertex forces, torques, energies (kernelCalcRigidBumpyForces1)
-//                     and their per-particle sums (kernelCalcRigidBumpyParticleForces1),
-//                     one pass
+//                     capacity, halts the loop until the chunk's end; else vertex forces,
+//                     torques, energies (kernelCalcRigidBumpyForces1) and their per-particle
+//                     sums (kernelCalcRigidBumpyParticleForces1), one pass
 //   k_bfire_partials  kick(dt/2), then the chunk partials of P = F.v + tau.w, PE and
 //                     max(F^2, tau^2)
 //   k_fire_ctl        stop test of the step and Fire::step's decision for the next
@@ -672,8 +672,9 @@ __global__ void k_bfire_check(Dev d, int pos, int gate) {
 //   k_bnve_vertices  the vertices' rotation; one thread decides the list rebuild
 //   list and vertex-row builds (gated on that decision), k_bfire_forces
 // with the closing kick of a chunk's last step in k_bnve_kick.  Halts, the rebuild chain and
-// the capacity's regrowth are those of the rigid FIRE loop.  Bound by launch latency up to some thousand particles: 3,001 particles, 200 steps take 5.6 ms (27.5 ms with
-// a dozen stand-alone launches and a blocking readback per step).
+// the capacity's regrowth are those of the rigid FIRE loop.  Bound by launch latency up to some
+// thousand particles: 200 steps of 3,001 particles take 4.7 ms (26.1 ms with a dozen stand-alone
+// launches and a blocking readback per step).
 __device__ __forceinline__ void rigid_kick(double2& v, double& w, double2 f, double t, double moi,
                                            double m, double hdt, int rotation) {
     // kernelUpdateRigidVelocities, rigid_bumpy/kernels.cu:123-150

@@ -1218,7 +1218,7 @@ __global__ void k_ctl_reset(Dev d, int config) {
 //   k_fire_move   : [uphill back-step, v=0] + kick(dt/2) + mix + drift(dt)
 //   k_fire_force  : zero + forces + kick(dt/2) + chunk partials of P, PE, |F|max
 //   k_fire_ctl    : canonical sums, minimizeFire's stop test for this step and
-//                   Fire::step's decision for the next (one wave)
+//                   Fire::step's decision for the next (one workgroup)
 // (Every load goes out before the control block is looked at, as in k_nve_fused.)
 __global__ __launch_bounds__(BLOCK) void k_fire_move(Dev d, NbrParams nb, int pos) {
     Ctl* c = d.ctl;

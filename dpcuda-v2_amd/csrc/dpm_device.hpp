@@ -156,7 +156,7 @@ __device__ __forceinline__ double pair_hot(double4 qi, double4 q, bool valid, co
     double fm = div_rn_normal(p.e_c * ov, rs * d);
     // Separations that the short sequences do not cover.  The whole wave branches: as a branch
     // of the lane the compiler folded it into selects, and every pair paid for the IEEE square
-    // root and two divisions (85 double precision instructions instead of 50).
+    // root and two divisions (85 double precision instructions instead of 46).
     const bool tiny = contact && d2 < 0x1p-700;
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(tiny) != 0, 0)) {
         if (tiny) {

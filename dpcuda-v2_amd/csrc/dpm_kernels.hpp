@@ -172,8 +172,8 @@ __device__ __forceinline__ bool within(double ax, double ay, double bx, double b
 
 // The candidates of a particle in cell (cx, cy) of a grid of nx x ny >= 3 x 3 cells, for lanes
 // that test them side by side: the list entries of the 3 x 3 cells around it, rows and cells of
-// a row in ascending order, which are one run in each row of cells, or two where the row wraps.  range(c0, c1, a, e) gives the entries
-// [a, e) of cells c0 to c1.
+// a row in ascending order, which are one run in each row of cells, or two where the row wraps.
+// range(c0, c1, a, e) gives the entries [a, e) of cells c0 to c1.
 struct CellRuns {
     int a[6], m[6], count;
     template <class Range>

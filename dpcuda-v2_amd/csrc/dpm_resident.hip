@@ -6,9 +6,10 @@
 // workgroup barriers, lists and cells are rebuilt in place.  Arithmetic, row order, particle
 // order and the canonical reduction order are those of the chunked loops, so results are the
 // same bits.  A row that outgrows the ELL halts the step, which the rebuild chain then finishes.
-// What bounds it: the CU's LDS and vector pipe and the chain of a step's phases (2 barriers and
-// two LDS round trips for NVE, 4 barriers, a reduction and the decision for FIRE): 1.5 us a step
-// with 128 particles, where no pipe is busy, 3.4 us with 1,000.  Measured (before, after, ms):
+// What bounds it: one CU's vector pipe (busy 57 % of the time with 777 disks, LDS 10 %) and the
+// chain of a step's phases, in which its waves wait (2 barriers and two LDS round trips for NVE, 4
+// barriers, a reduction and the decision for FIRE): 1.5 us a step with 128 particles, where no
+// pipe is busy, 3.4 us with 1,000.  Measured (before, after, ms):
 // 1,024 disks, 1000 NVE steps 5.9, 3.5; 777 disks, 2000 FIRE steps 38.6, 12.4.
 #include "dpm_resident.hpp"
 

@@ -1,7 +1,7 @@
 // dpm_resident.hpp -- a disk system of up to 4,096 particles held in one workgroup: positions,
 // radii and (up to 2,048) the list of pairs in LDS, the rest of a particle's state in the
-// registers of its thread.  Shared by the single-system loops (dpm_resident.hip) and the batched engine
-// (dpm_batch_resident.hpp).
+// registers of its thread.  Shared by the single-system loops (dpm_resident.hip) and the batched
+// engine (dpm_batch_resident.hpp).
 //
 // Near pairs.  The full rows (every particle within the list cutoff, what queries and the other
 // kernels read) go to the ELL in HBM; LDS holds the pairs that can touch before the list is next

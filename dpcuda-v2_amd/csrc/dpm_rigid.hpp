@@ -129,9 +129,9 @@ struct RingEntry {
 // Without it (boxes of a few diameters) every vertex is tested by its own image, and all of them
 // are candidates: another image of the ring than its centre's nearest may be within vc of v, and
 // the window looks at the nearest alone.
-// What bounds it: the vector pipe (some 450 instructions a wave; the entries' fields came by
-// cross-lane reads before: 82 us, now 70 us a build at 65,536
-// particles of 24 vertices).
+// What bounds it: the gathers of the row entries and of their rings' vertices (halving the vector
+// instructions, by fields in LDS instead of cross-lane reads, took a build of 65,536 particles of
+// 24 vertices from 82 us to 70).
 template <bool SHIFT, class Box, class Entry, class Emit>
 __device__ __forceinline__ int vertex_row(const Box& bx, const double4* P, const int* vst,
                                           const int* nvt, const double2* vpos, double rv,

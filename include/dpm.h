@@ -237,9 +237,9 @@ int dpm_bumpy_setup(dpm_system* s, const int64_t* n_vertices_per_particle, doubl
  * dpm_batch_config: pair law (e_c, n_c), Verlet cutoff and rebuild threshold (3 max d^2 >
  * disp_thresh_sq), common to all systems.  Small disk systems, and many of up to 4,096
  * particles, are each advanced by one workgroup in launches of many steps ("resident"), the
- * others by a sequence of kernels per step; results do not depend on it.  dpm_batch_jam: out[] has n_systems entries;
- * status -1 marks a system still running after max_batched_steps; steps_done returns the
- * batched steps executed.  dpm_batch_set_option takes DPM_OPT_GRAPH, DPM_OPT_CHUNK
+ * others by a sequence of kernels per step; results do not depend on it.
+ * dpm_batch_jam: out[] has n_systems entries; status -1 marks a system still running after
+ * max_batched_steps; steps_done returns the batched steps executed.  dpm_batch_set_option takes DPM_OPT_GRAPH, DPM_OPT_CHUNK
  * (batched steps per graph launch) and DPM_OPT_TIMING. */
 typedef struct dpm_batch dpm_batch;
 dpm_batch* dpm_batch_create(int64_t n_systems, const int64_t* n_particles);
@@ -283,9 +283,9 @@ int dpm_batch_minimize(dpm_batch* b, const dpm_fire_params* p, int64_t max_batch
  * it has not */
 int dpm_batch_finish_steps(dpm_batch* b, int64_t* steps_out);
 /* Measurement: with dpm_batch_set_option(b, DPM_OPT_TIMING, 1) no system is resident, and every
- * batched step is launched eagerly with HIP events around its force pass (the disk pass k_b_force, or the
- * rigid pass k_rb_force in a batch of rigid systems only); dpm_batch_kernel_time returns
- * the summed milliseconds and the number of timed passes since the option was set.
+ * batched step is launched eagerly with HIP events around its force pass (the disk pass
+ * k_b_force, or the rigid pass k_rb_force in a batch of rigid systems only);
+ * dpm_batch_kernel_time returns the summed milliseconds and the number of timed passes since the option was set.
  * dpm_batch_row_entries: the stored neighbour-row entries of every system's particles. */
 int dpm_batch_kernel_time(dpm_batch* b, double* force_ms, int64_t* launches);
 int dpm_batch_row_entries(dpm_batch* b, int64_t* total);
