@@ -1795,10 +1795,14 @@ struct PhasedLoad {  // the systems that the per-phase kernels would advance
 static int resident_table(dpm_batch* b, const std::vector<std::pair<int, int64_t>>& systems) {
     if (!b->rids && balloc_n(b, &b->rids, b->nsys)) return -1;
     std::vector<int> ids;
+    const bool crowd = std::count_if(systems.begin(), systems.end(), [](auto& e) {
+                           return e.second <= RES_LIMIT[0];
+                       }) > RES_CROWD;
     for (int c = 0; c < RES_CLASSES; ++c) {
         const size_t before = ids.size();
+        const int64_t above = c == 0 || (c == 1 && !crowd) ? 0 : RES_LIMIT[c - 1];
         for (auto& e : systems)
-            if (e.second <= RES_LIMIT[c] && (c == 0 || e.second > RES_LIMIT[c - 1]))
+            if (e.second <= RES_LIMIT[c] && e.second > above && (c > 0 || crowd))
                 ids.push_back(e.first);
         b->rcount[c] = (int)(ids.size() - before);
     }
@@ -1844,13 +1848,15 @@ static int resident_launch(dpm_batch* b, int64_t base, int64_t steps) {
         const long long b0 = base;
         const int k = (int)steps;
         switch (c) {
-            case 0: hipLaunchKernelGGL((k_b_resident<512, 256>), grid, dim3(512), 0, st, b->d, ids,
+            case 0: hipLaunchKernelGGL((k_b_resident<128, 128>), grid, dim3(128), 0, st, b->d, ids,
                                        b0, k, nullptr); break;
-            case 1: hipLaunchKernelGGL((k_b_resident<1024, 512>), grid, dim3(1024), 0, st, b->d, ids,
+            case 1: hipLaunchKernelGGL((k_b_resident<512, 256>), grid, dim3(512), 0, st, b->d, ids,
                                        b0, k, nullptr); break;
-            case 2: hipLaunchKernelGGL((k_b_resident<1024, 1024>), grid, dim3(1024), 0, st, b->d,
+            case 2: hipLaunchKernelGGL((k_b_resident<1024, 512>), grid, dim3(1024), 0, st, b->d, ids,
+                                       b0, k, nullptr); break;
+            case 3: hipLaunchKernelGGL((k_b_resident<1024, 1024>), grid, dim3(1024), 0, st, b->d,
                                        ids, b0, k, nullptr); break;
-            case 3: hipLaunchKernelGGL((k_b_resident<1024, 2048>), grid, dim3(1024), 0, st, b->d,
+            case 4: hipLaunchKernelGGL((k_b_resident<1024, 2048>), grid, dim3(1024), 0, st, b->d,
                                        ids, b0, k, b->rrows[0]); break;
             default: hipLaunchKernelGGL((k_b_resident<1024, 4096>), grid, dim3(1024), 0, st, b->d,
                                         ids, b0, k, b->rrows[1]);

@@ -14,15 +14,19 @@
 // Measured, 64 systems jammed, ms (full rows walked from both sides, as it is now): up to 256
 // particles 48, 35; 512 63, 47; 1,024 95, 64; 2,048 167, 123; 4,096 397, 308.  384 systems of 64
 // to 2,048 particles (log-uniform): 708 ms on the per-phase kernels (seven launches a step), 203,
-// 157.  4,096 systems of 16 particles leave most of their threads idle: 200 FIRE steps 10.6 ms,
-// 9.9 on the per-phase kernels.
+// 157.
 constexpr int RES_MAX_N = 4096;
 
 // The size classes: a wave or more per SIMD from 256 particles up; systems of more than 512
-// particles have a CU's LDS to themselves.
-constexpr int RES_CLASSES = 5;
-constexpr int RES_LIMIT[RES_CLASSES] = {256, 512, 1024, 2048, 4096};
-constexpr int RES_ROWS = 3;  // from this class on, the near rows lie in HBM
+// particles have a CU's LDS to themselves.  The first class is for more systems of its size than
+// there are CUs (RES_CROWD): its two waves leave room for several systems a CU, where the next
+// class's eight take them all.  us a FIRE step (row builds of a thread a row and the per-phase
+// kernels, class of 256, of 128): 1,024 systems of 16 disks 35, 16, 6.8; 16,384 of 16 157, 229,
+// 66; 8,192 of 64 128, 222, 53.
+constexpr int RES_CLASSES = 6;
+constexpr int RES_LIMIT[RES_CLASSES] = {128, 256, 512, 1024, 2048, 4096};
+constexpr int RES_CROWD = 256;
+constexpr int RES_ROWS = 4;  // from this class on, the near rows lie in HBM
 
 // bparams, held in scalar registers (every lane reads the same record)
 __device__ __forceinline__ PairParams res_params(const BDev& b, const BSys& S) {

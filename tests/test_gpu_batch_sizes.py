@@ -145,3 +145,48 @@ def test_served_systems_past_the_limits():
         got = sv.result(i)
         check(r, got["result"], got["x"], got["y"])
 
+
+
+CROWD = (1, 2, 9, 64, 127, 128, 129, 300)
+
+
+@pytest.mark.parametrize("count", (256, 257, 520))
+def test_crowds_of_small_systems(count):
+    """More small systems than CUs take the smallest class (and its neighbours the next)."""
+    kinds = [alone(n, 0.84, 60) for n in CROWD]
+    small = [r for r in kinds if r[0].n <= 128]
+    print("[gpu-case] crowd", count, flush=True)
+    minimise([small[k % len(small)] for k in range(count)] + kinds[-2:], 60)
+
+
+def test_crowd_jams_and_is_served():
+    prm = P.jam_params(pressure_target=1e-2, window_rel=0.5, strain_step=2e-2,
+                       max_compression_steps=8, fire=fire(40))
+    sts = [W.disk_config(n, 0.80, seed=n) for n in (20, 64, 100, 128)]
+    ref = []
+    for st in sts:
+        s = W.make_disk_system(P.System, st, W.neighbor_spec(st.side, method=P.NBR_VERLET),
+                               backend=oracle())
+        ref.append((s.jam(prm), s.download(P.F_X)))
+        s.close()
+    print("[gpu-case] crowd jams", flush=True)
+    b = P.Batch([sts[k % 4].n for k in range(300)])
+    sv = P.Server(max_systems=300, arena_slots=1 << 16, budget_bytes=1 << 30, vertex_slots=0)
+    ids = []
+    for k in range(300):
+        st = sts[k % 4]
+        b.set_system(k, st.x, st.y, st.rad, st.mass, st.side)
+        ids.append(sv.submit(st.x, st.y, st.rad, st.mass, st.side, prm))
+    res, _ = b.jam(prm)
+    while any(sv.progress(32)[1:]):  # (the crowd thins out: its systems change class)
+        pass
+    for k in range(300):
+        got = sv.result(ids[k])
+        for f in ("status", "compression_steps", "fire_steps_total", "pressure", "pe",
+                  "contacts"):
+            assert getattr(res[k], f) == getattr(ref[k % 4][0], f), (k, f)
+            assert getattr(got["result"], f) == getattr(ref[k % 4][0], f), (k, f)
+        assert np.array_equal(b.get_system(k)[0], ref[k % 4][1])
+        assert np.array_equal(got["x"], ref[k % 4][1])
+    b.close()
+    sv.close()
