@@ -37,8 +37,8 @@
 //               minimisation (Fire::step first half) and its displacement flags
 //   k_b_build_cells  the Verlet rows of the systems whose test (3 max d^2 > thr^2,
 //               b_rebuild_now) asks for them, from a cell grid in LDS
-//   k_b_build   the same by an O(n^2) pass for systems of more than 16,384 particles
-//               (launched when the arena holds one)
+//   k_b_build   the same by an O(n^2) pass for systems of more than 16,384 particles and
+//               for crowds of systems under 128 (launched when the arena holds such)
 //   k_b_force   forces (+ closing kick) and the chunk partials of P, PE, max F^2
 //   k_b_ctl     per system: minimizeFire's stop test and Fire::step's decision; clears
 //               the controller's applied requests and counts the step
@@ -146,7 +146,8 @@ struct BDev {
     // common parameters
     double n_c, ncm1, two_nc, inv2nc;
     double cell_scale;  // cell-grid cells: at least cell_scale * rc wide (>= 1)
-    int fastdiv, pad;
+    int fastdiv;
+    int crowd;          // systems under BC_MIN_N particles get their rows from k_b_build
     // rigid bumpy arena (nvslot = 0: none)
     long long nvslot;
     int vcap, pad2;
@@ -432,6 +433,7 @@ struct BCLds {
 
 __device__ __forceinline__ void bc_build_item(const BDev& b, int2 ct, BCLds& L) {
     const BSys& S = b.sys[ct.x];
+    if (b.crowd && S.n < BC_MIN_N) return;  // k_b_build builds this system
     if (!b_rebuild_now(b, S)) return;  // the same verdict in every wave of the workgroup
     BCGrid g;
     const bool grid = bc_grid(b, S, g);
@@ -546,14 +548,16 @@ __global__ __launch_bounds__(BC_BLOCK) void k_b_build_cells(BDev b) {
 }
 
 // kernelUpdateNeighborList (base/kernels.cu:256-293) for the systems of more than BC_MAX_N
-// particles that need it (launched when there is one): every other particle of the system with
-// d^2 < rc^2, ascending index.  One block per 256-slot tile of a system; the system's positions
-// pass through LDS.
+// particles that need it, and for a crowd of systems under BC_MIN_N (launched when there are
+// such): every other particle of the system with d^2 < rc^2, ascending index.  One block per
+// 256-slot tile of a system; the system's positions pass through LDS.  A crowd is more of them
+// than k_b_build_cells has workgroups (BC_GRID), whose turns add up.  us a FIRE step (there, here):
+// 1,024 systems of 16 rigid particles 272, 238; 4,096 of 16 994, 857; 2,048 of 64 721, 627.
 __global__ __launch_bounds__(BLOCK) void k_b_build(BDev b) {
     if ((int)blockIdx.x >= b.flags[4]) return;
     const int2 t = b.tiles[blockIdx.x];
     const BSys& S = b.sys[t.x];
-    if (S.n <= BC_MAX_N) return;   // k_b_build_cells builds this system
+    if (S.n <= BC_MAX_N && !(b.crowd && S.n < BC_MIN_N)) return;  // k_b_build_cells builds it
     if (!b_rebuild_now(b, S)) return;  // the same verdict in every wave of the block
     __shared__ double2 tp[BLOCK];
     const long long i = (long long)t.y + threadIdx.x;
@@ -1695,7 +1699,8 @@ static void enqueue_batch_step(dpm_batch* b) {
     dim3 vslots((unsigned)((b->nvslot + BLOCK - 1) / BLOCK));
     hipLaunchKernelGGL(k_b_prep_move, slots, dim3(BLOCK), 0, st, d);
     if (rigid) hipLaunchKernelGGL(k_rb_vmove, vslots, dim3(BLOCK), 0, st, d);
-    if (b->large) hipLaunchKernelGGL(k_b_build, dim3((unsigned)b->ntiles), dim3(BLOCK), 0, st, d);
+    if (b->large || d.crowd)
+        hipLaunchKernelGGL(k_b_build, dim3((unsigned)b->ntiles), dim3(BLOCK), 0, st, d);
     hipLaunchKernelGGL(k_b_build_cells, dim3((unsigned)std::min<long long>(d.nctiles, BC_GRID)),
                        dim3(BC_BLOCK), 0, st, d);
     if (rigid)
@@ -2338,13 +2343,16 @@ static int batch_run(dpm_batch* b, const dpm_jam_params* P, bool min_only,
         }
         S = f;
     }
+    int64_t small = 0;
     b->phased_disks = false;
     for (int64_t s = 0; s < b->nsys; ++s) {
         BSys& S = b->hsys[s];
         S.res = cost[s] >= 0.0 && cost[s] <= load.us() ? 1 : 0;
         if (S.res) resident.push_back({(int)s, S.n});
         else if (b->nv[s] == 0) b->phased_disks = true;
+        if (!S.res && S.n < BC_MIN_N) ++small;
     }
+    d.crowd = small > BC_GRID ? 1 : 0;
     b->phased = (int64_t)resident.size() < b->nsys;
     if (resident_table(b, resident)) return -1;
     DPM_HIP(hipMemcpyAsync(d.sys, b->hsys.data(), sizeof(BSys) * b->nsys, hipMemcpyHostToDevice,
@@ -2697,6 +2705,7 @@ static int serve_upload_tiles(dpm_server* sv) {
     std::vector<std::pair<int, int64_t>> resident;
     b->phased = b->slow_phased = false;
     bool large = false;
+    int64_t small = 0;
     for (size_t s = 0; s < sv->sys_req.size(); ++s) {
         if (!sv->sys_req[s]) continue;
         const dpm_server_req& q = sv->reqs.at(sv->sys_req[s]);
@@ -2706,12 +2715,15 @@ static int serve_upload_tiles(dpm_server* sv) {
             resident.push_back({(int)s, q.n});
         } else {
             b->phased = true;
+            small += q.n < BC_MIN_N ? 1 : 0;
             b->slow_phased = b->slow_phased || q.res_us < 0.0;
         }
     }
-    if (large != b->large) {  // the step's launches change
+    const int crowd = small > BC_GRID ? 1 : 0;
+    if (large != b->large || crowd != b->d.crowd) {  // the step's launches change
         drop_graph(b);
         b->large = large;
+        b->d.crowd = crowd;
     }
     if (resident_table(b, resident)) return -1;
     // the bound of batch_alloc: ct never exceeds d.nctiles entries

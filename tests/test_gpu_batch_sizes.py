@@ -190,3 +190,29 @@ def test_crowd_jams_and_is_served():
         assert np.array_equal(got["x"], ref[k % 4][1])
     b.close()
     sv.close()
+
+
+@pytest.mark.parametrize("count", (512, 513))
+def test_crowds_of_small_rigid_systems(count):
+    """More small rigid systems than the row build has workgroups get all-pairs rows."""
+    sts = [W.bumpy_config(n, 0.75, seed=n) for n in (2, 9, 30, 127, 128, 200)]
+    ref = []
+    for st in sts:
+        s = W.make_bumpy_system(P.System, st, backend=oracle(), e_c=W.bumpy_contact_scale(st),
+                                method=P.NBR_VERLET)
+        r = s.minimize_fire(fire(40))
+        ref.append((r.steps, s.reduce(P.RED_PE), s.download(P.F_X), s.download(P.F_ANGLE)))
+        s.close()
+    pick = [k % 4 for k in range(count)] + [4, 5]
+    print("[gpu-case] rigid crowd", count, flush=True)
+    b = P.Batch([sts[k].n for k in pick], [sts[k].nv for k in pick])
+    for i, k in enumerate(pick):
+        t = sts[k]
+        b.set_rigid_system(i, t.x, t.y, t.rad, t.mass, t.angle, t.nverts, t.rv, t.side,
+                           e_c=W.bumpy_contact_scale(t))
+    res, _ = b.minimize(fire(40))
+    for i, k in enumerate(pick):
+        x, y, a = b.get_rigid_system(i)[:3]
+        assert (res[i].fire_steps_total, res[i].pe) == ref[k][:2], sts[k].n
+        assert np.array_equal(x, ref[k][2]) and np.array_equal(a, ref[k][3]), sts[k].n
+    b.close()
