@@ -709,6 +709,7 @@ __global__ __launch_bounds__(BLOCK) void k_rb_vbuild(BDev b) {
     const PairParams pp = bparams(b, S);
     const double vc = sqrt(S.vc2);
     const bool shift = fmin(pp.halfLx, pp.halfLy) > ring_shift_limit(S.rmax, S.rv, vc);
+    const bool window = fmin(pp.halfLx, pp.halfLy) > ring_window_limit(S.rmax, S.rv, vc);
     __shared__ RingEntry rings[BLOCK / RB_HALF][RB_HALF];
     RingEntry* ring = rings[threadIdx.x / RB_HALF];
     const int hs = (int)(threadIdx.x % WAVE) / RB_HALF * RB_HALF;  // the half's first lane
@@ -727,9 +728,9 @@ __global__ __launch_bounds__(BLOCK) void k_rb_vbuild(BDev b) {
         };
         const int cnt =
             shift ? vertex_row<true>(pp, b.P, b.vst, b.nvt, b.vpos, S.rv, vc, S.vc2, S.vp2, lane,
-                                     hs, has, xv, cp, nn, true, ring, entry, emit)
+                                     hs, has, xv, cp, nn, window, ring, entry, emit)
                   : vertex_row<false>(pp, b.P, b.vst, b.nvt, b.vpos, S.rv, vc, S.vc2, S.vp2, lane,
-                                      hs, has, xv, cp, nn, true, ring, entry, emit);
+                                      hs, has, xv, cp, nn, window, ring, entry, emit);
         if (has) {
             b.vnum[v] = cnt;
             mx = max(mx, cnt);

@@ -285,6 +285,7 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb
     if (gated && d.ctl->kind < 1) return;
     const double vc = sqrt(nb.vc2);
     const bool shift = fmin(nb.halfLx, nb.halfLy) > ring_shift_limit(rmax, rv, vc);
+    const bool window = even && fmin(nb.halfLx, nb.halfLy) > ring_window_limit(rmax, rv, vc);
     __shared__ RingEntry rings[BLOCK / VB_HALF][VB_HALF];
     __shared__ int lists[LISTS ? BLOCK / VB_HALF : 1][VB_LIST];
     RingEntry* ring = rings[threadIdx.x / VB_HALF];
@@ -349,10 +350,10 @@ __global__ __launch_bounds__(BLOCK) void k_bumpy_vertex_rows(Dev d, NbrParams nb
             };
             const int cnt =
                 shift ? vertex_row<true>(nb, d.P0, d.vstart, d.nverts, d.vpos, rv, vc, nb.vc2,
-                                         nb.vp2, lane, hs, has, xv, cp, nn, even, ring, entry,
+                                         nb.vp2, lane, hs, has, xv, cp, nn, window, ring, entry,
                                          emit)
                       : vertex_row<false>(nb, d.P0, d.vstart, d.nverts, d.vpos, rv, vc, nb.vc2,
-                                          nb.vp2, lane, hs, has, xv, cp, nn, even, ring, entry,
+                                          nb.vp2, lane, hs, has, xv, cp, nn, window, ring, entry,
                                          emit);
             if (has) {
                 d.vnum[v] = cnt;

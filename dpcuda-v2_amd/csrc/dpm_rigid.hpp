@@ -83,6 +83,14 @@ __device__ __host__ inline double ring_shift_limit(double rmax, double rv, doubl
     return (3.0 * rmax - 3.0 * rv + vc) * (1.0 + 1e-6);
 }
 
+// The half box from which a ring's window can be taken around its centre's nearest image: a vertex of
+// the ring within vc of a point lies on an image of the ring whose centre is within ring radius +
+// vc of the point, and two such images are a box side apart.  In smaller boxes (one to three
+// particles) another image than the nearest may be the one that reaches the point.
+__device__ __host__ inline double ring_window_limit(double rmax, double rv, double vc) {
+    return (rmax - rv + vc) * (1.0 + 1e-6);
+}
+
 // atan2(y, x) to 1.2e-5 (an odd polynomial on [0, 1], fitted to the least largest error)
 __device__ __forceinline__ float atan2_coarse(float y, float x) {
     const float ax = fabsf(x), ay = fabsf(y), hi = fmaxf(ax, ay), lo = fminf(ax, ay);
@@ -115,9 +123,9 @@ struct RingEntry {
 // The vertex rows of one particle (kernelUpdateVertexNeighborList, rigid_bumpy/kernels.cu:
 // 870-922: for vertex v, over the particle row in order, the particles q whose centre lies
 // within vp of v, then q's vertices in order within vc of v), for vertices on their rings (even:
-// evenly spaced ones): a half-wave per particle, lane a0 + lane its vertex xv; the return value
-// is the lane's row length, emit(pos, u) stores entry pos.  R: 32 entries of LDS of the
-// half-wave's own.
+// evenly spaced ones, in a box of ring_window_limit): a half-wave per particle, lane a0 + lane
+// its vertex xv; the return value is the lane's row length, emit(pos, u) stores entry pos.  R: 32
+// entries of LDS of the half-wave's own.
 //   1. each lane loads one row entry and puts it into R if some vertex of the particle can
 //      reach it (in row order);
 //   2. every lane tests the entries (vp and the ring's reach) into a bit mask;
@@ -126,9 +134,7 @@ struct RingEntry {
 // SHIFT: the minimum image of x_p - x_q serves every vertex of both rings (ring_shift_limit):
 // pbc(v, u) = (v - u) - L k with one k, the same bits.  It is formed once per row entry; a lane
 // that formed it for every vertex and entry spent most of its instructions on it.
-// Without it (boxes of a few diameters) every vertex is tested by its own image, and all of them
-// are candidates: another image of the ring than its centre's nearest may be within vc of v, and
-// the window looks at the nearest alone.
+// Without it (boxes of a few diameters) every vertex is tested by its own image.
 // What bounds it: the gathers of the row entries and of their rings' vertices (halving the vector
 // instructions, by fields in LDS instead of cross-lane reads, took a build of 65,536 particles of
 // 24 vertices from 82 us to 70).
@@ -172,8 +178,7 @@ __device__ __forceinline__ int vertex_row(const Box& bx, const double4* P, const
                 e.per = (float)e.n * 0.15915494f;
                 const float x = (float)vc / (float)(c.z - rv);
                 e.half = (x + 0.25f * x * x * x) * e.per + 0.02f + 2e-5f * e.per;
-                if (!SHIFT || !even || !(x < 0.6f && 2.0f * e.half + 2.0f < (float)e.n))
-                    e.half = -1.0f;
+                if (!even || !(x < 0.6f && 2.0f * e.half + 2.0f < (float)e.n)) e.half = -1.0f;
             }
         }
         const unsigned nm = (unsigned)(__builtin_amdgcn_ballot_w64(near) >> hs);

@@ -11,7 +11,7 @@ P = pkg()
 W = workloads()
 pytestmark = pytest.mark.gpu
 
-SYSTEMS = [(n, phi) for n in (2, 3, 5, 9) for phi in (0.6, 0.84, 1.0, 1.3)]
+SYSTEMS = [(n, phi) for n in (1, 2, 3, 4, 5, 7, 9, 12) for phi in (0.6, 0.84, 1.0, 1.3)]
 
 
 def rows(s):
@@ -29,7 +29,7 @@ def spec():
 @pytest.mark.parametrize("n_small,n_large", ((20, 28), (9, 14), (33, 40)))
 def test_rows_and_forces(n, phi, n_small, n_large):
     print("[gpu-case] tiny box rows", n, phi, n_small, n_large, flush=True)
-    for seed in range(3):
+    for seed in range(4):
         st = W.bumpy_config(n, phi, seed=seed, n_small=n_small, n_large=n_large)
         got = []
         for be in (None, oracle()):
